@@ -9,7 +9,10 @@
 //
 // Sums over nodes use explicit fused multiply-adds in a fixed order, so a
 // trace computed in two different kernels (or twice in one) is bitwise the
-// same value: neighbours read exactly what the owner used.
+// same value: neighbours read exactly what the owner used.  The pointwise
+// functions below write their fused multiply-adds out too and switch the
+// compiler's own contraction off, so that a stage computed by another kernel
+// (one launch per stage, several steps per launch) has the same bits.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -39,8 +42,9 @@ __device__ __forceinline__ double line_dot(const double *__restrict__ l, const T
 // max over both sides of |(u_n +- sqrt(u_n^2 + 2 g H^3)) / (2H)|.
 __device__ __forceinline__ double sw_example_speed(double uOut, double pR, double uIn, double pL, double g)
 {
-    const double sR = sqrt(uOut * uOut + 2.0 * g * (pR * pR * pR));
-    const double sL = sqrt(uIn * uIn + 2.0 * g * (pL * pL * pL));
+    #pragma clang fp contract(off)
+    const double sR = sqrt(__builtin_fma(uOut, uOut, 2.0 * g * (pR * pR * pR)));
+    const double sL = sqrt(__builtin_fma(uIn, uIn, 2.0 * g * (pL * pL * pL)));
     return fmax(fmax(fabs(0.5 * (uOut + sR) / pR), fabs(0.5 * (uOut - sR) / pR)),
                 fmax(fabs(0.5 * (uIn + sL) / pL), fabs(0.5 * (uIn - sL) / pL)));
 }
@@ -52,21 +56,22 @@ __device__ __forceinline__ double sw_example_speed(double uOut, double pR, doubl
 __device__ __forceinline__ void sw_riemann(const double in[3], const double out[3], double nx,
                                            double ny, double g, double f[3], bool example = false)
 {
+    #pragma clang fp contract(off)
     const double uL = in[0], vL = in[1], pL = in[2];
     const double uR = out[0], vR = out[1], pR = out[2];
-    const double uOut = uR * nx + vR * ny;
-    const double uIn = uL * nx + vL * ny;
+    const double uOut = __builtin_fma(uR, nx, vR * ny);
+    const double uIn = __builtin_fma(uL, nx, vL * ny);
     const double cR = sqrt(g * pR), cL = sqrt(g * pL);
     const double wR = uOut / pR, wL = uIn / pL;
     const double fac = example ? sw_example_speed(uOut, pR, uIn, pL, g)
                                : fmax(fmax(fabs(wR + cR), fabs(wR - cR)), fmax(fabs(wL + cL), fabs(wL - cL)));
     const double hgR = 0.5 * g * pR * pR, hgL = 0.5 * g * pL * pL;
-    const double a0 = wR * uR + hgR * nx + wL * uL + hgL * nx;
-    const double a1 = wR * vR + hgR * ny + wL * vL + hgL * ny;
+    const double a0 = __builtin_fma(hgL, nx, __builtin_fma(wL, uL, __builtin_fma(hgR, nx, wR * uR)));
+    const double a1 = __builtin_fma(hgL, ny, __builtin_fma(wL, vL, __builtin_fma(hgR, ny, wR * vR)));
     const double a2 = uOut + uIn;
-    f[0] = 0.5 * (a0 - fac * (out[0] - in[0]));
-    f[1] = 0.5 * (a1 - fac * (out[1] - in[1]));
-    f[2] = 0.5 * (a2 - fac * (out[2] - in[2]));
+    f[0] = 0.5 * __builtin_fma(-fac, out[0] - in[0], a0);
+    f[1] = 0.5 * __builtin_fma(-fac, out[1] - in[1], a1);
+    f[2] = 0.5 * __builtin_fma(-fac, out[2] - in[2], a2);
 }
 
 // 1/x from the FP32 reciprocal refined by two FP64 Newton steps
@@ -87,10 +92,11 @@ __device__ __forceinline__ double rcp_refined(double x)
 __device__ __forceinline__ void sw_riemann_mixed(const double in[3], const double out[3], double nx, double ny,
                                                  double g, double f[3], bool example = false)
 {
+    #pragma clang fp contract(off)
     const double uL = in[0], vL = in[1], pL = in[2];
     const double uR = out[0], vR = out[1], pR = out[2];
-    const double uOut = uR * nx + vR * ny;
-    const double uIn = uL * nx + vL * ny;
+    const double uOut = __builtin_fma(uR, nx, vR * ny);
+    const double uIn = __builtin_fma(uL, nx, vL * ny);
     const double wR = uOut * rcp_refined(pR), wL = uIn * rcp_refined(pL);
     const float cR = __builtin_amdgcn_sqrtf((float)(g * pR)), cL = __builtin_amdgcn_sqrtf((float)(g * pL));
     const float wRf = (float)wR, wLf = (float)wL;
@@ -98,20 +104,22 @@ __device__ __forceinline__ void sw_riemann_mixed(const double in[3], const doubl
                                : (double)fmaxf(fmaxf(fabsf(wRf + cR), fabsf(wRf - cR)),
                                                fmaxf(fabsf(wLf + cL), fabsf(wLf - cL)));
     const double hgR = 0.5 * g * pR * pR, hgL = 0.5 * g * pL * pL;
-    const double a0 = wR * uR + hgR * nx + wL * uL + hgL * nx;
-    const double a1 = wR * vR + hgR * ny + wL * vL + hgL * ny;
+    const double a0 = __builtin_fma(hgL, nx, __builtin_fma(wL, uL, __builtin_fma(hgR, nx, wR * uR)));
+    const double a1 = __builtin_fma(hgL, ny, __builtin_fma(wL, vL, __builtin_fma(hgR, ny, wR * vR)));
     const double a2 = uOut + uIn;
-    f[0] = 0.5 * (a0 - fac * (out[0] - in[0]));
-    f[1] = 0.5 * (a1 - fac * (out[1] - in[1]));
-    f[2] = 0.5 * (a2 - fac * (out[2] - in[2]));
+    f[0] = 0.5 * __builtin_fma(-fac, out[0] - in[0], a0);
+    f[1] = 0.5 * __builtin_fma(-fac, out[1] - in[1], a1);
+    f[2] = 0.5 * __builtin_fma(-fac, out[2] - in[2], a2);
 }
 
 // GetExternalState, ConservativeShallowWaterClass.f90:1698-1729
 __device__ __forceinline__ void sw_external(int bc, double nx, double ny, const double in[3], double ex[3])
 {
+    #pragma clang fp contract(off)
     if (bc == -100) {  // NO_NORMAL_FLOW: reflect the momentum about the wall
-        ex[0] = (ny * ny - nx * nx) * in[0] - 2.0 * nx * ny * in[1];
-        ex[1] = (nx * nx - ny * ny) * in[1] - 2.0 * nx * ny * in[0];
+        const double d = __builtin_fma(ny, ny, -(nx * nx)), c = 2.0 * nx * ny;
+        ex[0] = __builtin_fma(d, in[0], -(c * in[1]));
+        ex[1] = -__builtin_fma(d, in[1], c * in[0]);
         ex[2] = in[2];
     } else {           // RADIATION and unknown flags: zero state
         ex[0] = 0.0; ex[1] = 0.0; ex[2] = 0.0;
@@ -122,14 +130,15 @@ __device__ __forceinline__ void sw_external(int bc, double nx, double ny, const 
 template <bool FAST = false>
 __device__ __forceinline__ void sw_fluxes(const double s[3], double g, double xF[3], double yF[3])
 {
+    #pragma clang fp contract(off)
     // one reciprocal instead of four divisions (differs from U*U/H by at most 1 ulp)
     const double invH = FAST ? rcp_refined(s[2]) : 1.0 / s[2];
     const double hp = g * 0.5 * s[2] * s[2];
-    xF[0] = s[0] * s[0] * invH + hp;
+    xF[0] = __builtin_fma(s[0] * s[0], invH, hp);
     xF[1] = s[0] * s[1] * invH;
     xF[2] = s[0];
     yF[0] = s[1] * s[0] * invH;
-    yF[1] = s[1] * s[1] * invH + hp;
+    yF[1] = __builtin_fma(s[1] * s[1], invH, hp);
     yF[2] = s[1];
 }
 

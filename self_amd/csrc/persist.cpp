@@ -1,0 +1,122 @@
+// persist.cpp -- admission of kernels whose workgroups wait for each other
+// (persist.hpp).
+#include "persist.hpp"
+
+#include <cstdlib>
+#include <map>
+#include <mutex>
+#include <vector>
+
+namespace self {
+
+namespace {
+
+struct Flight {
+    int device;
+    hipStream_t stream;
+    double demand, share;  // CUs' worth of workgroups; a workgroup's share of a CU
+    hipEvent_t done;
+};
+
+std::mutex g_mutex;
+std::vector<Flight> g_flights;
+std::vector<std::pair<int, hipEvent_t>> g_events;  // finished flights' events, by device
+
+void prune()
+{
+    size_t k = 0;
+    for (Flight &f : g_flights) {
+        if (hipEventQuery(f.done) == hipErrorNotReady) g_flights[k++] = f;
+        else g_events.emplace_back(f.device, f.done);
+    }
+    g_flights.resize(k);
+    (void)hipGetLastError();  // "not ready" is an answer here, not an error of a later call
+}
+
+}  // namespace
+
+int persist_cus(int device)
+{
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 0;
+    return n;
+}
+
+int persist_blocks_per_cu(const void *kernel, int threads)
+{
+    static std::mutex m;
+    static std::map<std::pair<const void *, int>, int> known;
+    std::lock_guard<std::mutex> lock(m);
+    auto it = known.find({kernel, threads});
+    if (it != known.end()) return it->second;
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        n = 0;
+    }
+    known[{kernel, threads}] = n;
+    return n;
+}
+
+// About a microsecond a poll.  SELF_AMD_SPIN_LIMIT overrides it (a test of
+// the fallback sets 0: the first unsuccessful poll gives up).
+unsigned persist_spin_limit()
+{
+    const char *s = std::getenv("SELF_AMD_SPIN_LIMIT");
+    if (s && *s) return (unsigned)std::strtoul(s, nullptr, 10);
+    return 2000;
+}
+
+// Alone on the device, `blocks` <= perCu x CUs workgroups of one kernel all
+// become resident.  Beside others, by shares of a CU: a workgroup of share s
+// finds no room only if every CU has more than 1 - s in use, that is, if the
+// launches in flight use more than CUs x (1 - s) together; half the device is
+// kept free beyond that, since the room on a CU need not be in one piece.
+// Launches on one stream run one after another and count once.
+PersistGate::PersistGate(int device, hipStream_t stream, int blocks, int perCu)
+    : rc(SELF_OK), device_(device), stream_(stream), demand_((double)blocks / perCu), share_(1.0 / perCu)
+{
+    g_mutex.lock();
+    prune();
+    std::map<hipStream_t, double> per;
+    double largest = share_;
+    for (const Flight &f : g_flights) {
+        if (f.device != device || f.stream == stream) continue;
+        double &d = per[f.stream];
+        if (f.demand > d) d = f.demand;
+        if (f.share > largest) largest = f.share;
+    }
+    if (per.empty()) return;
+    double sum = demand_;
+    for (const auto &p : per) sum += p.second;
+    if (sum <= 0.5 * persist_cus(device) * (1.0 - largest)) return;
+    for (const Flight &f : g_flights) {
+        if (f.device != device || f.stream == stream) continue;
+        const hipError_t e = hipStreamWaitEvent(stream, f.done, 0);
+        if (e != hipSuccess && rc == SELF_OK) rc = hip_fail(e, "hipStreamWaitEvent", __FILE__, __LINE__);
+    }
+}
+
+PersistGate::~PersistGate() { g_mutex.unlock(); }
+
+int PersistGate::launched()
+{
+    hipEvent_t ev = nullptr;
+    for (size_t k = 0; k < g_events.size(); ++k)
+        if (g_events[k].first == device_) {
+            ev = g_events[k].second;
+            g_events.erase(g_events.begin() + (long)k);
+            break;
+        }
+    hipError_t e = ev ? hipSuccess : hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventRecord(ev, stream_);
+    if (e != hipSuccess) {  // without its event the launch cannot be waited for by others: wait here
+        (void)hipStreamSynchronize(stream_);
+        if (ev) g_events.emplace_back(device_, ev);
+        return hip_fail(e, "persistent launch event", __FILE__, __LINE__);
+    }
+    g_flights.push_back({device_, stream_, demand_, share_, ev});
+    return SELF_OK;
+}
+
+}  // namespace self

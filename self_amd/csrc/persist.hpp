@@ -1,0 +1,137 @@
+// persist.hpp -- kernels whose workgroups stay resident and wait for each
+// other (several RK stages or solver iterations per launch).
+//
+// Exchange: up to three doubles travel as four 8-byte words (two 16-byte
+// accesses), each word 48 bits of payload under the 16-bit tag of the step it
+// belongs to.  A reader polls the words themselves until all carry the tag it
+// wants, so no fence, flag or ordering between words is needed: an aligned
+// 8-byte half of an access is single-copy atomic, and agent-scope accesses
+// (sc1) are coherent across the 8 XCDs' L2s.  Buffers are double-buffered by
+// the tag's parity: a writer overwrites a word only after it has received a
+// value its reader sent after reading that word, so a word holds the wanted
+// tag or that of two steps before and 16 bits of tag are enough.
+// What bounds it is the number of accesses in flight past the L2s: with
+// 32-bit tags, six 8-byte accesses a message and every lane polling until the
+// slowest of its wavefront was done, 262 144 messages a stage took 91 us; with
+// each lane polling for itself 18 us.
+//
+// Progress: a workgroup waits only for workgroups of its own launch, so every
+// wait ends once all of them are resident.  PersistGate orders the process's
+// own launches so that their workgroups fit beside each other, but whether the
+// last workgroup is placed is not the host's to say: kernels of other streams
+// that run at the start can leave a CU's LDS and registers in pieces too small
+// for it (seen: a launch of 1024 workgroups beside another model's stage
+// kernels).  So every wait is bounded: past `limit` polls (about a millisecond,
+// hundreds of times the longest wait of a resident launch) the launch records
+// its number in *status, every other wait sees that and all workgroups end,
+// leaving the launch's input untouched; the launches queued behind it return at
+// once, and the host runs the steps through ordinary launches.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "common.hpp"
+
+namespace self {
+
+typedef unsigned long long ll_word;
+typedef unsigned ll_quad __attribute__((ext_vector_type(4)));
+
+// A message buffer: [slot][2][lane] quads, 16-byte half h of message m of a
+// slot of n messages at quad (slot 2 + h) n + m.
+struct LLBuf {
+    __amdgpu_buffer_rsrc_t r;
+    __device__ __forceinline__ LLBuf(void *p, size_t bytes)
+        : r(__builtin_amdgcn_make_buffer_rsrc(p, 0, (int)bytes, 0x00020000))
+    {
+    }
+};
+
+constexpr int kLLAgent = 16;                   // sc1: agent scope
+constexpr int kLLPoll = 16 | (int)0x80000000;  // and volatile: each poll loads again
+
+// words of a message: three payloads of 48 bits, their three top halves in a fourth
+__device__ __forceinline__ void ll_store3(const LLBuf &B, unsigned off0, unsigned off1, const double v[3], unsigned tag)
+{
+    unsigned lo[3], hi[3];
+    #pragma unroll
+    for (int f = 0; f < 3; ++f) {
+        const ll_word b = (ll_word)__double_as_longlong(v[f]);
+        lo[f] = (unsigned)b;
+        hi[f] = (unsigned)(b >> 32);
+    }
+    const unsigned t = tag << 16;
+    const ll_quad a = {lo[0], (hi[0] & 0xffffu) | t, lo[1], (hi[1] & 0xffffu) | t};
+    const ll_quad c = {lo[2], (hi[2] & 0xffffu) | t, (hi[0] >> 16) | (hi[1] & 0xffff0000u), (hi[2] >> 16) | t};
+    __builtin_amdgcn_raw_buffer_store_b128(a, B.r, (int)off0, 0, kLLAgent);
+    __builtin_amdgcn_raw_buffer_store_b128(c, B.r, (int)off1, 0, kLLAgent);
+}
+
+// true when every word of the message carries the tag
+__device__ __forceinline__ bool ll_try3(const LLBuf &B, unsigned off0, unsigned off1, unsigned tag, double v[3])
+{
+    const ll_quad a = __builtin_amdgcn_raw_buffer_load_b128(B.r, (int)off0, 0, kLLPoll);
+    const ll_quad c = __builtin_amdgcn_raw_buffer_load_b128(B.r, (int)off1, 0, kLLPoll);
+    const unsigned t = tag & 0xffffu;
+    const unsigned hi[3] = {(a.y & 0xffffu) | (c.z << 16), (a.w & 0xffffu) | (c.z & 0xffff0000u),
+                            (c.y & 0xffffu) | (c.w << 16)};
+    const unsigned lo[3] = {a.x, a.z, c.x};
+    #pragma unroll
+    for (int f = 0; f < 3; ++f) v[f] = __longlong_as_double((long long)(((ll_word)hi[f] << 32) | lo[f]));
+    return (a.y >> 16) == t && (a.w >> 16) == t && (c.y >> 16) == t && (c.w >> 16) == t;
+}
+
+// One launch's bookkeeping, shared by the kernels' waits.
+struct PersistArgs {
+    int *status;      // 0, or the number of the first launch that gave up (device memory)
+    int launch;       // this launch's number (>= 1)
+    unsigned limit;   // polls before a wait gives up
+};
+
+__device__ __forceinline__ bool persist_given_up(const PersistArgs &P)
+{
+    return __hip_atomic_load(P.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+}
+
+// Every lane of the wavefront calls this; lanes with need wait for their
+// message, each polling until it has its own.  False: the wait gave up (the
+// same answer in every lane).
+__device__ __forceinline__ bool ll_wait3(const LLBuf &B, unsigned off0, unsigned off1, unsigned tag, bool need,
+                                         double v[3], const PersistArgs &P)
+{
+    bool ok = !need;
+    for (unsigned n = 0;; ++n) {
+        if (!ok) ok = ll_try3(B, off0, off1, tag, v);
+        if (__all(ok)) return true;
+        __builtin_amdgcn_s_sleep(1);
+        if ((n & 63u) == 63u && persist_given_up(P)) return false;
+        if (n >= P.limit) {
+            __hip_atomic_store(P.status, P.launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return false;
+        }
+    }
+}
+
+// Host side.  Resident workgroups of a kernel per CU (0 on error).
+int persist_blocks_per_cu(const void *kernel, int threads);
+int persist_cus(int device);
+unsigned persist_spin_limit();
+
+// Admission of one launch of `blocks` workgroups, `perCu` of which fit a CU.
+// The gate keeps the process's resident launches from taking each other's CUs:
+// a launch that might not become resident beside the ones in flight on other
+// streams is ordered after them.  Construct, check rc, launch, call launched().
+class PersistGate {
+public:
+    PersistGate(int device, hipStream_t stream, int blocks, int perCu);
+    ~PersistGate();
+    int rc;
+    int launched();
+
+private:
+    int device_;
+    hipStream_t stream_;
+    double demand_, share_;
+};
+
+}  // namespace self
