@@ -30,6 +30,7 @@
 #include <memory>
 #include <vector>
 
+#include "cg_resident.hpp"
 #include "common.hpp"
 #include "dg2d_device.hpp"
 #include "fempc.hpp"
@@ -432,12 +433,19 @@ struct CgsemOp final : DevOp {
     float *G3f = nullptr, *Df = nullptr, *dinvf = nullptr, *Lbuf32 = nullptr;
     double *xg = nullptr;  // global solution vector
     size_t bytes = 0;
+    // the resident form (cg_resident.hpp): messages, partial sums, its end
+    int maxCopies = 0;              // copies of the most shared DOF
+    char *resBuf = nullptr;
+    size_t resBytes = 0;
+    int resLaunches = 0, resGaveUp = 0;
+    unsigned resTag = 0;
+    bool resident = true;
     std::vector<double> kH;         // flux coefficient last set (host, local layout; empty = ONE)
     std::unique_ptr<FemPC> pc;      // CGsemPreconditioner_2D (self_cgsem2d_set_preconditioner)
 
     ~CgsemOp() override
     {
-        void *p[] = {gid, cs, ci, G3, D, bl, uD, dinv, Lbuf, G3f, Df, dinvf, Lbuf32, xg, metD, kD, wD};
+        void *p[] = {gid, cs, ci, G3, D, bl, uD, dinv, Lbuf, G3f, Df, dinvf, Lbuf32, xg, metD, kD, wD, resBuf};
         for (void *q : p)
             if (q) (void)hipFree(q);
         if (stream) (void)hipStreamDestroy(stream);
@@ -523,6 +531,90 @@ struct CgsemOp final : DevOp {
                        SolverState *st, const RedSlot &slot, int it, bool pending, hipStream_t s) override
     {
         return cg_iter<float>(dinvA, u, r, w, vOld, vNew, G3f, Df, Lbuf32, st, slot, it, pending, s);
+    }
+
+    // exchange messages | red1 | red2 | end of the launch | status
+    static constexpr size_t kResRed = (size_t)kCgResReplicas * (16 * 256 + 32 * 256);
+    size_t res_exch() const { return 16 * nLocal; }
+
+    template <int NN, int K>
+    int resident_launch(KrylovWork &wk, bool precond, int most, bool &taken, hipStream_t s)
+    {
+        constexpr int epb = kCgResThreads / ((NN + 1) * (NN + 1));
+        const void *f = reinterpret_cast<const void *>(&k_cg_resident<NN, K>);
+        const int blocks = (int)((nE + (size_t)epb * K - 1) / ((size_t)epb * K));
+        int device = 0;
+        SELF_HIP(hipGetDevice(&device));
+        if (persist_blocks_per_cu(f, kCgResThreads) < 1 || blocks > most * persist_cus(device) / 8) return SELF_OK;
+        if (!resBuf) {
+            resBytes = res_exch() + kResRed + sizeof(CgResOut) + 64;
+            if (dev(&resBuf, resBytes) != SELF_OK) {  // no memory for it: the two-launch form needs none
+                (void)hipGetLastError();
+                resGaveUp = 4;
+                return SELF_OK;
+            }
+            SELF_HIP(hipMemsetAsync(resBuf, 0, resBytes, s));  // tags start at 1
+        }
+        CgResArgs A{};
+        A.gid = gid;
+        A.cs = cs;
+        A.ci = ci;
+        A.G3 = G3;
+        A.D = D;
+        A.dinv = precond ? dinv : nullptr;
+        A.r = wk.r;
+        A.u = wk.u;
+        A.uOut = wk.z;
+        A.st = wk.st;
+        A.exch = reinterpret_cast<ll_quad *>(resBuf);
+        A.red1 = reinterpret_cast<ll_quad *>(resBuf + res_exch());
+        A.red2 = A.red1 + 256 * kCgResReplicas;
+        A.exchBytes = (unsigned)res_exch();
+        A.nE = (int)nE;
+        A.tag0 = resTag;
+        A.out = reinterpret_cast<CgResOut *>(resBuf + res_exch() + kResRed);
+        A.P.status = reinterpret_cast<int *>(resBuf + resBytes - 64);
+        A.P.launch = ++resLaunches;
+        A.P.limit = persist_spin_limit();
+        PersistGate gate(device, s, blocks, 1);
+        if (gate.rc) return gate.rc;
+        hipLaunchKernelGGL((k_cg_resident<NN, K>), dim3((unsigned)blocks), dim3(kCgResThreads), 0, s, A);
+        SELF_HIP(hipGetLastError());
+        hipLaunchKernelGGL(k_cg_res_commit, dim3(1), dim3(1), 0, s, wk.st, (const CgResOut *)A.out,
+                           (const int *)A.P.status);
+        SELF_HIP(hipGetLastError());
+        taken = true;
+        return gate.launched();
+    }
+
+    int resident_cg(KrylovWork &wk, bool precond, bool &taken, hipStream_t s) override
+    {
+        taken = false;
+        if (!resident || resGaveUp >= 4 || maxCopies > 4 || res_exch() >= (1u << 31)) return SELF_OK;
+        int rc = SELF_OK;
+        // As few nodes a thread as the device has workgroups for; one a thread
+        // only on up to 7/8 of the CUs (64x64, N = 7: 7.8 us an iteration on 256
+        // workgroups, 7.1 on 128 with two; 56x56 on 196: 6.3 against 6.4 on 98).
+        CG_DISPATCH_N(N, if constexpr (NN > 1) {
+            rc = (resident_launch<NN, 1>(wk, precond, 7, taken, s));
+            if (!rc && !taken) rc = (resident_launch<NN, 2>(wk, precond, 8, taken, s));
+            if (!rc && !taken) rc = (resident_launch<NN, 4>(wk, precond, 8, taken, s));
+        });
+        return rc;
+    }
+
+    int resident_cg_end(KrylovWork &wk, const SolverState &h, bool &gaveUp, hipStream_t s) override
+    {
+        gaveUp = h.done == kCgGaveUp;
+        if (gaveUp) {  // beside much other work on the device it will happen again
+            ++resGaveUp;
+            resTag = 0;
+            SELF_HIP(hipMemsetAsync(resBuf, 0, resBytes, s));
+        } else if (h.done != 3) {  // 3: nothing to solve, the launch returned at once
+            std::swap(wk.u, wk.z);
+            resTag += (unsigned)h.iter;
+        }
+        return SELF_OK;
     }
 
     int residual(const double *x, double *r, SolverState *st, int fin, const RedSlot &slot, hipStream_t s) override
@@ -670,6 +762,7 @@ int build_maps(CgsemOp &op, int nEdges, int nNodes, const int *edges, const int 
         const int d = order[g];
         for (int c = cpStart[d]; c < cpStart[d + 1]; ++c) op.ciH.push_back(cpList[c]);
         op.csH[g + 1] = (int)op.ciH.size();
+        op.maxCopies = std::max(op.maxCopies, op.csH[g + 1] - op.csH[g]);
     }
     return SELF_OK;
 }
@@ -1245,8 +1338,43 @@ try {
     int *tblD = reinterpret_cast<int *>(tables + descBytes);
     int *flagsD = tblD + 3 * nProblems + 2;
     SELF_HIP(hipEventRecord(h0->ev0, s));
+    // Problems with a resident form take it, as their single solves do (so the
+    // results are the same bits), each on its own stream: the gate lets them
+    // run side by side while CUs last.  One stream begins them all, so that no
+    // other launch is under way when they start.
+    std::vector<char> solved(nProblems, 0);
+    {
+        std::vector<char> taken(nProblems, 0);
+        for (int p = 0; p < nProblems; ++p) {
+            int rc = hs[p]->wk.ensure(hs[p]->op.n, 0, maxIters + 1, false);
+            if (!rc) rc = krylov_cg_begin(hs[p]->op, hs[p]->wk, precond == 1, kStopNormRel, tol, maxIters, hs[p]->op.xg, s);
+            if (rc) return rc;
+        }
+        SELF_HIP(hipStreamSynchronize(s));
+        for (int p = 0; p < nProblems; ++p) {
+            bool t = false;
+            if (int rc = hs[p]->op.resident_cg(hs[p]->wk, precond == 1, t, hs[p]->op.stream)) return rc;
+            taken[p] = t;
+        }
+        for (int p = 0; p < nProblems; ++p) {
+            if (!taken[p]) continue;
+            bool done = false;
+            if (int rc = krylov_cg_resident_end(hs[p]->op, hs[p]->wk, done, hs[p]->op.stream)) return rc;
+            if (done) {
+                KrylovResult res;
+                if (int rc = krylov_cg_finish(hs[p]->op, hs[p]->wk, kStopNormRel, tol, hs[p]->op.xg, res, hs[p]->op.stream))
+                    return rc;
+                ioerr[p] = res.ioerr;
+                iterations[p] = res.iterations;
+                solved[p] = 1;
+            }
+        }
+        for (int p = 0; p < nProblems; ++p)
+            if (solved[p]) SELF_HIP(hipStreamSynchronize(hs[p]->op.stream));
+    }
     std::vector<CgBatchProb> P(nProblems);
     for (int p = 0; p < nProblems; ++p) {
+        if (solved[p]) continue;
         self_cgsem2d_s *h = hs[p];
         CgsemOp &op = h->op;
         int rc = h->wk.ensure(op.n, 0, maxIters + 1, false);
@@ -1281,8 +1409,9 @@ try {
     SELF_HIP(hipGetLastError());
     SELF_HIP(hipMemcpyAsync(probsD, P.data(), descBytes, hipMemcpyHostToDevice, s));
     std::vector<int> act(nProblems), flags(nProblems);
-    for (int p = 0; p < nProblems; ++p) act[p] = p;
-    int nAct = nProblems;
+    int nAct = 0;
+    for (int p = 0; p < nProblems; ++p)
+        if (!solved[p]) act[nAct++] = p;
     for (int it0 = 1; it0 <= maxIters && nAct > 0; it0 += kCgbChunk) {
         const int it1 = std::min(it0 + kCgbChunk - 1, maxIters);
         // running list | direction prefix (nAct + 1) | update prefix (nAct + 1)
@@ -1313,6 +1442,7 @@ try {
         nAct = m;
     }
     for (int p = 0; p < nProblems; ++p) {
+        if (solved[p]) continue;
         KrylovResult res;
         const int rc = krylov_cg_finish(hs[p]->op, hs[p]->wk, kStopNormRel, tol, hs[p]->op.xg, res, s);
         if (rc) return rc;

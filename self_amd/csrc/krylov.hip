@@ -551,6 +551,17 @@ int krylov_cg_begin(DevOp &op, KrylovWork &wk, bool precond, int stopRule, doubl
     return SELF_OK;
 }
 
+int krylov_cg_resident_end(DevOp &op, KrylovWork &wk, bool &done, hipStream_t s)
+{
+    SolverState h{};
+    int rc = read_state(wk, h, s);
+    if (rc) return rc;
+    bool gaveUp = false;
+    if ((rc = op.resident_cg_end(wk, h, gaveUp, s))) return rc;
+    done = !gaveUp;
+    return SELF_OK;
+}
+
 int krylov_cg_finish(DevOp &op, KrylovWork &wk, int stopRule, double tol, double *sol, KrylovResult &res,
                      hipStream_t s)
 {
@@ -578,6 +589,13 @@ int run_cg(DevOp &op, KrylovWork &wk, bool precond, int stopRule, double tol, in
 {
     int rc = krylov_cg_begin(op, wk, precond, stopRule, tol, maxIters, sol, s);
     if (rc) return rc;
+    bool taken = false, done = false;
+    if ((rc = op.resident_cg(wk, precond, taken, s))) return rc;
+    if (taken) {
+        if ((rc = krylov_cg_resident_end(op, wk, done, s))) return rc;
+        if (done) return krylov_cg_finish(op, wk, stopRule, tol, sol, res, s);
+        if ((rc = krylov_cg_begin(op, wk, precond, stopRule, tol, maxIters, sol, s))) return rc;
+    }
     const double *dinv = precond ? op.inv_diag() : nullptr;
     for (int it0 = 1; it0 <= maxIters; it0 += kChunk) {
         if ((rc = cg_chunk<double>(op, wk.u, wk.r, wk.w, wk.v, wk.vB, wk.z, dinv, op.n, wk.st, wk.slot, it0,

@@ -160,6 +160,8 @@ __device__ __forceinline__ void cg_fold_end_wave(SolverState *st, const RedSlot 
     if (threadIdx.x == 0) cg_end_apply(st, it, S0, S1);
 }
 
+struct KrylovWork;
+
 // Operator plug-in (the deferred procedures of IterativeSolver).
 struct DevOp {
     size_t n = 0;                   // vector length the solver sees
@@ -192,6 +194,20 @@ struct DevOp {
     }
     virtual int cg_iteration32(const float *dinv, float *u, float *r, float *w, const float *vOld, float *vNew,
                                SolverState *st, const RedSlot &slot, int it, bool pending, hipStream_t s)
+    {
+        return SELF_ERR_STATE;
+    }
+    // The CG iterations of a solve begun by krylov_cg_begin in one launch, where
+    // the operator has one and the problem fits it (resident_cg launches it and
+    // sets taken).  resident_cg_end, with the state read after it, says whether
+    // the launch gave up (its input is untouched) and otherwise leaves the
+    // solution in wk.u.
+    virtual int resident_cg(KrylovWork &wk, bool precond, bool &taken, hipStream_t s)
+    {
+        taken = false;
+        return SELF_OK;
+    }
+    virtual int resident_cg_end(KrylovWork &wk, const SolverState &h, bool &gaveUp, hipStream_t s)
     {
         return SELF_ERR_STATE;
     }
@@ -267,6 +283,10 @@ int krylov_cg_begin(DevOp &op, KrylovWork &wk, bool precond, int stopRule, doubl
                     const double *sol, hipStream_t s);
 int krylov_cg_finish(DevOp &op, KrylovWork &wk, int stopRule, double tol, double *sol, KrylovResult &res,
                      hipStream_t s);
+// ... and between the two, for operators with a resident form: settles the
+// launch of DevOp::resident_cg (waits for it); done is false where it gave up
+// and the solve has to begin again.
+int krylov_cg_resident_end(DevOp &op, KrylovWork &wk, bool &done, hipStream_t s);
 
 // Mixed precision: FP32 PCG inner solves, FP64 residual and iterative
 // refinement to |b - A x| / |b - A x0| <= tol.

@@ -72,7 +72,8 @@ unsigned persist_spin_limit()
 // finds no room only if every CU has more than 1 - s in use, that is, if the
 // launches in flight use more than CUs x (1 - s) together; half the device is
 // kept free beyond that, since the room on a CU need not be in one piece.
-// Launches on one stream run one after another and count once.
+// Where every launch takes a CU a workgroup, each needs only as many CUs as it
+// has.  Launches on one stream run one after another and count once.
 PersistGate::PersistGate(int device, hipStream_t stream, int blocks, int perCu)
     : rc(SELF_OK), device_(device), stream_(stream), demand_((double)blocks / perCu), share_(1.0 / perCu)
 {
@@ -80,16 +81,19 @@ PersistGate::PersistGate(int device, hipStream_t stream, int blocks, int perCu)
     prune();
     std::map<hipStream_t, double> per;
     double largest = share_;
+    bool wholeCu = perCu == 1;
     for (const Flight &f : g_flights) {
         if (f.device != device || f.stream == stream) continue;
         double &d = per[f.stream];
         if (f.demand > d) d = f.demand;
         if (f.share > largest) largest = f.share;
+        wholeCu = wholeCu && f.share == 1.0;
     }
     if (per.empty()) return;
     double sum = demand_;
     for (const auto &p : per) sum += p.second;
-    if (sum <= 0.5 * persist_cus(device) * (1.0 - largest)) return;
+    const int cus = persist_cus(device);
+    if (wholeCu ? sum <= cus : sum <= 0.5 * cus * (1.0 - largest)) return;
     for (const Flight &f : g_flights) {
         if (f.device != device || f.stream == stream) continue;
         const hipError_t e = hipStreamWaitEvent(stream, f.done, 0);

@@ -50,6 +50,12 @@ struct LLBuf {
 constexpr int kLLAgent = 16;                   // sc1: agent scope
 constexpr int kLLPoll = 16 | (int)0x80000000;  // and volatile: each poll loads again
 
+// bytes 0, 1 of lo16 under bytes 0, 1 of hi16
+__device__ __forceinline__ unsigned ll_pair(unsigned hi16, unsigned lo16)
+{
+    return __builtin_amdgcn_perm(hi16, lo16, 0x05040100u);
+}
+
 // words of a message: three payloads of 48 bits, their three top halves in a fourth
 __device__ __forceinline__ void ll_store3(const LLBuf &B, unsigned off0, unsigned off1, const double v[3], unsigned tag)
 {
@@ -60,9 +66,8 @@ __device__ __forceinline__ void ll_store3(const LLBuf &B, unsigned off0, unsigne
         lo[f] = (unsigned)b;
         hi[f] = (unsigned)(b >> 32);
     }
-    const unsigned t = tag << 16;
-    const ll_quad a = {lo[0], (hi[0] & 0xffffu) | t, lo[1], (hi[1] & 0xffffu) | t};
-    const ll_quad c = {lo[2], (hi[2] & 0xffffu) | t, (hi[0] >> 16) | (hi[1] & 0xffff0000u), (hi[2] >> 16) | t};
+    const ll_quad a = {lo[0], ll_pair(tag, hi[0]), lo[1], ll_pair(tag, hi[1])};
+    const ll_quad c = {lo[2], ll_pair(tag, hi[2]), (hi[0] >> 16) | (hi[1] & 0xffff0000u), (hi[2] >> 16) | (tag << 16)};
     __builtin_amdgcn_raw_buffer_store_b128(a, B.r, (int)off0, 0, kLLAgent);
     __builtin_amdgcn_raw_buffer_store_b128(c, B.r, (int)off1, 0, kLLAgent);
 }
@@ -72,13 +77,37 @@ __device__ __forceinline__ bool ll_try3(const LLBuf &B, unsigned off0, unsigned 
 {
     const ll_quad a = __builtin_amdgcn_raw_buffer_load_b128(B.r, (int)off0, 0, kLLPoll);
     const ll_quad c = __builtin_amdgcn_raw_buffer_load_b128(B.r, (int)off1, 0, kLLPoll);
-    const unsigned t = tag & 0xffffu;
-    const unsigned hi[3] = {(a.y & 0xffffu) | (c.z << 16), (a.w & 0xffffu) | (c.z & 0xffff0000u),
-                            (c.y & 0xffffu) | (c.w << 16)};
+    const unsigned T = tag << 16;
+    const unsigned hi[3] = {ll_pair(c.z, a.y), (a.w & 0xffffu) | (c.z & 0xffff0000u), ll_pair(c.w, c.y)};
     const unsigned lo[3] = {a.x, a.z, c.x};
     #pragma unroll
     for (int f = 0; f < 3; ++f) v[f] = __longlong_as_double((long long)(((ll_word)hi[f] << 32) | lo[f]));
-    return (a.y >> 16) == t && (a.w >> 16) == t && (c.y >> 16) == t && (c.w >> 16) == t;
+    return (((a.y ^ T) | (a.w ^ T) | (c.y ^ T) | (c.w ^ T)) >> 16) == 0;
+}
+
+// one double in one quad
+__device__ __forceinline__ void ll_store1(const LLBuf &B, unsigned off, double v, unsigned tag)
+{
+    const ll_word b = (ll_word)__double_as_longlong(v);
+    const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+    const ll_quad a = {lo, ll_pair(tag, hi), hi >> 16, tag << 16};
+    __builtin_amdgcn_raw_buffer_store_b128(a, B.r, (int)off, 0, kLLAgent);
+}
+
+// its value; the tag bits that differ come back in the top half of `wrong`
+__device__ __forceinline__ double ll_load1(const LLBuf &B, unsigned off, unsigned tag, unsigned &wrong)
+{
+    const ll_quad a = __builtin_amdgcn_raw_buffer_load_b128(B.r, (int)off, 0, kLLPoll);
+    const unsigned T = tag << 16;
+    wrong = (a.y ^ T) | (a.w ^ T);
+    return __longlong_as_double((long long)(((ll_word)ll_pair(a.z, a.y) << 32) | a.x));
+}
+
+__device__ __forceinline__ bool ll_try1(const LLBuf &B, unsigned off, unsigned tag, double &v)
+{
+    unsigned wrong;
+    v = ll_load1(B, off, tag, wrong);
+    return (wrong >> 16) == 0;
 }
 
 // One launch's bookkeeping, shared by the kernels' waits.
@@ -93,15 +122,15 @@ __device__ __forceinline__ bool persist_given_up(const PersistArgs &P)
     return __hip_atomic_load(P.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
 }
 
-// Every lane of the wavefront calls this; lanes with need wait for their
-// message, each polling until it has its own.  False: the wait gave up (the
+// Every lane of the wavefront calls this; attempt() of a lane is true once it
+// has its message, each lane polling until then.  False: the wait gave up (the
 // same answer in every lane).
-__device__ __forceinline__ bool ll_wait3(const LLBuf &B, unsigned off0, unsigned off1, unsigned tag, bool need,
-                                         double v[3], const PersistArgs &P)
+template <typename F>
+__device__ __forceinline__ bool ll_wait(bool need, const PersistArgs &P, F attempt)
 {
     bool ok = !need;
     for (unsigned n = 0;; ++n) {
-        if (!ok) ok = ll_try3(B, off0, off1, tag, v);
+        if (!ok) ok = attempt();
         if (__all(ok)) return true;
         __builtin_amdgcn_s_sleep(1);
         if ((n & 63u) == 63u && persist_given_up(P)) return false;

@@ -31,6 +31,33 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
+// sum over the 64 lanes of a wavefront, in every lane, by data-parallel
+// primitives: lane moves of the vector pipe (row shifts by 1, 2, 4, 8, then the
+// rows' last lanes handed on to lane 63) instead of six trips through LDS
+// (7.07 -> 6.11 us a CG iteration of four such sums at 16x16, N = 3).  Every
+// lane of the wavefront is active.  Its order differs from wave_sum's.
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double x)
+{
+    const long long b = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+__device__ __forceinline__ double wave_sum_dpp(double v)
+{
+    v += dpp_move<0x111>(v);  // row_shr:1
+    v += dpp_move<0x112>(v);
+    v += dpp_move<0x114>(v);
+    v += dpp_move<0x118>(v);
+    v += dpp_move<0x142>(v);  // row_bcast:15
+    v += dpp_move<0x143>(v);  // row_bcast:31
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
 // sum over a 256-thread block (fixed tree), result valid in thread 0
 __device__ __forceinline__ double block_sum(double v, double *lds4)
 {

@@ -257,62 +257,6 @@ __device__ __forceinline__ void trace3(const NodalLDS<N> &L, const double *qs, i
     }
 }
 
-// Contractions on the FP64 matrix cores, for the degrees whose (N+1) x (N+1)
-// operator splits into 4 x 4 blocks (N = 3, 7).  v_mfma_f64_4x4x4 multiplies
-// four independent 4 x 4 blocks: lane l works for block (l >> 2) & 3, holds
-// A[l & 3][l >> 4] and B[l >> 4][l & 3] and gets D[l >> 4][l & 3].  At N = 7 a
-// wavefront holds one element and the four blocks are the quarters of its
-// 8 x 8 result (two instructions, K = 8); at N = 3 they are four elements.
-// The operator's entries stay in registers (one per lane and instruction), so
-// a field and direction needs 2 LDS reads per lane instead of 32 (N = 7), and
-// the multiply-adds leave the vector pipe, which the Riemann fluxes need
-// (FP64 stage kernel at 64x64, N = 7: 10.9 -> 10.1 us).
-// Element, node and side node of a lane follow the instruction's layout.
-template <int N>
-struct Mf {
-    static constexpr bool on = N == 3 || N == 7;
-    static constexpr int K = N == 7 ? 2 : 1;  // instructions per product
-};
-
-// element slot of a thread in its workgroup and its lane tl in the element
-template <int N>
-__device__ __forceinline__ int lane_element(int t, int &tl)
-{
-    if constexpr (N == 3) {
-        tl = (t & 3) + 4 * ((t >> 4) & 3);
-        return 4 * (t >> 6) + ((t >> 2) & 3);
-    } else {
-        constexpr int np = (N + 1) * (N + 1);
-        const int le = t / np;
-        tl = t - le * np;
-        return le;
-    }
-}
-
-// indices of lane tl in the instruction's layout: operand row / column c,
-// inner index (and result row) k, result quarter (bi, bj) at N = 7
-template <int N>
-struct MfLane {
-    int c, k, bi, bj;
-    __device__ __forceinline__ explicit MfLane(int tl)
-        : c(tl & 3), k(N == 7 ? (tl >> 4) & 3 : (tl >> 2) & 3), bi(N == 7 ? (tl >> 2) & 1 : 0),
-          bj(N == 7 ? (tl >> 3) & 1 : 0)
-    {
-    }
-};
-
-// node of lane tl
-template <int N>
-__device__ __forceinline__ int lane_node(int tl)
-{
-    if constexpr (Mf<N>::on) {
-        const MfLane<N> m(tl);
-        return (4 * m.bi + m.k) + (N + 1) * (4 * m.bj + m.c);
-    } else {
-        return tl;
-    }
-}
-
 // first side node (side (N+1) + k) of lane tl, or -1.  At N = 7 the quarter's
 // bits select the direction (bj: across p) and the half of the side (bi).
 template <int N>
@@ -1102,7 +1046,7 @@ __global__ __launch_bounds__(256, 4) void k_sw_steps(SWKernelArgs A, SWStepsArgs
             if (c > 0) info = A.side[(size_t)(act ? e : 0) * 4 + sd];
             double oth[3] = {0, 0, 0};
             const unsigned off = llMember + ll_slot<N>(side ? e : 0, side ? w : 0);
-            good = ll_wait3(ll, off, off + 16 * ns4, tag, side && info.x >= 0, oth, T.P) && good;
+            good = ll_wait(side && info.x >= 0, T.P, [&] { return ll_try3(ll, off, off + 16 * ns4, tag, oth); }) && good;
             if (side) {
                 double fn[3], fl[3], tr[3];
                 #pragma unroll

@@ -1,0 +1,80 @@
+"""The CGSEM CG as one launch per solve against its two launches an iteration
+(which a launch whose first unsuccessful poll gives up falls back to): every
+degree, one, two and four nodes a thread, ragged last workgroups, curved
+elements, prescribed boundary values, no preconditioner, a start at the
+solution, and sizes past the device's (which stay with the launches).
+
+After a fixed number of iterations the two differ by the rounding of their
+sums only: 12 iterations amplify 1e-16 by far less than 1e4 on these
+well-scaled problems, so 1e-12 relative.  Converged solutions to a relative
+residual of 1e-11 differ by at most that times the condition number (< 1e4
+here after the diagonal's scaling): 1e-7."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(N, nX, nY, warp=0.0, boundary=False):
+    from self_amd.krylov import CGsemElliptic2D, CGsemParams
+    m = CGsemElliptic2D(CGsemParams(polyDeg=N, nXElem=nX, nYElem=nY, warp=warp))
+    x, y = m.mesh.x, m.mesh.y
+    rng = np.random.default_rng(N + nX)
+    m.SetFluxCoefficient(1.0 + 0.5 * np.sin(2 * np.pi * x) * np.sin(2 * np.pi * y))
+    m.SetSource(np.cos(3 * x) * (1.0 + y) + 0.1 * rng.standard_normal(x.shape))
+    m.SetDirichletBoundaryCondition(np.cos(2 * x + y) if boundary else 0 * x)
+    return m
+
+
+def _solve(m, precond, tol, iters, start=None):
+    m.SetSolution(np.zeros_like(m.mesh.x) if start is None else start)
+    io, it, _ = m.Solve("cgsem_pcg", precond, tolerance=tol, maxIters=iters)
+    return m.GetSolution(), it, io, m.resi.copy()
+
+
+SHAPES = [(2, 7, 9), (3, 4, 4), (3, 21, 13), (4, 11, 6), (5, 3, 2), (5, 30, 17), (6, 8, 8), (7, 5, 7),
+          (7, 63, 57), (8, 9, 5), (9, 6, 6), (10, 4, 5), (11, 5, 3), (7, 80, 61), (3, 150, 131), (5, 122, 101),
+          (7, 128, 127), (10, 75, 60), (7, 130, 128)]
+
+
+@pytest.mark.parametrize("N,nX,nY", SHAPES)
+def test_one_launch_follows_the_launched_iterations(gpu_lib, N, nX, nY, monkeypatch):
+    m = _model(N, nX, nY, warp=0.03 if nX < 40 else 0.0, boundary=True)
+    for precond in ("jacobi", "none"):
+        a, ia, _, ra = _solve(m, precond, 1e-300, 12)
+        monkeypatch.setenv("SELF_AMD_SPIN_LIMIT", "0")
+        b, ib, _, rb = _solve(m, precond, 1e-300, 12)
+        monkeypatch.delenv("SELF_AMD_SPIN_LIMIT")
+        assert ia == ib == 12
+        assert rel_l2(a, b) < 1e-12
+        assert np.allclose(ra[:13], rb[:13], rtol=1e-10, atol=0)
+    m.Trash()
+
+
+@pytest.mark.parametrize("N,nX,nY", [(2, 7, 9), (3, 21, 13), (5, 30, 17), (7, 33, 31), (10, 4, 5)])
+def test_solutions_and_stop(gpu_lib, N, nX, nY, monkeypatch):
+    m = _model(N, nX, nY, warp=0.03, boundary=True)
+    a, ia, ioa, ra = _solve(m, "jacobi", 1e-11, 20000)
+    again, ic, _, _ = _solve(m, "jacobi", 1e-11, 20000)
+    assert ic == ia and np.array_equal(a, again)  # the same bits every time
+    monkeypatch.setenv("SELF_AMD_SPIN_LIMIT", "0")
+    b, ib, iob, _ = _solve(m, "jacobi", 1e-11, 20000)
+    monkeypatch.delenv("SELF_AMD_SPIN_LIMIT")
+    assert ioa == iob and abs(ia - ib) <= 2 + ib // 100
+    assert ra[ia] / ra[0] < 1e-11 <= ra[ia - 1] / ra[0]
+    assert rel_l2(a, b) < 1e-7
+    # begun at the solution: few iterations, and the form is still taken
+    c, it, _, _ = _solve(m, "jacobi", 1e-3, 100, start=a)
+    assert np.isfinite(c).all() and it <= 100
+    m.Trash()
+
+
+def test_nothing_to_solve(gpu_lib):
+    """A zero source from the zero solution: the loop ends before its first iteration."""
+    m = _model(7, 4, 3)
+    m.SetSource(0 * m.mesh.x)
+    u, it, _, _ = _solve(m, "jacobi", 1e-10, 50)
+    assert it == 0 and not u.any()
+    m.Trash()
