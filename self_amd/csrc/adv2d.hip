@@ -27,6 +27,7 @@
 #include "common.hpp"
 #include "dg2d_device.hpp"
 #include "dg2d_host.hpp"
+#include "layout.hpp"
 
 namespace self {
 namespace {
@@ -332,6 +333,7 @@ struct self_adv2d_s {
     size_t nE = 0;
     double kappa = 0.0, dt = 0.0;
     hipStream_t stream = nullptr;
+    HostStage stage;
     double *nodal = nullptr, *c = nullptr, *G = nullptr, *tend = nullptr, *grad = nullptr, *vel = nullptr;
     double *velTr = nullptr, *fvel = nullptr, *metric = nullptr, *fnrm = nullptr, *tr[2] = {nullptr, nullptr};
     double *trG = nullptr, *relax = nullptr, *rFac = nullptr;
@@ -429,13 +431,6 @@ int stage(self_adv2d_s *h, double t, int m, int mode)
     SELF_HIP(hipGetLastError());
     if (mode == 0) h->cur = 1 - h->cur;
     return SELF_OK;
-}
-
-void from_dev(const double *src, double *dst, size_t nE, int nf, int np)
-{
-    for (size_t e = 0; e < nE; ++e)
-        for (int f = 0; f < nf; ++f)
-            std::memcpy(dst + (e * nf + f) * np, src + ((size_t)f * nE + e) * np, sizeof(double) * np);
 }
 
 void to_dev(const double *src, double *dst, size_t nE, int nf, int np)
@@ -605,10 +600,7 @@ try {
         std::memset(data, 0, sizeof(double) * nq * nE * np);
         return SELF_OK;
     }
-    std::vector<double> buf(nq * nE * np);
-    SELF_HIP(hipMemcpy(buf.data(), src, sizeof(double) * buf.size(), hipMemcpyDeviceToHost));
-    from_dev(buf.data(), data, nE, (int)nq, (int)np);
-    return SELF_OK;
+    return fields_to_host(src, data, nE, (int)nq, (int)np, h->stage, h->stream);
 }
 SELF_CATCH_ALL
 

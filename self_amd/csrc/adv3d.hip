@@ -35,6 +35,7 @@
 #include "common.hpp"
 #include "dg2d_device.hpp"
 #include "dg3d_device.hpp"
+#include "layout.hpp"
 #include "mfma.hpp"
 
 namespace self {
@@ -575,6 +576,7 @@ struct self_adv3d_s {
     size_t nE = 0, nSlots = 0;
     double dt = 0.0;
     hipStream_t stream = nullptr;
+    HostStage stage;
     double *nodal = nullptr, *c = nullptr, *G = nullptr, *tend = nullptr, *vel = nullptr, *geo = nullptr;
     double *fdat = nullptr, *nrm = nullptr, *bpos = nullptr, *tr[2] = {nullptr, nullptr}, *velTr = nullptr;
     double *relax = nullptr, *rFac = nullptr, *E1 = nullptr, *E2 = nullptr, *lim = nullptr;
@@ -695,13 +697,6 @@ void h2d_fields(const double *src, double *dst, size_t nE, int nf, int np)
     for (size_t e = 0; e < nE; ++e)
         for (int f = 0; f < nf; ++f)
             std::memcpy(dst + ((size_t)f * nE + e) * np, src + (e * nf + f) * np, sizeof(double) * np);
-}
-
-void d2h_fields(const double *src, double *dst, size_t nE, int nf, int np)
-{
-    for (size_t e = 0; e < nE; ++e)
-        for (int f = 0; f < nf; ++f)
-            std::memcpy(dst + (e * nf + f) * np, src + ((size_t)f * nE + e) * np, sizeof(double) * np);
 }
 
 void free_all(self_adv3d_s *h)
@@ -903,10 +898,7 @@ try {
         SELF_HIP(hipMemcpy(data + 2 * nq * nE, h->lim, sizeof(double) * 3 * nq * nE, hipMemcpyDeviceToHost));
         return SELF_OK;
     }
-    std::vector<double> buf(nq * nE * np);
-    SELF_HIP(hipMemcpy(buf.data(), field == 0 ? h->c : h->tend, sizeof(double) * buf.size(), hipMemcpyDeviceToHost));
-    d2h_fields(buf.data(), data, nE, (int)nq, (int)np);
-    return SELF_OK;
+    return fields_to_host(field == 0 ? h->c : h->tend, data, nE, (int)nq, (int)np, h->stage, h->stream);
 }
 SELF_CATCH_ALL
 

@@ -46,6 +46,7 @@
 
 #include "common.hpp"
 #include "dg3d_device.hpp"
+#include "layout.hpp"
 
 namespace self {
 void cofactor3(const double *m, int dir, double out[3]);
@@ -61,6 +62,7 @@ struct self_hpe_s {
     size_t nE = 0, nH = 0, nL = 0;
     double dt = 0.0;
     hipStream_t stream = nullptr;
+    self::HostStage stage;
     double *nodal = nullptr, *sol = nullptr, *G = nullptr, *tend = nullptr, *geo = nullptr, *height = nullptr;
     double *nrm = nullptr, *fdat = nullptr, *tr = nullptr, *Bvol = nullptr, *divU = nullptr;
     int2 *side = nullptr;
@@ -779,12 +781,7 @@ try {
     }
     const int nf = field == 0 ? 5 : field == 1 ? 3 : 1;
     const double *src = field == 0 ? h->sol : field == 1 ? h->tend : h->divU;
-    std::vector<double> buf((size_t)nf * nE * np);
-    SELF_HIP(hipMemcpy(buf.data(), src, sizeof(double) * buf.size(), hipMemcpyDeviceToHost));
-    for (size_t e = 0; e < nE; ++e)
-        for (int f = 0; f < nf; ++f)
-            std::memcpy(data + (e * nf + f) * np, buf.data() + ((size_t)f * nE + e) * np, sizeof(double) * np);
-    return SELF_OK;
+    return fields_to_host(src, data, nE, nf, (int)np, h->stage, h->stream);
 }
 SELF_CATCH_ALL
 

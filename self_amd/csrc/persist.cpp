@@ -16,7 +16,11 @@ struct Flight {
     hipStream_t stream;
     double demand, share;  // CUs' worth of workgroups; a workgroup's share of a CU
     hipEvent_t done;
+    unsigned long long group;
 };
+
+// Launches of one group may run side by side; each waits for the groups before.
+unsigned long long g_group = 1;
 
 std::mutex g_mutex;
 std::vector<Flight> g_flights;
@@ -83,19 +87,19 @@ PersistGate::PersistGate(int device, hipStream_t stream, int blocks, int perCu)
     double largest = share_;
     bool wholeCu = perCu == 1;
     for (const Flight &f : g_flights) {
-        if (f.device != device || f.stream == stream) continue;
+        if (f.device != device || f.stream == stream || f.group != g_group) continue;
         double &d = per[f.stream];
         if (f.demand > d) d = f.demand;
         if (f.share > largest) largest = f.share;
         wholeCu = wholeCu && f.share == 1.0;
     }
-    if (per.empty()) return;
     double sum = demand_;
     for (const auto &p : per) sum += p.second;
     const int cus = persist_cus(device);
-    if (wholeCu ? sum <= cus : sum <= 0.5 * cus * (1.0 - largest)) return;
+    const bool fits = per.empty() || (wholeCu ? sum <= cus : sum <= 0.5 * cus * (1.0 - largest));
+    if (!fits) ++g_group;
     for (const Flight &f : g_flights) {
-        if (f.device != device || f.stream == stream) continue;
+        if (f.device != device || f.stream == stream || f.group == g_group) continue;
         const hipError_t e = hipStreamWaitEvent(stream, f.done, 0);
         if (e != hipSuccess && rc == SELF_OK) rc = hip_fail(e, "hipStreamWaitEvent", __FILE__, __LINE__);
     }
@@ -119,7 +123,7 @@ int PersistGate::launched()
         if (ev) g_events.emplace_back(device_, ev);
         return hip_fail(e, "persistent launch event", __FILE__, __LINE__);
     }
-    g_flights.push_back({device_, stream_, demand_, share_, ev});
+    g_flights.push_back({device_, stream_, demand_, share_, ev, g_group});
     return SELF_OK;
 }
 

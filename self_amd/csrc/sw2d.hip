@@ -41,6 +41,7 @@
 
 #include "common.hpp"
 #include "dg2d_device.hpp"
+#include "layout.hpp"
 #include "persist.hpp"
 
 namespace self {
@@ -1233,6 +1234,7 @@ struct self_sw2d_s {
     self_sw2d_desc d{};
     int device = 0;
     hipStream_t stream = nullptr;
+    HostStage stage;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int n1 = 0, np = 0;
     size_t nE = 0;
@@ -1705,19 +1707,12 @@ int check_ready(self_sw2d_s *h, bool settled = true)
     return settled ? settle(h) : SELF_OK;
 }
 
-// host layout [e][f][node] <-> device [f][e][node]
+// host layout [e][f][node] -> device [f][e][node]
 void to_device_layout(const double *src, double *dst, size_t nE, int nf, int np)
 {
     for (size_t e = 0; e < nE; ++e)
         for (int f = 0; f < nf; ++f)
             std::memcpy(dst + ((size_t)f * nE + e) * np, src + (e * nf + f) * np, sizeof(double) * np);
-}
-
-void from_device_layout(const double *src, double *dst, size_t nE, int nf, int np)
-{
-    for (size_t e = 0; e < nE; ++e)
-        for (int f = 0; f < nf; ++f)
-            std::memcpy(dst + (e * nf + f) * np, src + ((size_t)f * nE + e) * np, sizeof(double) * np);
 }
 
 }  // namespace
@@ -2000,12 +1995,8 @@ try {
     if (int rs = settle(h)) return rs;
     SELF_HIP(hipStreamSynchronize(h->stream));
     const size_t nE = h->nE, np = h->np, n1 = h->n1;
-    std::vector<double> buf;
     auto get_nodal = [&](const double *dev, int nf) -> int {
-        buf.resize((size_t)nf * nE * np);
-        SELF_HIP(hipMemcpy(buf.data(), dev, sizeof(double) * buf.size(), hipMemcpyDeviceToHost));
-        from_device_layout(buf.data(), data, nE, nf, (int)np);
-        return SELF_OK;
+        return fields_to_host(dev, data, nE, nf, (int)np, h->stage, h->stream);
     };
     switch (field) {
     case SELF_SW_SOLUTION: return get_nodal(h->q, 3);
@@ -2371,11 +2362,7 @@ try {
     SELF_HIP(hipSetDevice(h->device));
     SELF_HIP(hipStreamSynchronize(h->stream));
     const size_t nE = h->nE, np = h->np;
-    std::vector<double> buf(3 * nE * np);
-    SELF_HIP(hipMemcpy(buf.data(), h->q + (size_t)member * buf.size(), sizeof(double) * buf.size(),
-                       hipMemcpyDeviceToHost));
-    from_device_layout(buf.data(), data, nE, 3, (int)np);
-    return SELF_OK;
+    return fields_to_host(h->q + (size_t)member * 3 * nE * np, data, nE, 3, (int)np, h->stage, h->stream);
 }
 SELF_CATCH_ALL
 
