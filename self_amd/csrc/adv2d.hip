@@ -21,6 +21,8 @@
 // Velocity is static: its traces are computed once when it is set (the
 // reference recomputes them every stage).
 
+#include <algorithm>
+#include <chrono>
 #include <cstring>
 #include <vector>
 
@@ -28,6 +30,7 @@
 #include "dg2d_device.hpp"
 #include "dg2d_host.hpp"
 #include "layout.hpp"
+#include "persist.hpp"
 
 namespace self {
 namespace {
@@ -73,21 +76,82 @@ __device__ __forceinline__ double trace1(const NodalLDS<N> &L, const double *q, 
     return acc;
 }
 
-// DGSystemDerivative in s and p of one node: sum_m D(i,m) sl[m] + lift_s,
-// sum_m D(j,m) pl[m] + lift_p
+// The pointwise functions write their fused multiply-adds out and switch the
+// compiler's contraction off: the launched and the resident form of a stage
+// have the same bits.
+
+// line contractions of one node: sum_m D(i,m) sl[m] and sum_m D(j,m) pl[m]
 template <int N>
-__device__ __forceinline__ void dg_pair(const NodalLDS<N> &L, const double *sl, const double *pl, int i, int j,
-                                        double bE, double bW, double bN, double bS, double &t1, double &t2)
+__device__ __forceinline__ void dg_lines(const NodalLDS<N> &L, const double *sl, const double *pl, int i, int j,
+                                         double &a, double &b)
 {
     constexpr int n1 = N + 1;
-    double a = L.dS[i] * sl[0], b = L.dP[j] * pl[0];
+    a = L.dS[i] * sl[0];
+    b = L.dP[j] * pl[0];
     #pragma unroll
     for (int m = 1; m < n1; ++m) {
         a = __builtin_fma(L.dS[i + n1 * m], sl[m], a);
         b = __builtin_fma(L.dP[j + n1 * m], pl[n1 * m], b);
     }
-    t1 = a + (bE * L.lE[i] + bW * L.lW[i]) * L.iwS[i];
-    t2 = b + (bN * L.lN[j] + bS * L.lS[j]) * L.iwP[j];
+}
+
+// DGSystemDerivative in s and p of one node: line contractions plus lift
+template <int N>
+__device__ __forceinline__ void dg_lift(const NodalLDS<N> &L, int i, int j, double bE, double bW, double bN, double bS,
+                                        double &a, double &b)
+{
+    #pragma clang fp contract(off)
+    a = __builtin_fma(__builtin_fma(bE, L.lE[i], bW * L.lW[i]), L.iwS[i], a);
+    b = __builtin_fma(__builtin_fma(bN, L.lN[j], bS * L.lS[j]), L.iwP[j], b);
+}
+
+// The two sides of a side node in the edge's primary orientation (boundary:
+// the external state behind it), so that both elements form the value the
+// reference stores once.
+struct AdvSides {
+    double in, ex, dx, dy, sign;
+};
+
+// own, nbr: tracer and its gradient's two components at the node
+__device__ __forceinline__ AdvSides adv_sides(int2 info, const double own[3], const double nbr[3], double ext)
+{
+    AdvSides o;
+    const bool bnd = info.x < 0, prim = bnd || side_primary(info.y);
+    const double oc = bnd ? ext : nbr[0];
+    o.in = prim ? own[0] : oc;
+    o.ex = prim ? oc : own[0];
+    o.dx = bnd ? own[1] : (own[1] + nbr[1]) * 0.5;
+    o.dy = bnd ? own[2] : (own[2] + nbr[2]) * 0.5;
+    o.sign = prim ? 1.0 : -1.0;
+    return o;
+}
+
+// upwind plus diffusive flux of a side node (EdgeFlux, RiemannSolver :1756-1787)
+__device__ __forceinline__ double adv_side_flux(const AdvSides &o, double uN, double nx, double ny, double len,
+                                                double kappa)
+{
+    #pragma clang fp contract(off)
+    const double fl = 0.5 * __builtin_fma(uN, o.ex + o.in, -(fabs(uN) * (o.ex - o.in)));
+    const double dcdn = __builtin_fma(o.dx, nx, o.dy * ny);
+    return o.sign * (__builtin_fma(-kappa, dcdn, fl) * len);
+}
+
+// contravariant volume flux of c u - kappa grad c (XFlux, YFlux :1791-1825)
+__device__ __forceinline__ void adv_volume_flux(double c, double u, double v, double kappa, double dx, double dy,
+                                                const double met[4], double &s, double &p)
+{
+    #pragma clang fp contract(off)
+    const double xF = __builtin_fma(c, u, -(kappa * dx)), yF = __builtin_fma(c, v, -(kappa * dy));
+    s = __builtin_fma(met[3], xF, -(met[1] * yF));
+    p = __builtin_fma(met[0], yF, -(met[2] * xF));
+}
+
+__device__ __forceinline__ double adv_tendency(double t1, double t2, double J, bool relax, double field, double factor,
+                                               double c)
+{
+    #pragma clang fp contract(off)
+    const double tend = (-t1 - t2) / J;
+    return relax ? __builtin_fma(field - c, factor, tend) : tend;
 }
 
 template <int N, int NQ>
@@ -188,12 +252,12 @@ __global__ __launch_bounds__(256) void k_adv_gradient(AdvArgs A)
         for (int f = 0; f < NQ; ++f) {
             const int o = lo + f * np;
             double t1, t2, u1, u2;
-            dg_pair<N>(L, sx + o + n1 * j, px + o + i, i, j, bfE[((1 * 2 + 0) * NQ + f) * n1 + j],
-                       bfE[((3 * 2 + 0) * NQ + f) * n1 + j], bfE[((2 * 2 + 0) * NQ + f) * n1 + i],
-                       bfE[((0 * 2 + 0) * NQ + f) * n1 + i], t1, t2);
-            dg_pair<N>(L, sy + o + n1 * j, py + o + i, i, j, bfE[((1 * 2 + 1) * NQ + f) * n1 + j],
-                       bfE[((3 * 2 + 1) * NQ + f) * n1 + j], bfE[((2 * 2 + 1) * NQ + f) * n1 + i],
-                       bfE[((0 * 2 + 1) * NQ + f) * n1 + i], u1, u2);
+            dg_lines<N>(L, sx + o + n1 * j, px + o + i, i, j, t1, t2);
+            dg_lift<N>(L, i, j, bfE[((1 * 2 + 0) * NQ + f) * n1 + j], bfE[((3 * 2 + 0) * NQ + f) * n1 + j],
+                       bfE[((2 * 2 + 0) * NQ + f) * n1 + i], bfE[((0 * 2 + 0) * NQ + f) * n1 + i], t1, t2);
+            dg_lines<N>(L, sy + o + n1 * j, py + o + i, i, j, u1, u2);
+            dg_lift<N>(L, i, j, bfE[((1 * 2 + 1) * NQ + f) * n1 + j], bfE[((3 * 2 + 1) * NQ + f) * n1 + j],
+                       bfE[((2 * 2 + 1) * NQ + f) * n1 + i], bfE[((0 * 2 + 1) * NQ + f) * n1 + i], u1, u2);
             gxv[f] = (t1 + t2) / J;
             gyv[f] = (u1 + u2) / J;
             A.grad[((size_t)0 * NQ + f) * mstride + base] = gxv[f];
@@ -249,10 +313,8 @@ __global__ __launch_bounds__(256) void k_adv_stage(AdvArgs A)
             cE[f * np + nd] = c[f];
             gxE[f * np + nd] = dx;
             gyE[f * np + nd] = dy;
-            const double xF = c[f] * u - A.kappa * dx;  // XFlux :1791-1807
-            const double yF = c[f] * v - A.kappa * dy;  // YFlux :1809-1825
-            sCE[f * np + nd] = dydp * xF - dxdp * yF;
-            pCE[f * np + nd] = -dyds * xF + dxds * yF;
+            const double met[4] = {dxds, dxdp, dyds, dydp};
+            adv_volume_flux(c[f], u, v, A.kappa, dx, dy, met, sCE[f * np + nd], pCE[f * np + nd]);
         }
     }
     __syncthreads();
@@ -264,14 +326,15 @@ __global__ __launch_bounds__(256) void k_adv_stage(AdvArgs A)
             const double nx = A.fnrm[nb], ny = A.fnrm[nb + n1], len = A.fnrm[nb + 2 * n1];
             const double u = A.fvel[(((size_t)e * 4 + sd) * 2 + 0) * n1 + k];
             const double v = A.fvel[(((size_t)e * 4 + sd) * 2 + 1) * n1 + k];
-            const double uN = u * nx + v * ny;
+            const double uN = __builtin_fma(u, nx, v * ny);
             for (int f = 0; f < NQ; ++f) {
                 const double ownC = trace1<N>(L, cE + f * np, sd, k);
                 const double ownX = trace1<N>(L, gxE + f * np, sd, k);
                 const double ownY = trace1<N>(L, gyE + f * np, sd, k);
-                double in, ex, dx, dy, sign = 1.0;
+                AdvSides o;
+                o.sign = 1.0;
                 if (info.x < 0) {
-                    in = ownC; ex = adv_external(info.x, f, A.t); dx = ownX; dy = ownY;
+                    o.in = ownC; o.ex = adv_external(info.x, f, A.t); o.dx = ownX; o.dy = ownY;
                 } else {
                     const int kk = side_flip(info.y) ? N - k : k;
                     const size_t ns = (size_t)info.x * 4 + side_nbr_side(info.y);
@@ -279,16 +342,12 @@ __global__ __launch_bounds__(256) void k_adv_stage(AdvArgs A)
                     const double nbX = A.trG[((ns * 2 + 0) * NQ + f) * n1 + kk];
                     const double nbY = A.trG[((ns * 2 + 1) * NQ + f) * n1 + kk];
                     if (side_primary(info.y)) {
-                        in = ownC; ex = nbC; dx = (ownX + nbX) * 0.5; dy = (ownY + nbY) * 0.5;
+                        o.in = ownC; o.ex = nbC; o.dx = (ownX + nbX) * 0.5; o.dy = (ownY + nbY) * 0.5;
                     } else {
-                        in = nbC; ex = ownC; dx = (nbX + ownX) * 0.5; dy = (nbY + ownY) * 0.5; sign = -1.0;
+                        o.in = nbC; o.ex = ownC; o.dx = (nbX + ownX) * 0.5; o.dy = (nbY + ownY) * 0.5; o.sign = -1.0;
                     }
                 }
-                const double jump = ex - in;
-                double fl = 0.5 * (uN * (ex + in) - fabs(uN) * jump);  // RiemannSolver :1756-1787
-                const double dcdn = dx * nx + dy * ny;
-                fl = fl - A.kappa * dcdn;
-                bfE[(sd * NQ + f) * n1 + k] = sign * (fl * len);
+                bfE[(sd * NQ + f) * n1 + k] = adv_side_flux(o, uN, nx, ny, len, A.kappa);
             }
         }
     }
@@ -296,17 +355,18 @@ __global__ __launch_bounds__(256) void k_adv_stage(AdvArgs A)
     if (act) {
         for (int f = 0; f < NQ; ++f) {
             double t1, t2;
-            dg_pair<N>(L, sCE + f * np + n1 * j, pCE + f * np + i, i, j, bfE[(1 * NQ + f) * n1 + j],
-                       bfE[(3 * NQ + f) * n1 + j], bfE[(2 * NQ + f) * n1 + i], bfE[(0 * NQ + f) * n1 + i], t1, t2);
-            double tend = (-t1 - t2) / J;
-            if (A.hasRelax) tend = tend + (A.relax[f * mstride + base] - c[f]) * A.rFac[f * mstride + base];
+            dg_lines<N>(L, sCE + f * np + n1 * j, pCE + f * np + i, i, j, t1, t2);
+            dg_lift<N>(L, i, j, bfE[(1 * NQ + f) * n1 + j], bfE[(3 * NQ + f) * n1 + j], bfE[(2 * NQ + f) * n1 + i],
+                       bfE[(0 * NQ + f) * n1 + i], t1, t2);
+            const double tend = adv_tendency(t1, t2, J, A.hasRelax, A.hasRelax ? A.relax[f * mstride + base] : 0.0,
+                                             A.hasRelax ? A.rFac[f * mstride + base] : 0.0, c[f]);
             if (A.mode == 1) {
                 A.tend[f * mstride + base] = tend;
             } else {
                 const double gold = (A.a != 0.0) ? A.G[f * mstride + base] : 0.0;
-                const double gv = A.a * gold + tend;
+                const double gv = __builtin_fma(A.a, gold, tend);
                 A.G[f * mstride + base] = gv;
-                const double qn = c[f] + A.gdt * gv;
+                const double qn = __builtin_fma(A.gdt, gv, c[f]);
                 A.c[f * mstride + base] = qn;
                 cE[f * np + nd] = qn;
             }
@@ -320,6 +380,262 @@ __global__ __launch_bounds__(256) void k_adv_stage(AdvArgs A)
             for (int f = 0; f < NQ; ++f)
                 A.trOut[(((size_t)e * 4 + sd) * NQ + f) * n1 + k] = trace1<N>(L, cE + f * np, sd, k);
         }
+    }
+}
+
+// ---- several RK3 steps in one launch, for models whose every element is
+// resident at once.  The launched stage is two kernels (4.6 us each with their
+// gaps for 10x10, N = 7: launch latency) that pass gradient, state and traces
+// through memory.  Here tracers, register and geometry stay in registers and
+// the two exchanges of a stage travel as tagged messages into the neighbours'
+// slots (persist.hpp); contractions that need no neighbour run while they are
+// under way.  One buffer each is enough: a neighbour sends its next tracer
+// traces only after my gradient traces, which I send after reading its
+// tracers, and its next gradient traces after my next tracers.  Measured, us a
+// stage: 10x10 N = 7 8.1 -> 3.4, 61x45 N = 4 of three tracers 19.2 -> 7.9,
+// 40x40 N = 3 of four 14.5 -> 6.0; a call of one step 26.8 -> 20.
+struct AdvStepsArgs {
+    PersistArgs P;
+    int nStages;
+    unsigned tag0;          // tag of the first stage
+    double tn, dt;
+    double a[3], b[3], gc[3];
+    double *cOut;
+    ll_quad *llC, *llG;     // [nE][NQ][4 n1], [nE][2 NQ][4 n1]
+    unsigned bytesC;        // of llC; llG has twice as many
+};
+
+template <int N, int NQ>
+__global__ __launch_bounds__(256) void k_adv_steps(AdvArgs A, AdvStepsArgs T)
+{
+    using S = Shape<N>;
+    constexpr int n1 = S::n1, np = S::np, epb = S::epb, ns4 = 4 * n1, kSide = (ns4 + np - 1) / np;
+    constexpr bool WL = 64 % np == 0;
+    __shared__ NodalLDS<N> L;
+    __shared__ double cs[epb * NQ * np], sx[epb * NQ * np], sy[epb * NQ * np], px[epb * NQ * np],
+        py[epb * NQ * np], bf[epb * 4 * 2 * NQ * n1];
+    __shared__ int stop;
+    if (threadIdx.x == 0) stop = persist_given_up(T.P);
+    stage_nodal<N, false>(L, A.nodal, nullptr, nullptr);
+    __syncthreads();
+    if (stop) return;  // an earlier launch of this model gave up: leave the state to the host
+    auto sync = [] {
+        if constexpr (WL) wave_sync();
+        else __syncthreads();
+    };
+    const int t = threadIdx.x, le = t / np, nd = t - le * np;
+    const int e = xcd_block(blockIdx.x, gridDim.x) * epb + le;
+    const bool act = le < epb && e < A.nE;
+    const int i = nd % n1, j = nd / n1;
+    const size_t mstride = (size_t)A.nE * np, base = act ? (size_t)e * np + nd : 0;
+    const int lo = (le < epb ? le : 0) * NQ * np;
+    double *bfE = bf + (le < epb ? le : 0) * 4 * 2 * NQ * n1;
+    const LLBuf llC(T.llC, T.bytesC), llG(T.llG, 2 * T.bytesC);
+    double c[NQ], G[NQ], met[4];
+    #pragma unroll
+    for (int k = 0; k < 4; ++k) met[k] = A.metric[k * mstride + base];
+    const double J = A.metric[4 * mstride + base], u = A.vel[base], v = A.vel[mstride + base];
+    #pragma unroll
+    for (int f = 0; f < NQ; ++f) {
+        c[f] = A.c[f * mstride + base];
+        G[f] = 0.0;
+        if (act) cs[lo + f * np + nd] = c[f];
+    }
+    // the thread's side nodes: descriptor, normal, normal velocity, own and neighbour's tracers
+    int2 info[kSide];
+    double nx[kSide], ny[kSide], len[kSide], uN[kSide], ownC[kSide][NQ], nbC[kSide][NQ], ownX[kSide][NQ], ownY[kSide][NQ];
+    bool side[kSide];
+    #pragma unroll
+    for (int q = 0; q < kSide; ++q) {
+        const int w = nd + q * np;
+        side[q] = act && w < ns4;
+        const int sd = side[q] ? w / n1 : 0, k = side[q] ? w - sd * n1 : 0;
+        const size_t es = (size_t)(act ? e : 0) * 4 + sd, nb = es * 3 * n1 + k;
+        info[q] = A.side[es];
+        nx[q] = A.fnrm[nb];
+        ny[q] = A.fnrm[nb + n1];
+        len[q] = A.fnrm[nb + 2 * n1];
+        uN[q] = __builtin_fma(A.fvel[(es * 2) * n1 + k], nx[q], A.fvel[(es * 2 + 1) * n1 + k] * ny[q]);
+    }
+    // byte offset of value f of the neighbour's side node that matches mine
+    auto dest = [&](int q, int nf, int f) {
+        const int w = nd + q * np, k = w % n1;
+        const int kk = side_nbr_side(info[q].y) * n1 + (side_flip(info[q].y) ? N - k : k);
+        return 16u * (((unsigned)info[q].x * nf + f) * ns4 + kk);
+    };
+    auto mine = [&](int q, int nf, int f) {
+        return side[q] ? 16u * (((unsigned)e * nf + f) * ns4 + nd + q * np) : 0u;
+    };
+    auto send_c = [&](unsigned tag) {
+        #pragma unroll
+        for (int q = 0; q < kSide; ++q) {
+            if (!side[q]) continue;
+            const int w = nd + q * np, sd = w / n1, k = w - sd * n1;
+            #pragma unroll
+            for (int f = 0; f < NQ; ++f) {
+                ownC[q][f] = trace1<N>(L, cs + lo + f * np, sd, k);
+                if (info[q].x >= 0) ll_store1(llC, dest(q, NQ, f), ownC[q][f], tag);
+            }
+        }
+    };
+    sync();
+    send_c(T.tag0);
+    int rk = 0;
+    double tStep = T.tn;
+    for (int st = 0, step = 0; st < T.nStages; ++st) {
+        #pragma clang fp contract(off)
+        const unsigned tag = T.tag0 + st;
+        const double time = tStep + (rk == 0 ? T.b[0] : rk == 1 ? T.b[1] : T.b[2]) * T.dt;
+        bool good = true;
+        // ---- contractions of the gradient
+        if (act) {
+            #pragma unroll
+            for (int f = 0; f < NQ; ++f) {
+                sx[lo + f * np + nd] = met[3] * c[f];
+                sy[lo + f * np + nd] = -(met[1] * c[f]);
+                px[lo + f * np + nd] = -(met[2] * c[f]);
+                py[lo + f * np + nd] = met[0] * c[f];
+            }
+        }
+        sync();
+        double x1[NQ], x2[NQ], y1[NQ], y2[NQ];
+        if (act) {
+            #pragma unroll
+            for (int f = 0; f < NQ; ++f) {
+                const int o = lo + f * np;
+                dg_lines<N>(L, sx + o + n1 * j, px + o + i, i, j, x1[f], x2[f]);
+                dg_lines<N>(L, sy + o + n1 * j, py + o + i, i, j, y1[f], y2[f]);
+            }
+        }
+        // ---- neighbours' tracers, central gradient flux
+        #pragma unroll
+        for (int q = 0; q < kSide; ++q) {
+            good = ll_wait(side[q] && info[q].x >= 0, T.P, [&] {
+                unsigned wrong = 0, w1;
+                #pragma unroll
+                for (int f = 0; f < NQ; ++f) {
+                    nbC[q][f] = ll_load1(llC, mine(q, NQ, f), tag, w1);
+                    wrong |= w1;
+                }
+                return (wrong >> 16) == 0;
+            }) && good;
+            if (side[q]) {
+                const int w = nd + q * np, sd = w / n1, k = w - sd * n1;
+                #pragma unroll
+                for (int f = 0; f < NQ; ++f) {
+                    const double ext = info[q].x < 0 ? adv_external(info[q].x, f, time) : 0.0;
+                    const double own[3] = {ownC[q][f], 0.0, 0.0}, nbr[3] = {nbC[q][f], 0.0, 0.0};
+                    const AdvSides o = adv_sides(info[q], own, nbr, ext);
+                    const double avg = 0.5 * (o.in + o.ex);
+                    bfE[((sd * 2 + 0) * NQ + f) * n1 + k] = o.sign * (avg * nx[q] * len[q]);
+                    bfE[((sd * 2 + 1) * NQ + f) * n1 + k] = o.sign * (avg * ny[q] * len[q]);
+                }
+            }
+        }
+        if constexpr (WL) {
+            if (!good) return;  // the whole wavefront, and no workgroup barrier follows
+            wave_sync();
+        } else {
+            if (__syncthreads_or(!good)) return;
+        }
+        // ---- gradient, its traces on their way, contravariant volume flux
+        double gx[NQ], gy[NQ];
+        if (act) {
+            #pragma unroll
+            for (int f = 0; f < NQ; ++f) {
+                dg_lift<N>(L, i, j, bfE[((1 * 2 + 0) * NQ + f) * n1 + j], bfE[((3 * 2 + 0) * NQ + f) * n1 + j],
+                           bfE[((2 * 2 + 0) * NQ + f) * n1 + i], bfE[((0 * 2 + 0) * NQ + f) * n1 + i], x1[f], x2[f]);
+                dg_lift<N>(L, i, j, bfE[((1 * 2 + 1) * NQ + f) * n1 + j], bfE[((3 * 2 + 1) * NQ + f) * n1 + j],
+                           bfE[((2 * 2 + 1) * NQ + f) * n1 + i], bfE[((0 * 2 + 1) * NQ + f) * n1 + i], y1[f], y2[f]);
+                gx[f] = (x1[f] + x2[f]) / J;
+                gy[f] = (y1[f] + y2[f]) / J;
+                // every lane is past its contractions: the flux arrays take the gradient and the volume flux
+                sx[lo + f * np + nd] = gx[f];
+                sy[lo + f * np + nd] = gy[f];
+            }
+        }
+        sync();
+        #pragma unroll
+        for (int q = 0; q < kSide; ++q) {
+            if (!side[q]) continue;
+            const int w = nd + q * np, sd = w / n1, k = w - sd * n1;
+            #pragma unroll
+            for (int f = 0; f < NQ; ++f) {
+                ownX[q][f] = trace1<N>(L, sx + lo + f * np, sd, k);
+                ownY[q][f] = trace1<N>(L, sy + lo + f * np, sd, k);
+                if (info[q].x >= 0) {
+                    ll_store1(llG, dest(q, 2 * NQ, f), ownX[q][f], tag);
+                    ll_store1(llG, dest(q, 2 * NQ, NQ + f), ownY[q][f], tag);
+                }
+            }
+        }
+        sync();  // every lane is past its traces of the gradient
+        if (act) {
+            #pragma unroll
+            for (int f = 0; f < NQ; ++f)
+                adv_volume_flux(c[f], u, v, A.kappa, gx[f], gy[f], met, sx[lo + f * np + nd], px[lo + f * np + nd]);
+        }
+        sync();
+        if (act) {
+            #pragma unroll
+            for (int f = 0; f < NQ; ++f)
+                dg_lines<N>(L, sx + lo + f * np + n1 * j, px + lo + f * np + i, i, j, x1[f], x2[f]);
+        }
+        // ---- neighbours' gradients, upwind and diffusive flux
+        #pragma unroll
+        for (int q = 0; q < kSide; ++q) {
+            double nb[2 * NQ];
+            good = ll_wait(side[q] && info[q].x >= 0, T.P, [&] {
+                unsigned wrong = 0, w1;
+                #pragma unroll
+                for (int f = 0; f < 2 * NQ; ++f) {
+                    nb[f] = ll_load1(llG, mine(q, 2 * NQ, f), tag, w1);
+                    wrong |= w1;
+                }
+                return (wrong >> 16) == 0;
+            }) && good;
+            if (side[q]) {
+                const int w = nd + q * np, sd = w / n1, k = w - sd * n1;
+                #pragma unroll
+                for (int f = 0; f < NQ; ++f) {
+                    const double ext = info[q].x < 0 ? adv_external(info[q].x, f, time) : 0.0;
+                    const double own[3] = {ownC[q][f], ownX[q][f], ownY[q][f]}, nbr[3] = {nbC[q][f], nb[f], nb[NQ + f]};
+                    bfE[(sd * NQ + f) * n1 + k] = adv_side_flux(adv_sides(info[q], own, nbr, ext), uN[q], nx[q], ny[q], len[q],
+                                                                A.kappa);
+                }
+            }
+        }
+        if constexpr (WL) {
+            if (!good) return;
+            wave_sync();
+        } else {
+            if (__syncthreads_or(!good)) return;
+        }
+        // ---- lift, source, RK3 update
+        if (act) {
+            const double ra = rk == 0 ? T.a[0] : rk == 1 ? T.a[1] : T.a[2];
+            const double gdt = (rk == 0 ? T.gc[0] : rk == 1 ? T.gc[1] : T.gc[2]) * T.dt;
+            #pragma unroll
+            for (int f = 0; f < NQ; ++f) {
+                dg_lift<N>(L, i, j, bfE[(1 * NQ + f) * n1 + j], bfE[(3 * NQ + f) * n1 + j], bfE[(2 * NQ + f) * n1 + i],
+                           bfE[(0 * NQ + f) * n1 + i], x1[f], x2[f]);
+                const double tend = adv_tendency(x1[f], x2[f], J, A.hasRelax, A.hasRelax ? A.relax[f * mstride + base] : 0.0,
+                                                 A.hasRelax ? A.rFac[f * mstride + base] : 0.0, c[f]);
+                G[f] = __builtin_fma(ra, ra != 0.0 ? G[f] : 0.0, tend);
+                c[f] = __builtin_fma(gdt, G[f], c[f]);
+                cs[lo + f * np + nd] = c[f];
+            }
+        }
+        if (++rk == 3) {
+            rk = 0;
+            tStep = T.tn + (double)(++step) * T.dt;
+        }
+        sync();
+        if (st + 1 < T.nStages) send_c(tag + 1);
+    }
+    if (act) {
+        #pragma unroll
+        for (int f = 0; f < NQ; ++f) T.cOut[f * mstride + base] = c[f];
     }
 }
 
@@ -341,6 +657,11 @@ struct self_adv2d_s {
     int *pnode = nullptr;
     int cur = 0;
     bool trValid = false, ready = false, hasRelax = false;
+    // several steps in one launch (k_adv_steps): second state, messages, launches in flight
+    double *cAlt = nullptr;
+    ll_quad *ll = nullptr;
+    unsigned tag = 0;
+    ResidentRuns runs;
 };
 
 namespace {
@@ -433,6 +754,104 @@ int stage(self_adv2d_s *h, double t, int m, int mode)
     return SELF_OK;
 }
 
+// ---- several steps in one launch
+size_t ll_quads(const self_adv2d_s *h) { return h->nE * (size_t)h->nq * 4 * h->n1; }  // of the tracers' messages
+
+template <int N, int NQ>
+int resident_blocks(self_adv2d_s *h, int &perCu, size_t &blocks)
+{
+    perCu = persist_blocks_per_cu(reinterpret_cast<const void *>(&k_adv_steps<N, NQ>), 256);
+    blocks = (size_t)agrid<N>(h->nE);
+    return perCu >= 1 && 32 * ll_quads(h) < (1u << 31) && blocks <= (size_t)perCu * persist_cus(h->device);
+}
+
+// Buffers of the resident form, at creation, where the model fits it; without
+// memory for them it keeps to the ordinary launches, which need none.
+int resident_prepare(self_adv2d_s *h)
+{
+    int fits = 0, perCu = 0;
+    size_t blocks = 0;
+    ADV_DISPATCH(h->N, h->nq, fits = (resident_blocks<NN, QQ>(h, perCu, blocks)));
+    h->runs.off = !fits;
+    if (!fits) return SELF_OK;
+    if (hipMalloc(reinterpret_cast<void **>(&h->cAlt), sizeof(double) * h->nq * h->nE * h->np) != hipSuccess ||
+        hipMalloc(reinterpret_cast<void **>(&h->ll), 3 * sizeof(ll_quad) * ll_quads(h)) != hipSuccess ||
+        hipMalloc(reinterpret_cast<void **>(&h->runs.status), sizeof(int)) != hipSuccess) {
+        (void)hipGetLastError();
+        h->runs.off = true;
+        return SELF_OK;
+    }
+    SELF_HIP(hipMemsetAsync(h->ll, 0, 3 * sizeof(ll_quad) * ll_quads(h), h->stream));  // tags start at 1
+    SELF_HIP(hipMemsetAsync(h->runs.status, 0, sizeof(int), h->stream));
+    return SELF_OK;
+}
+
+template <int N, int NQ>
+int launch_steps(self_adv2d_s *h, double tn, int nSteps)
+{
+    int perCu = 0;
+    size_t blocks = 0;
+    (void)resident_blocks<N, NQ>(h, perCu, blocks);
+    AdvArgs A = adv_args(h);
+    AdvStepsArgs T{};
+    T.P = h->runs.args();
+    T.nStages = 3 * nSteps;
+    T.tag0 = h->tag + 1;
+    T.tn = tn;
+    T.dt = h->dt;
+    for (int m = 0; m < 3; ++m) {
+        T.a[m] = kRkA[m];
+        T.b[m] = kRkB[m];
+        T.gc[m] = kRkG[m];
+    }
+    T.cOut = h->cAlt;
+    T.llC = h->ll;
+    T.llG = h->ll + ll_quads(h);
+    T.bytesC = (unsigned)(sizeof(ll_quad) * ll_quads(h));
+    {
+        PersistGate gate(h->device, h->stream, (int)blocks, perCu);
+        if (gate.rc) return gate.rc;
+        hipLaunchKernelGGL((k_adv_steps<N, NQ>), dim3((unsigned)blocks), dim3(256), 0, h->stream, A, T);
+        SELF_HIP(hipGetLastError());
+        if (int rc = gate.launched()) return rc;
+    }
+    h->tag += 3u * (unsigned)nSteps;
+    h->runs.launched(nSteps, tn, h->c);
+    std::swap(h->c, h->cAlt);
+    h->trValid = false;
+    return SELF_OK;
+}
+
+int launched_steps(self_adv2d_s *h, double tn, int nSteps)
+{
+    int rc = SELF_OK;
+    if (!h->trValid) {
+        if ((rc = launch_c_traces(h, h->tr[h->cur]))) return rc;
+        h->trValid = true;
+    }
+    for (int s = 0; s < nSteps && !rc; ++s) {
+        const double t0 = tn + s * h->dt;
+        for (int m = 0; m < 3 && !rc; ++m) rc = stage(h, t0 + kRkB[m] * h->dt, m, 0);
+    }
+    return rc;
+}
+
+// Every call but a further ForwardStepRK3 settles the launches in flight first.
+int settle(self_adv2d_s *h)
+{
+    if (h->runs.pending.empty()) return SELF_OK;
+    SELF_HIP(hipSetDevice(h->device));
+    std::vector<ResidentRuns::Run> again;
+    if (int rc = h->runs.settle(h->stream, again)) return rc;
+    if (again.empty()) return SELF_OK;
+    if (h->c != again[0].in) std::swap(h->c, h->cAlt);
+    h->trValid = false;
+    for (const auto &r : again)
+        if (int rc = launched_steps(h, r.t0, r.steps)) return rc;
+    SELF_HIP(hipStreamSynchronize(h->stream));
+    return SELF_OK;
+}
+
 void to_dev(const double *src, double *dst, size_t nE, int nf, int np)
 {
     for (size_t e = 0; e < nE; ++e)
@@ -469,7 +888,7 @@ try {
     const size_t nE = h->nE, np = h->np, n1 = h->n1, nq = h->nq;
     auto fail = [&](hipError_t e) {
         void *p[] = {h->nodal, h->c, h->G, h->tend, h->grad, h->vel, h->velTr, h->fvel, h->metric, h->fnrm,
-                     h->tr[0], h->tr[1], h->trG, h->relax, h->rFac, h->side, h->pnode};
+                     h->tr[0], h->tr[1], h->trG, h->relax, h->rFac, h->side, h->pnode, h->cAlt, h->ll, h->runs.status};
         for (void *q : p)
             if (q) (void)hipFree(q);
         if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -518,6 +937,7 @@ try {
     if (e == hipSuccess) e = hipMemset(h->vel, 0, sizeof(double) * 2 * nE * np);
     if (e == hipSuccess) e = hipMemset(h->fvel, 0, sizeof(double) * nE * 8 * n1);
     if (e != hipSuccess) return fail(e);
+    if (resident_prepare(h) != SELF_OK) return fail(hipErrorUnknown);
     *out = h;
     return SELF_OK;
 }
@@ -529,7 +949,7 @@ int self_adv2d_destroy(self_adv2d_t h)
     (void)hipSetDevice(h->device);
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     void *p[] = {h->nodal, h->c, h->G, h->tend, h->grad, h->vel, h->velTr, h->fvel, h->metric, h->fnrm,
-                 h->tr[0], h->tr[1], h->trG, h->relax, h->rFac, h->side, h->pnode};
+                 h->tr[0], h->tr[1], h->trG, h->relax, h->rFac, h->side, h->pnode, h->cAlt, h->ll, h->runs.status};
     for (void *q : p)
         if (q) (void)hipFree(q);
     if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -543,6 +963,7 @@ int self_adv2d_set_field(self_adv2d_t h, int field, const double *data)
 try {
     SELF_REQUIRE(h && data, SELF_ERR_ARG, "null argument");
     SELF_HIP(hipSetDevice(h->device));
+    if (int rc = settle(h)) return rc;
     SELF_HIP(hipStreamSynchronize(h->stream));
     const size_t nE = h->nE, np = h->np;
     const int nf = field == 1 ? 2 : h->nq;
@@ -582,6 +1003,7 @@ int self_adv2d_get_field(self_adv2d_t h, int field, double *data)
 try {
     SELF_REQUIRE(h && data, SELF_ERR_ARG, "null argument");
     SELF_HIP(hipSetDevice(h->device));
+    if (int rc = settle(h)) return rc;
     SELF_HIP(hipStreamSynchronize(h->stream));
     const size_t nE = h->nE, np = h->np;
     size_t nq = h->nq;
@@ -608,18 +1030,22 @@ int self_adv2d_global_time_derivative(self_adv2d_t h, double t)
 {
     SELF_REQUIRE(h, SELF_ERR_ARG, "null handle");
     SELF_HIP(hipSetDevice(h->device));
-    int rc = launch_c_traces(h, h->tr[h->cur]);
+    int rc = settle(h);
+    if (!rc) rc = launch_c_traces(h, h->tr[h->cur]);
     if (rc) return rc;
     h->trValid = true;
     return stage(h, t, -1, 1);
 }
 
 int self_adv2d_forward_step_rk3(self_adv2d_t h, double tn, int nSteps, double *elapsed_ms)
-{
+try {
     SELF_REQUIRE(h && nSteps >= 0, SELF_ERR_ARG, "bad arguments");
     SELF_HIP(hipSetDevice(h->device));
     int rc = SELF_OK;
-    if (!h->trValid) {
+    const bool resident = !h->runs.off && nSteps >= 1;
+    if (!resident || elapsed_ms || h->runs.pending.size() >= 64)
+        if ((rc = settle(h))) return rc;
+    if (!resident && !h->trValid) {
         if ((rc = launch_c_traces(h, h->tr[h->cur]))) return rc;
         h->trValid = true;
     }
@@ -629,9 +1055,10 @@ int self_adv2d_forward_step_rk3(self_adv2d_t h, double tn, int nSteps, double *e
         SELF_HIP(hipEventCreate(&e1));
         SELF_HIP(hipEventRecord(e0, h->stream));
     }
-    for (int s = 0; s < nSteps && !rc; ++s) {
-        const double t0 = tn + s * h->dt;
-        for (int m = 0; m < 3 && !rc; ++m) rc = stage(h, t0 + kRkB[m] * h->dt, m, 0);
+    if (resident && !h->runs.off) {
+        ADV_DISPATCH(h->N, h->nq, rc = (launch_steps<NN, QQ>(h, tn, nSteps)));
+    } else {
+        rc = launched_steps(h, tn, nSteps);
     }
     if (elapsed_ms) {
         SELF_HIP(hipEventRecord(e1, h->stream));
@@ -641,9 +1068,15 @@ int self_adv2d_forward_step_rk3(self_adv2d_t h, double tn, int nSteps, double *e
         *elapsed_ms = ms;
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
+        const int gaveUp = h->runs.gaveUp;
+        const auto t0 = std::chrono::steady_clock::now();
+        if (!rc) rc = settle(h);
+        if (h->runs.gaveUp != gaveUp)  // the steps ran (again) in there
+            *elapsed_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     }
     return rc;
 }
+SELF_CATCH_ALL
 
 // WritePickup_Advection (AdvectionClass.f90:2040-2103)
 int self_adv2d_write_pickup(self_adv2d_t h, const char *path)
@@ -679,7 +1112,7 @@ int self_adv2d_synchronize(self_adv2d_t h)
 {
     SELF_REQUIRE(h, SELF_ERR_ARG, "null handle");
     SELF_HIP(hipStreamSynchronize(h->stream));
-    return SELF_OK;
+    return settle(h);
 }
 
 }  // extern "C"

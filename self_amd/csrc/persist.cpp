@@ -71,6 +71,25 @@ unsigned persist_spin_limit()
     return 2000;
 }
 
+int ResidentRuns::settle(hipStream_t s, std::vector<Run> &again)
+{
+    again.clear();
+    if (pending.empty()) return SELF_OK;
+    int bad = 0;
+    SELF_HIP(hipMemcpyAsync(&bad, status, sizeof(int), hipMemcpyDeviceToHost, s));
+    SELF_HIP(hipStreamSynchronize(s));
+    std::vector<Run> done;
+    done.swap(pending);
+    if (bad == 0) return SELF_OK;
+    if (++gaveUp >= 4) off = true;
+    SELF_HIP(hipMemsetAsync(status, 0, sizeof(int), s));
+    size_t first = 0;
+    while (first < done.size() && done[first].launch != bad) ++first;
+    SELF_REQUIRE(first < done.size(), SELF_ERR_HIP, "a resident launch gave up and cannot be found (%d)", bad);
+    again.assign(done.begin() + (long)first, done.end());
+    return SELF_OK;
+}
+
 // Alone on the device, `blocks` <= perCu x CUs workgroups of one kernel all
 // become resident.  Beside others, by shares of a CU: a workgroup of share s
 // finds no room only if every CU has more than 1 - s in use, that is, if the

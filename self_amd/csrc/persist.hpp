@@ -30,6 +30,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <vector>
+
 #include "common.hpp"
 
 namespace self {
@@ -145,6 +147,26 @@ __device__ __forceinline__ bool ll_wait(bool need, const PersistArgs &P, F attem
 int persist_blocks_per_cu(const void *kernel, int threads);
 int persist_cus(int device);
 unsigned persist_spin_limit();
+
+// Launches of resident time steps that are not yet known to have finished.  One
+// that gave up left its input as it was and made the later ones return at
+// once: settle() waits for them and lists the runs to do over by ordinary
+// launches.  After several such launches `off` is set: beside much other work
+// on the device it happens again.
+struct ResidentRuns {
+    struct Run {
+        int launch, steps;
+        double t0;
+        double *in;  // the state the run began with
+    };
+    int *status = nullptr;
+    int launches = 0, gaveUp = 0;
+    bool off = false;
+    std::vector<Run> pending;
+    PersistArgs args() const { return {status, launches + 1, persist_spin_limit()}; }
+    void launched(int steps, double t0, double *in) { pending.push_back({++launches, steps, t0, in}); }
+    int settle(hipStream_t s, std::vector<Run> &again);
+};
 
 // Admission of one launch of `blocks` workgroups, `perCu` of which fit a CU.
 // The gate keeps the process's resident launches from taking each other's CUs:

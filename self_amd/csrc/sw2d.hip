@@ -1262,21 +1262,13 @@ struct self_sw2d_s {
     hipGraphExec_t graphExec = nullptr;
     SWKernelArgs graphArgs[6];
     int graphDims[4] = {0, 0, 0, 0};
-    // several steps in one launch (k_sw_steps): second state buffer, exchange
-    // words, status word, launches not yet known to have finished
-    struct Pending {
-        int launch, steps;
-        double *qIn;
-    };
+    // several steps in one launch (k_sw_steps): second state buffer, messages,
+    // launches in flight (off also where the buffers could not be had)
     double *qAlt = nullptr;
     ll_quad *ll = nullptr;
-    int *status = nullptr;
-    int launches = 0;
     unsigned tag = 0;
     bool llClear = false;
-    int gaveUp = 0;           // launches that gave up
-    bool persistOff = false;  // after several, or where the buffers could not be had
-    std::vector<Pending> pending;
+    ResidentRuns runs;
 };
 
 namespace {
@@ -1300,7 +1292,7 @@ void free_all(self_sw2d_s *h)
         if (p) (void)hipFree(p);
     if (h->qAlt) (void)hipFree(h->qAlt);
     if (h->ll) (void)hipFree(h->ll);
-    if (h->status) (void)hipFree(h->status);
+    if (h->runs.status) (void)hipFree(h->runs.status);
 }
 
 // fills A member by member (callers that compare argument blocks bytewise
@@ -1557,22 +1549,22 @@ template <int N, bool MIXED>
 int steps_ready(self_sw2d_s *h, bool &ok, int &perCu, size_t &blocks)
 {
     ok = false;
-    if (h->persistOff) return SELF_OK;
+    if (h->runs.off) return SELF_OK;
     perCu = persist_blocks_per_cu(reinterpret_cast<const void *>(&k_sw_steps<N, MIXED>), 256);
     blocks = (size_t)grid_fused<N>(h->nE, 1) * h->members;
     if (perCu < 1 || sizeof(ll_quad) * ll_quads(h) >= (1u << 31) || blocks > (size_t)perCu * persist_cus(h->device))
         return SELF_OK;
     const size_t nq = 3 * (size_t)h->members * h->nE * h->np;
     if ((!h->qAlt && dalloc(h, &h->qAlt, nq) != SELF_OK) || (!h->ll && dalloc(h, &h->ll, 2 * ll_quads(h)) != SELF_OK) ||
-        (!h->status && dalloc(h, &h->status, 1) != SELF_OK)) {
+        (!h->runs.status && dalloc(h, &h->runs.status, 1) != SELF_OK)) {
         (void)hipGetLastError();  // no memory for it: the ordinary launches need none
         persist_free(h);
-        h->persistOff = true;
+        h->runs.off = true;
         return SELF_OK;
     }
     if (!h->llClear) {  // tags start at 1
         SELF_HIP(hipMemsetAsync(h->ll, 0, 2 * sizeof(ll_quad) * ll_quads(h), h->stream));
-        SELF_HIP(hipMemsetAsync(h->status, 0, sizeof(int), h->stream));
+        SELF_HIP(hipMemsetAsync(h->runs.status, 0, sizeof(int), h->stream));
         h->llClear = true;
         h->tag = 0;
     }
@@ -1591,9 +1583,7 @@ int launch_steps(self_sw2d_s *h, int nSteps, bool &taken)
     SWKernelArgs A = make_args(h);
     A.trIn = h->tr[h->trCur];
     SWStepsArgs T{};
-    T.P.status = h->status;
-    T.P.launch = h->launches + 1;
-    T.P.limit = persist_spin_limit();
+    T.P = h->runs.args();
     T.nStages = 3 * nSteps;
     T.tag0 = h->tag + 1;
     for (int m = 0; m < 3; ++m) { T.a[m] = kRkA[m]; T.gc[m] = kRkG[m]; }
@@ -1608,9 +1598,8 @@ int launch_steps(self_sw2d_s *h, int nSteps, bool &taken)
         SELF_HIP(hipGetLastError());
         if (int rc = gate.launched()) return rc;
     }
-    h->launches = T.P.launch;
     h->tag += 3u * (unsigned)nSteps;
-    h->pending.push_back({T.P.launch, nSteps, h->q});
+    h->runs.launched(nSteps, 0.0, h->q);
     std::swap(h->q, h->qAlt);
     h->trValid = false;
     return SELF_OK;
@@ -1641,29 +1630,18 @@ int steps_persistent(self_sw2d_s *h, int nSteps, bool &taken)
     return rc;
 }
 
-// Every call but a further ForwardStepRK3 settles the launches in flight
-// first: one that gave up left its input state as it was and made the later
-// ones return at once, so their steps run again through ordinary launches.
+// Every call but a further ForwardStepRK3 settles the launches in flight first.
 int settle(self_sw2d_s *h)
 {
-    if (h->pending.empty()) return SELF_OK;
+    if (h->runs.pending.empty()) return SELF_OK;
     SELF_HIP(hipSetDevice(h->device));
-    int bad = 0;
-    SELF_HIP(hipMemcpyAsync(&bad, h->status, sizeof(int), hipMemcpyDeviceToHost, h->stream));
-    SELF_HIP(hipStreamSynchronize(h->stream));
-    std::vector<self_sw2d_s::Pending> done;
-    done.swap(h->pending);
-    if (bad == 0) return SELF_OK;
-    // beside much other work on the device it will happen again
-    if (++h->gaveUp >= 4) h->persistOff = true;
-    SELF_HIP(hipMemsetAsync(h->status, 0, sizeof(int), h->stream));
-    size_t first = 0;
-    while (first < done.size() && done[first].launch != bad) ++first;
-    SELF_REQUIRE(first < done.size(), SELF_ERR_HIP, "a resident launch gave up and cannot be found (%d)", bad);
-    if (h->q != done[first].qIn) std::swap(h->q, h->qAlt);
+    std::vector<ResidentRuns::Run> again;
+    if (int rc = h->runs.settle(h->stream, again)) return rc;
+    if (again.empty()) return SELF_OK;
+    if (h->q != again[0].in) std::swap(h->q, h->qAlt);
     h->trValid = false;
-    for (; first < done.size(); ++first)
-        for (int s = 0; s < done[first].steps; ++s)
+    for (const auto &r : again)
+        for (int s = 0; s < r.steps; ++s)
             if (int rc = step_fused(h)) return rc;
     SELF_HIP(hipStreamSynchronize(h->stream));
     return SELF_OK;
@@ -2148,14 +2126,14 @@ int self_sw2d_forward_step_rk3(self_sw2d_t h, double tn, int nSteps)
     if (rc) return rc;
     SELF_REQUIRE(nSteps >= 0, SELF_ERR_ARG, "negative step count");
     int s = 0;
-    if (h->d.form == SELF_FUSED && h->useGraph && !h->persistOff && nSteps >= 2 &&
+    if (h->d.form == SELF_FUSED && h->useGraph && !h->runs.off && nSteps >= 2 &&
         fused_groups(h->groups, h->nE, 0) == 1) {
         // at most kMaxSteps a launch; launches in flight stay countable
         constexpr int kMaxSteps = 1 << 16;
         bool taken = true;
         while (s < nSteps && taken) {
-            if (h->pending.size() >= 64 && (rc = settle(h))) return rc;
-            if (h->persistOff) break;
+            if (h->runs.pending.size() >= 64 && (rc = settle(h))) return rc;
+            if (h->runs.off) break;
             const int n = std::min(nSteps - s, kMaxSteps);
             if ((rc = steps_persistent(h, n, taken))) return rc;
             if (taken) s += n;
@@ -2191,10 +2169,10 @@ int self_sw2d_forward_step_rk3_timed(self_sw2d_t h, double tn, int nSteps, doubl
     float ms = 0.0f;
     SELF_HIP(hipEventElapsedTime(&ms, h->ev0, h->ev1));
     *elapsed_ms = ms;
-    const int gaveUp = h->gaveUp;
+    const int gaveUp = h->runs.gaveUp;
     const auto t0 = std::chrono::steady_clock::now();
     rc = settle(h);
-    if (h->gaveUp != gaveUp)  // the steps ran (again) in there
+    if (h->runs.gaveUp != gaveUp)  // the steps ran (again) in there
         *elapsed_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     return rc;
 }
