@@ -37,6 +37,7 @@
 #include "dg3d_device.hpp"
 #include "layout.hpp"
 #include "mfma.hpp"
+#include "reduce.hpp"
 
 namespace self {
 void cofactor3(const double *m, int dir, double out[3]);
@@ -188,19 +189,44 @@ __device__ __forceinline__ void adv3_filter_prefetch(const Adv3Args &A, int ec, 
     }
 }
 
+// The limiter of one element and tracer from its energies (every thread of the
+// element decides alike; one of them records the state).
+template <int NQ>
+__device__ __forceinline__ bool adv3_limiter(const Adv3Args &A, double E1, double E2, int f, int e, int stage, bool record,
+                                             const Adv3FilterPre<NQ> &P)
+{
+    const double dE1 = E1 - P.E1[f], dE2 = E2 - P.E2[f], xi = E2 / E1;
+    double lim = P.lim[f];
+    if (dE2 > 0.0 && fabs(dE1) / dE2 > 1.0) lim = xi;
+    else if (dE2 < 0.0) lim = xi;
+    else if (stage > 1) lim = P.limPrev[f];
+    const bool filter = xi > 1.05 * lim;
+    if (record) {
+        A.lim[((size_t)(stage - 1) * NQ + f) * A.nE + e] = lim;
+        A.E1[(size_t)f * A.nE + e] = E1;
+        A.E2[(size_t)f * A.nE + e] = E2;
+        if (filter && A.nFiltered) atomicAdd(A.nFiltered, 1u);
+    }
+    return filter;
+}
+
 // DoTheAdaptiveFiltering for the element group's state in cs (LDS) at the
 // given stage; t1, t2, t3 are LDS scratch of the size of cs; red holds
-// 2 n2 per element.  Replaces cs (and the register copy c) when the
+// 2 (n2 + n1) per element.  Replaces cs (and the register copy c) when the
 // limiter asks for it.  Every thread of the block must call it.  pre: the
-// element's stored energies and limiters loaded in advance (or null).
+// element's stored energies and limiters, loaded in advance.
+// The energies were one thread's sum of 2 (N+1)^2 line integrals while the
+// workgroup waited; now rows of lines, then n1 row sums by every thread
+// (stage of 19x13x11, N = 5, two tracers: 38.7 -> 35.7 us).
 template <int N, int NQ>
 __device__ void adaptive_filter(const Adv3Args &A, const Nodal3<N> &L, double *cs, double *t1, double *t2,
-                                double *t3, double *red, int *flag, int le, int nd, int e, bool act, double J,
-                                double (&c)[NQ], int stage, const Adv3FilterPre<NQ> *pre = nullptr)
+                                double *t3, double *red, int le, int nd, int e, bool act, double J,
+                                double (&c)[NQ], int stage, const Adv3FilterPre<NQ> &pre)
 {
     using S = Shape3<N>;
     constexpr int n1 = S::n1, n2 = S::n2, np = S::np;
     const int i = nd % n1, j = (nd / n1) % n1, k = nd / n2;
+    double *line = red + le * 2 * (n2 + n1), *rows = line + 2 * n2;
     for (int f = 0; f < NQ; ++f) {
         const int o = (le * NQ + f) * np;
         double cf = 0.0;
@@ -228,7 +254,7 @@ __device__ void adaptive_filter(const Adv3Args &A, const Nodal3<N> &L, double *c
             t3[o + nd] = (d * d) * J;    // marginally resolved energy density
         }
         __syncthreads();
-        // line integrals in s, weighted by w_p w_q (the reference's order)
+        // line integrals in s, weighted by w_p w_q
         if (act && nd < n2) {
             const int jj = nd % n1, kk = nd / n1;
             double d1 = 0.0, d2 = 0.0;
@@ -237,35 +263,71 @@ __device__ void adaptive_filter(const Adv3Args &A, const Nodal3<N> &L, double *c
                 d1 = __builtin_fma(t1[o + m + n1 * nd], L.w[m], d1);
                 d2 = __builtin_fma(t3[o + m + n1 * nd], L.w[m], d2);
             }
-            red[le * 2 * n2 + nd] = d1 * L.w[jj] * L.w[kk];
-            red[le * 2 * n2 + n2 + nd] = d2 * L.w[jj] * L.w[kk];
+            line[nd] = d1 * L.w[jj] * L.w[kk];
+            line[n2 + nd] = d2 * L.w[jj] * L.w[kk];
         }
         __syncthreads();
-        if (act && nd == 0) {
-            double E1 = 0.0, E2 = 0.0;
-            for (int q = 0; q < n2; ++q) {
-                E1 = E1 + red[le * 2 * n2 + q];
-                E2 = E2 + red[le * 2 * n2 + n2 + q];
+        for (int q = nd; act && q < 2 * n1; q += np) {
+            double sum = line[q * n1];
+            #pragma unroll
+            for (int m = 1; m < n1; ++m) sum += line[q * n1 + m];
+            rows[q] = sum;
+        }
+        __syncthreads();
+        if (act) {
+            double E1 = rows[0], E2 = rows[n1];
+            #pragma unroll
+            for (int m = 1; m < n1; ++m) {
+                E1 += rows[m];
+                E2 += rows[n1 + m];
             }
-            const size_t ei = (size_t)f * A.nE + e;
-            const double E1o = pre ? pre->E1[f] : A.E1[ei], E2o = pre ? pre->E2[f] : A.E2[ei];
-            const double dE1 = E1 - E1o, dE2 = E2 - E2o, xi = E2 / E1;
-            const size_t li = ((size_t)(stage - 1) * NQ + f) * A.nE + e;
-            double lim = pre ? pre->lim[f] : A.lim[li];
-            if (dE2 > 0.0 && fabs(dE1) / dE2 > 1.0) lim = xi;
-            else if (dE2 < 0.0) lim = xi;
-            else if (stage > 1) lim = pre ? pre->limPrev[f] : A.lim[li - (size_t)NQ * A.nE];
-            A.lim[li] = lim;
-            A.E1[ei] = E1;
-            A.E2[ei] = E2;
-            const int fl = (xi > 1.05 * lim) ? 1 : 0;
-            flag[le * NQ + f] = fl;
-            if (fl && A.nFiltered) atomicAdd(A.nFiltered, 1u);
+            if (adv3_limiter<NQ>(A, E1, E2, f, e, stage, nd == 0, pre)) {
+                cs[o + nd] = cf;
+                c[f] = cf;
+            }
         }
-        __syncthreads();
-        if (act && flag[le * NQ + f]) {
-            cs[o + nd] = cf;
-            c[f] = cf;
+    }
+    __syncthreads();
+}
+
+// The same at N = 7 on the matrix cores (512 threads, one element): the three
+// passes in the order q, s, p, so that the last leaves each thread its own
+// node's filtered value and one workgroup barrier separates them; energies as
+// wavefront sums of weighted node values, then eight partials by every thread.
+template <int NQ>
+__device__ __forceinline__ void adaptive_filter_mf(const Adv3Args &A, const Mf3Ops &F, double w3, double *cs, double *t1,
+                                                   double *t2, double *red, int nd, int ln, int wv, int tl, int e, double J,
+                                                   double (&c)[NQ], int stage, const Adv3FilterPre<NQ> &pre)
+{
+    #pragma unroll
+    for (int f = 0; f < NQ; ++f) t1[f * kMf3Size + mf3_q_node(wv, tl)] = mf3_q(F, cs + f * kMf3Size, wv, tl);
+    __syncthreads();
+    double cf[NQ];
+    #pragma unroll
+    for (int f = 0; f < NQ; ++f) t2[f * kMf3Size + ln] = mf3_s(F, t1 + f * kMf3Size, wv, tl);
+    wave_sync();  // the plane k = wv is this wavefront's
+    #pragma unroll
+    for (int f = 0; f < NQ; ++f) {
+        cf[f] = mf3_p(F, t2 + f * kMf3Size, wv, tl);
+        const double d = c[f] - cf[f], jw = J * w3;
+        const double E1 = wave_sum_dpp((cf[f] * cf[f]) * jw), E2 = wave_sum_dpp((d * d) * jw);
+        if (tl == 0) {
+            red[f * 16 + wv] = E1;
+            red[f * 16 + 8 + wv] = E2;
+        }
+    }
+    __syncthreads();
+    #pragma unroll
+    for (int f = 0; f < NQ; ++f) {
+        double E1 = red[f * 16], E2 = red[f * 16 + 8];
+        #pragma unroll
+        for (int m = 1; m < 8; ++m) {
+            E1 += red[f * 16 + m];
+            E2 += red[f * 16 + 8 + m];
+        }
+        if (adv3_limiter<NQ>(A, E1, E2, f, e, stage, nd == 0, pre)) {
+            cs[f * kMf3Size + ln] = cf[f];
+            c[f] = cf[f];
         }
     }
     __syncthreads();
@@ -316,8 +378,7 @@ __global__ __launch_bounds__(Shape3<N>::threads) void k_adv3d_prologue(Adv3Args 
     constexpr int n2 = S::n2, np = S::np, epb = S::epb;
     __shared__ Nodal3<N> L;
     __shared__ double cs[epb * NQ * np], t1[epb * NQ * np], t2[epb * NQ * np], t3[epb * NQ * np];
-    __shared__ double red[epb * 2 * n2];
-    __shared__ int flag[epb * NQ];
+    __shared__ double red[epb * 2 * (n2 + S::n1)];
     stage_nodal3<N>(L, A.nodal);
     const int t = threadIdx.x, le = t / np, nd = t - le * np;
     const int e = blockIdx.x * epb + le;
@@ -333,7 +394,9 @@ __global__ __launch_bounds__(Shape3<N>::threads) void k_adv3d_prologue(Adv3Args 
     }
     __syncthreads();
     if (A.useFilter) {
-        adaptive_filter<N, NQ>(A, L, cs, t1, t2, t3, red, flag, le, nd, e, act, J, c, A.stage);
+        Adv3FilterPre<NQ> fp;
+        adv3_filter_prefetch<NQ>(A, act ? e : 0, A.stage, fp);
+        adaptive_filter<N, NQ>(A, L, cs, t1, t2, t3, red, le, nd, e, act, J, c, A.stage, fp);
         if (act)
             for (int f = 0; f < NQ; ++f) A.c[f * ms + base] = c[f];
     }
@@ -343,28 +406,56 @@ __global__ __launch_bounds__(Shape3<N>::threads) void k_adv3d_prologue(Adv3Args 
 // PREC 0: FP64 contractions; 1: FP32 matrix-core contractions; 2: split-BF16
 // matrix-core contractions (mfma.hpp).  State, register, geometry, face
 // fluxes, lift, Jacobian and the filter are FP64 in every form.
+// N = 7 in FP64 runs on the matrix cores.  Bound: HBM, 738 MB a stage at
+// 32x32x16 and one tracer, 154 us at the rate of a large copy; the LDS reads of
+// the line sums (16 b64 a node and contraction, ~80 us) and the occupancy they
+// left were added to that.  Measured a stage: 192.8 -> 158.7 us there, 55.2 ->
+// 41.1 at 16x16x8 and two tracers, 11.2 -> 8.1 at 8x8x8.  Three workgroups of
+// 512 threads a CU (80 registers): two gave 194.7, three 172.0, and 158.7 with
+// the element and wavefront numbers in scalar registers; four spill (215.5).
 template <int N, int NQ, int PREC>
-__global__ __launch_bounds__(Shape3<N>::threads, 4) void k_adv3d_stage(Adv3Args A)
+__global__ __launch_bounds__(Shape3<N>::threads, (N == 7 && NQ == 1 && PREC == 0) ? 6 : 4) void k_adv3d_stage(Adv3Args A)
 {
     using S = Shape3<N>;
     constexpr int n1 = S::n1, n2 = S::n2, np = S::np, epb = S::epb;
     constexpr int nT = PREC ? epb * NQ * 3 * np : 1;
+    // FP64 at N = 7: contractions, traces and filter on the matrix cores
+    constexpr bool MF = N == 7 && PREC == 0;
+    constexpr int nl = MF ? kMf3Size : np;  // LDS values of one tracer
     __shared__ Nodal3<N> L;
-    __shared__ double cs[epb * NQ * np], Fs[epb * NQ * np], Fp[epb * NQ * np], Fq[epb * NQ * np];
+    __shared__ double cs[epb * NQ * nl], Fs[epb * NQ * nl], Fp[epb * NQ * nl], Fq[epb * NQ * nl];
     __shared__ double bf[epb * 6 * NQ * n2];
-    __shared__ double red[epb * 2 * n2];
-    __shared__ int flag[epb * NQ];
+    __shared__ double red[epb * 2 * (n2 + n1)];
+    static_assert(epb * 2 * (n2 + n1) >= 16 * NQ, "wavefront energies of every tracer");
     __shared__ float Tm[nT];
     __shared__ float Df[64];
     __shared__ double rs[n1];
     constexpr int nF = epb * 6 * n2;                       // face nodes of the element group
     constexpr int FQ = (nF + S::threads - 1) / S::threads;  // per thread
-    const int t = threadIdx.x, le = t / np, nd = t - le * np;
+    const int t = threadIdx.x, le = MF ? 0 : t / np, wv = __builtin_amdgcn_readfirstlane(t >> 6), tl = t & 63;
+    const int nd = MF ? 64 * wv + lane_node<7>(tl) : t - le * np;
     const int e = blockIdx.x * epb + le;
-    const bool act = le < epb && e < A.nE;
+    const bool act = MF || (le < epb && e < A.nE);  // one workgroup an element at N = 7
     const int i = nd % n1, j = (nd / n1) % n1, k = nd / n2;
+    const int ln = MF ? mf3_at(i, j, k) : nd;
     const size_t ms = (size_t)A.nE * np, base = act ? (size_t)e * np + nd : 0;
     const int ec = act ? e : 0;
+    // the thread's q-th face node: element slot, side, node (slot 0, side 0,
+    // node 0 and false for none)
+    auto face = [&](int q, int &l2, int &sd, int &node) {
+        if constexpr (MF) {
+            l2 = 0;
+            const bool has = mf3_face(wv, tl, sd, node);
+            return has;
+        } else {
+            const int w = t + q * S::threads, wc = w < nF ? w : 0;
+            l2 = wc / (6 * n2);
+            const int rem = wc - l2 * 6 * n2;
+            sd = rem / n2;
+            node = rem - sd * n2;
+            return w < nF;
+        }
+    };
     // Loads first, in the order they are used, with no thread-dependent
     // branch around them (a thread without a node or face node loads from a
     // clamped valid address and ignores the value): the nodal constants,
@@ -376,9 +467,8 @@ __global__ __launch_bounds__(Shape3<N>::threads, 4) void k_adv3d_stage(Adv3Args 
     double fuN[FQ], flen[FQ], fnbr[FQ][NQ];
     #pragma unroll
     for (int q = 0; q < FQ; ++q) {
-        const int w = t + q * S::threads;
-        const int wc = w < nF ? w : 0;
-        const int l2 = wc / (6 * n2), rem = wc - l2 * 6 * n2, sd = rem / n2, node = rem - sd * n2;
+        int l2, sd, node;
+        (void)face(q, l2, sd, node);
         const int e2 = blockIdx.x * epb + l2, e2c = e2 < A.nE ? e2 : 0;
         finfo[q] = A.side[(size_t)e2c * 6 + sd];
         const size_t fb = (((size_t)e2c * 6 + sd) * 2) * n2 + node;
@@ -405,9 +495,8 @@ __global__ __launch_bounds__(Shape3<N>::threads, 4) void k_adv3d_stage(Adv3Args 
     }
     #pragma unroll
     for (int q = 0; q < FQ; ++q) {
-        const int w = t + q * S::threads;
-        const int wc = w < nF ? w : 0;
-        const int rem = wc % (6 * n2), node = rem % n2;
+        int l2, sd, node;
+        (void)face(q, l2, sd, node);
         const int2 info = finfo[q];
         int na = node % n1, nb = node / n1;
         if (info.x >= 0) s3_map<N>(info.y, node % n1, node / n1, na, nb);
@@ -430,7 +519,7 @@ __global__ __launch_bounds__(Shape3<N>::threads, 4) void k_adv3d_stage(Adv3Args 
     }
     if (act) {
         for (int f = 0; f < NQ; ++f) {
-            const int o = (le * NQ + f) * np + nd;
+            const int o = (le * NQ + f) * nl + ln;
             cs[o] = c[f];
             Fs[o] = as * c[f];
             Fp[o] = ap * c[f];
@@ -438,6 +527,19 @@ __global__ __launch_bounds__(Shape3<N>::threads, 4) void k_adv3d_stage(Adv3Args 
         }
     }
     __syncthreads();
+    [[maybe_unused]] double mfTr[NQ];
+    if constexpr (MF) {  // operands are read again where needed: fewer registers
+        Mf3Ops M;
+        Mf3Lag ML;
+        mf3_load(M, L.D, tl);
+        mf3_load_lag(ML, L.lL, L.lR, tl);
+        #pragma unroll
+        for (int f = 0; f < NQ; ++f) {
+            const double tq = mf3_q(M, Fq + f * nl, wv, tl);
+            Fq[f * nl + mf3_q_node(wv, tl)] = tq;  // read back after the next barrier
+            mfTr[f] = mf3_trace(ML, cs + f * nl, wv, tl);
+        }
+    }
     if (PREC) {  // matrix-core contractions of the volume fluxes, one 16x16 tile per wavefront
         const int wave = threadIdx.x >> 6, nw = blockDim.x >> 6, nTiles = epb * NQ * 3 * 2;
         for (int tile = wave; tile < nTiles; tile += nw) {
@@ -450,16 +552,17 @@ __global__ __launch_bounds__(Shape3<N>::threads, 4) void k_adv3d_stage(Adv3Args 
     // face fluxes (EdgeFlux :1237-1341 with RiemannSolver :1595-1620)
     #pragma unroll
     for (int q = 0; q < FQ; ++q) {
-        const int w = t + q * S::threads;
-        if (w >= nF) continue;
-        const int l2 = w / (6 * n2), rem = w - l2 * 6 * n2, sd = rem / n2, node = rem - sd * n2;
+        int l2, sd, node;
+        if (!face(q, l2, sd, node)) continue;
         const int e2 = blockIdx.x * epb + l2;
         if (e2 >= A.nE) continue;
         const int a = node % n1, b = node / n1;
         const int2 info = finfo[q];
         const double uN = fuN[q], len = flen[q];
         for (int f = 0; f < NQ; ++f) {
-            const double own = trace3<N>(L, cs + (l2 * NQ + f) * np, sd, a, b);
+            double own;
+            if constexpr (MF) own = mfTr[f];
+            else own = trace3<N>(L, cs + (l2 * NQ + f) * np, sd, a, b);
             double in, ex, sign = 1.0;
             if (info.x < 0) {
                 in = own;
@@ -477,11 +580,17 @@ __global__ __launch_bounds__(Shape3<N>::threads, 4) void k_adv3d_stage(Adv3Args 
     __syncthreads();
     // weak divergence + lift (MappedTimeDerivative :1345-1562), source, RK3
     if (act) {
+        [[maybe_unused]] Mf3Ops M;
+        if constexpr (MF) mf3_load(M, L.D, tl);
         const double *bfE = bf + le * 6 * NQ * n2;
         for (int f = 0; f < NQ; ++f) {
-            const int o = (le * NQ + f) * np;
+            const int o = (le * NQ + f) * nl;
             double ts = 0.0, tp = 0.0, tq = 0.0;
-            if (PREC == 0) {
+            if constexpr (MF) {
+                ts = mf3_s(M, Fs + o, wv, tl);
+                tp = mf3_p(M, Fp + o, wv, tl);
+                tq = Fq[o + ln];
+            } else if (PREC == 0) {
                 #pragma unroll
                 for (int m = 0; m < n1; ++m) {
                     ts = __builtin_fma(L.D[i + n1 * m], Fs[o + m + n1 * (j + n1 * k)], ts);
@@ -518,13 +627,32 @@ __global__ __launch_bounds__(Shape3<N>::threads, 4) void k_adv3d_stage(Adv3Args 
     adv3_filter_prefetch<NQ>(A, ec, A.filterNext, fp);
     __syncthreads();  // all reads of cs / Fs / Fp / Fq for the divergence are done
     if (act)
-        for (int f = 0; f < NQ; ++f) cs[(le * NQ + f) * np + nd] = c[f];
+        for (int f = 0; f < NQ; ++f) cs[(le * NQ + f) * nl + ln] = c[f];
     __syncthreads();
-    if (A.filterNext)
-        adaptive_filter<N, NQ>(A, L, cs, Fs, Fp, Fq, red, flag, le, nd, e, act, J, c, A.filterNext, &fp);
-    if (act)
+    if constexpr (MF) {
+        if (A.filterNext) {
+            Mf3Ops F;
+            mf3_load(F, L.F1, tl);
+            adaptive_filter_mf<NQ>(A, F, L.w[i] * L.w[j] * L.w[k], cs, Fs, Fp, red, nd, ln, wv, tl, e, J, c, A.filterNext, fp);
+        }
+        #pragma unroll
         for (int f = 0; f < NQ; ++f) A.c[f * ms + base] = c[f];
-    write_traces<N, NQ>(A, L, cs);
+        int sd, node;
+        const bool has = mf3_face(wv, tl, sd, node);
+        Mf3Lag ML;
+        mf3_load_lag(ML, L.lL, L.lR, tl);
+        #pragma unroll
+        for (int f = 0; f < NQ; ++f) {
+            const double v = mf3_trace(ML, cs + f * nl, wv, tl);
+            if (has) A.trOut[(((size_t)e * 6 + sd) * NQ + f) * n2 + node] = v;
+        }
+    } else {
+        if (A.filterNext)
+            adaptive_filter<N, NQ>(A, L, cs, Fs, Fp, Fq, red, le, nd, e, act, J, c, A.filterNext, fp);
+        if (act)
+            for (int f = 0; f < NQ; ++f) A.c[f * ms + base] = c[f];
+        write_traces<N, NQ>(A, L, cs);
+    }
 }
 
 // u.n and |n| of each face node in its face's primary orientation, from the

@@ -6,6 +6,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "dg2d_device.hpp"
+
 namespace self {
 
 // Side descriptor (int2) of one element side: x = neighbour element (>= 0)
@@ -56,6 +58,110 @@ __device__ __forceinline__ double face_trace3(const double *lL, const double *lR
     #pragma unroll
     for (int m = 1; m < n1; ++m) acc = __builtin_fma(l[m], q[off + m * stride], acc);
     return acc;
+}
+
+// ---- N = 7 on the FP64 matrix cores (Mf in dg2d_device.hpp).  An element's 512
+// nodes are eight wavefronts, wavefront wv the plane k = wv with the node
+// order of the instruction's layout: contractions in s and p give each lane its
+// own node's value, 2 LDS reads instead of 16.  A contraction in q runs on the
+// plane j = wv; its results go back through LDS, in place (a plane j = wv is
+// read and written by wavefront wv only, in order).  Face traces take four
+// instructions a wavefront: the four sides that cross plane k = wv in lanes of
+// result rows 0 and 1, bottom and top of plane j = wv in rows 2 and 3.
+// Rows 9 and planes 72 apart: the operand reads of all three directions then
+// spread over the LDS banks (8 and 64: two lanes a bank in s, four in q).
+constexpr int kMf3Size = 576;
+
+__device__ __forceinline__ int mf3_at(int i, int j, int k)
+{
+    return i + 9 * j + 72 * k;
+}
+
+struct Mf3Ops {
+    double a[2], b[2];  // left operand (rows), right operand (transposed)
+};
+
+__device__ __forceinline__ void mf3_load(Mf3Ops &M, const double *D, int tl)
+{
+    const MfLane<7> a(tl);
+    #pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        M.a[q] = D[(4 * a.bi + a.c) + 8 * (4 * q + a.k)];
+        M.b[q] = D[(4 * a.bj + a.c) + 8 * (4 * q + a.k)];
+    }
+}
+
+__device__ __forceinline__ double mf3_s(const Mf3Ops &M, const double *X, int wv, int tl)
+{
+    const MfLane<7> a(tl);
+    double r = 0.0;
+    #pragma unroll
+    for (int q = 0; q < 2; ++q)
+        r = __builtin_amdgcn_mfma_f64_4x4x4f64(M.a[q], X[mf3_at(4 * q + a.k, 4 * a.bj + a.c, wv)], r, 0, 0, 0);
+    return r;
+}
+
+__device__ __forceinline__ double mf3_p(const Mf3Ops &M, const double *X, int wv, int tl)
+{
+    const MfLane<7> a(tl);
+    double r = 0.0;
+    #pragma unroll
+    for (int q = 0; q < 2; ++q)
+        r = __builtin_amdgcn_mfma_f64_4x4x4f64(X[mf3_at(4 * a.bi + a.c, 4 * q + a.k, wv)], M.b[q], r, 0, 0, 0);
+    return r;
+}
+
+// q contraction on plane j = wv: the result's node is mf3_q_node
+__device__ __forceinline__ double mf3_q(const Mf3Ops &M, const double *X, int wv, int tl)
+{
+    const MfLane<7> a(tl);
+    double r = 0.0;
+    #pragma unroll
+    for (int q = 0; q < 2; ++q)
+        r = __builtin_amdgcn_mfma_f64_4x4x4f64(M.a[q], X[mf3_at(4 * a.bj + a.c, wv, 4 * q + a.k)], r, 0, 0, 0);
+    return r;
+}
+
+// its place in the array
+__device__ __forceinline__ int mf3_q_node(int wv, int tl)
+{
+    const MfLane<7> a(tl);
+    return mf3_at(4 * a.bj + a.c, wv, 4 * a.bi + a.k);
+}
+
+// left operand of the traces: rows 0 and 2 left, 1 and 3 right interpolation
+struct Mf3Lag {
+    double v[2];
+};
+
+__device__ __forceinline__ void mf3_load_lag(Mf3Lag &M, const double *lL, const double *lR, int tl)
+{
+    const MfLane<7> a(tl);
+    #pragma unroll
+    for (int q = 0; q < 2; ++q) M.v[q] = (a.c & 1 ? lR : lL)[4 * q + a.k];
+}
+
+// side and node of the lane's face node; false where it has none
+__device__ __forceinline__ bool mf3_face(int wv, int tl, int &sd, int &node)
+{
+    const MfLane<7> a(tl);
+    sd = a.k < 2 ? (a.bj ? 2 * a.k : 3 - 2 * a.k) : a.k + 2;
+    node = (4 * a.bi + a.c) + 8 * wv;
+    return a.k < 2 || a.bj == 0;
+}
+
+__device__ __forceinline__ double mf3_trace(const Mf3Lag &M, const double *X, int wv, int tl)
+{
+    const MfLane<7> a(tl);
+    const int n = 4 * a.bi + a.c;
+    double u = 0.0, v = 0.0;
+    #pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int m = 4 * q + a.k;
+        u = __builtin_amdgcn_mfma_f64_4x4x4f64(M.v[q], X[a.bj ? mf3_at(n, m, wv) : mf3_at(m, n, wv)], u, 0, 0, 0);
+        v = __builtin_amdgcn_mfma_f64_4x4x4f64(M.v[q], X[mf3_at(n, wv, m)], v, 0, 0, 0);
+    }
+    return a.k < 2 ? u : v;
 }
 
 }  // namespace self
