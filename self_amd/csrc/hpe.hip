@@ -38,6 +38,8 @@
 //     exactly opposite fluxes), the weak divergence of the contravariant
 //     fluxes in s, p, q with the lift, 1/J, then the RK3 or AB2 update of
 //     u, v, b, or the tendency alone.
+// At N = 7 both run on the FP64 matrix cores (k_hpe_columns_mf,
+// k_hpe_stage_mf), the column's running sums folded into the matrices.
 
 #include <cmath>
 #include <cstdlib>
@@ -333,6 +335,172 @@ __global__ __launch_bounds__(HShape<N>::threads, 4) void k_hpe_columns(HpeArgs A
     }
 }
 
+// N = 7 on the matrix cores (Mf3Ops).  One loop: iteration l integrates the
+// pressure of layer nL-1-l and the vertical velocity of layer l, three
+// barriers for both.  Wavefront wv owns plane k = wv of the lateral
+// derivatives and plane j = wv of everything along the column, where lane and
+// running value stay in registers: the increments' running sums are folded on
+// the host into one matrix each (HpeColumn), and the face value that starts
+// the next layer into one more row, so no thread sums for others.  The
+// face values of w are formed one iteration later, behind the next barrier.
+// Bound: HBM, 433 MB at 24x21x12 (90 us at the rate of a large copy).  Measured
+// there: 113.7 us for the two sweeps of k_hpe_columns, 85.9 here; with the
+// operands kept in registers (24 spilled) the stage as a whole was slower
+// than before (292 us against 284).
+struct HpeColumn {  // in the nodal buffer after Iup
+    double Cdn[64], Cup[64];  // [k][m], running sums of Idn from the top, of Iup from the bottom
+    double td[8], tu[8];      // their face values: lL . Cdn, lR . Cup
+    double sl, sr;            // the face value of a constant
+};
+
+__global__ __launch_bounds__(512, 4) void k_hpe_columns_mf(HpeArgs A)
+{
+    constexpr int n1 = 8, n2 = 64, np = 512;
+    __shared__ HNodal<7> L;
+    __shared__ double su[kMf3Size], sv[kMf3Size], Fs[kMf3Size], Fp[kMf3Size], Fq[kMf3Size];
+    __shared__ double sb[kMf3Size], sp[kMf3Size], sw[kMf3Size], sd[kMf3Size];
+    __shared__ double fF[6 * n2], floor0[n2];
+    stage_hnodal<7>(L, A.nodal);
+    constexpr int nC = sizeof(HpeColumn) / sizeof(double);
+    __shared__ HpeColumn C;
+    if (threadIdx.x < nC) ((double *)&C)[threadIdx.x] = A.nodal[3 * n2 + 3 * n1 + threadIdx.x];
+    const int hE = blockIdx.x, tl = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const size_t nEp = (size_t)A.nE * np;
+    const double *u = A.sol, *v = A.sol + nEp, *b = A.sol + 2 * nEp;
+    double *w = A.sol + 3 * nEp, *p = A.sol + 4 * nEp;
+    const int qi = 4 * MfLane<7>(tl).bj + MfLane<7>(tl).c;
+    // uniform address plus 32-bit lane offset: no 64-bit lane addresses to keep
+    const unsigned on = 64 * wv + lane_node<7>(tl), qh = qi + 8 * wv, qn = qh + 64 * (4 * MfLane<7>(tl).bi + MfLane<7>(tl).k);
+    int sdn, node;
+    (void)mf3_face(wv, tl, sdn, node);
+    const unsigned of = sdn * 4 * n2 + node, ot = sdn * 3 * n2 + node;
+    // the next layers' loads are in flight while the current ones are integrated
+    struct Layer {
+        double b, p, hp, u, v, g0, g1, g3, g4, g6, g7, J, h, nx, ny, nz, len;
+    };
+    const auto load = [&](int l) {
+        Layer Y;
+        const size_t ep = (size_t)hE + (size_t)A.nH * (A.nL - 1 - l), e = (size_t)hE + (size_t)A.nH * l;
+        Y.b = (b + ep * np)[qn];
+        Y.p = A.diagnoseP ? 0.0 : (p + ep * np)[qn];
+        Y.hp = (A.height + ep * n2)[qh];
+        Y.u = (u + e * np)[on];
+        Y.v = (v + e * np)[on];
+        const double *g = A.geo + e * np;
+        Y.g0 = g[on];
+        Y.g1 = (g + nEp)[on];
+        Y.g3 = (g + 3 * nEp)[on];
+        Y.g4 = (g + 4 * nEp)[on];
+        Y.g6 = (g + 6 * nEp)[on];
+        Y.g7 = (g + 7 * nEp)[on];
+        Y.J = (g + 9 * nEp)[on];
+        Y.h = (A.height + e * n2)[qh];
+        const double *nr = A.nrm + e * 6 * 4 * n2;
+        Y.nx = nr[of];
+        Y.ny = (nr + n2)[of];
+        Y.nz = (nr + 2 * n2)[of];
+        Y.len = (nr + 3 * n2)[of];
+        return Y;
+    };
+    Layer Ynx = load(0);
+    double baseP = 0.0, baseW = 0.0;
+    __syncthreads();
+    for (int l = 0; l < A.nL; ++l) {
+        const size_t ep = (size_t)hE + (size_t)A.nH * (A.nL - 1 - l), e = (size_t)hE + (size_t)A.nH * l;
+        // A lane number that the compiler cannot follow over iterations: the
+        // addresses and operands derived from it are formed again, not kept
+        // in registers (they spilled, and a spilled value's load waits for
+        // the layer loads in flight).
+        const bool first = l == 0;
+        int lane = tl;
+        asm volatile("" : "+v"(lane));
+        const MfLane<7> a(lane);
+        const int i = lane_node<7>(lane) % n1, j = lane_node<7>(lane) / n1, k = wv;
+        const int ln = mf3_at(i, j, k), qi = 4 * a.bj + a.c, ql = mf3_q_node(wv, lane);  // own node; plane j = wv
+        const int row = 4 * a.bi + a.c;  // of a left operand
+        int sdn, node;
+        const bool has = mf3_face(wv, lane, sdn, node);
+        const Layer &X = Ynx;
+        su[ln] = X.u;
+        sv[ln] = X.v;
+        Fs[ln] = X.g0 * X.u + X.g1 * X.v;
+        Fp[ln] = X.g3 * X.u + X.g4 * X.v;
+        Fq[ln] = X.g6 * X.u + X.g7 * X.v;
+        sb[ql] = X.b;
+        const Layer Y = X;  // J, heights and face normal are used below
+        if (l + 1 < A.nL) Ynx = load(l + 1);
+        double pv = Y.p;
+        if (A.diagnoseP) {
+            wave_sync();  // plane j = wv is this wavefront's
+            double acc = 0.0, top = 0.0;
+            #pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const double x = sb[mf3_at(qi, wv, 4 * q + a.k)];
+                acc = __builtin_amdgcn_mfma_f64_4x4x4f64(C.Cdn[row * n1 + 4 * q + a.k], x, acc, 0, 0, 0);
+                top = __builtin_amdgcn_mfma_f64_4x4x4f64(C.td[4 * q + a.k], x, top, 0, 0, 0);
+            }
+            pv = __builtin_fma(Y.hp, acc, baseP);
+            baseP = __builtin_fma(Y.hp, top, C.sl * baseP);
+            (p + ep * np)[qn] = pv;
+        }
+        sp[ql] = pv;
+        __syncthreads();
+        Mf3Lag ML;
+        mf3_load_lag(ML, L.lL, L.lR, lane);
+        {
+            const double ub = mf3_trace(ML, su, wv, lane), vb = mf3_trace(ML, sv, wv, lane);
+            const double un = ub * Y.nx + vb * Y.ny;
+            if (has) fF[sdn * n2 + node] = un * Y.len;
+            if (first && has && sdn == 4) floor0[node] = -un / Y.nz;
+            const double bt = mf3_trace(ML, sb, wv, lane), pt = mf3_trace(ML, sp, wv, lane);
+            const double wt = !first ? mf3_trace(ML, sw, wv, lane) : 0.0;
+            if (has) {
+                double *o = A.tr + ep * 18 * n2;
+                o[ot] = bt;
+                (o + 2 * n2)[ot] = pt;
+                if (!first) (A.tr + ((e - A.nH) * 18 + 1) * n2)[ot] = wt;
+            }
+        }
+        Mf3Ops M;
+        mf3_load(M, L.D, lane);
+        const double tq = mf3_q(M, Fq, wv, lane);
+        Fq[ql] = tq;  // read back after the barrier
+        __syncthreads();
+        {
+            double ds = mf3_s(M, Fs, wv, lane), dp = mf3_p(M, Fp, wv, lane), dq = Fq[ln];
+            ds += (fF[1 * n2 + j + n1 * k] * L.lR[i] + fF[3 * n2 + j + n1 * k] * L.lL[i]) * L.iw[i];
+            dp += (fF[2 * n2 + i + n1 * k] * L.lR[j] + fF[0 * n2 + i + n1 * k] * L.lL[j]) * L.iw[j];
+            dq += (fF[5 * n2 + i + n1 * j] * L.lR[k] + fF[4 * n2 + i + n1 * j] * L.lL[k]) * L.iw[k];
+            const double div = ((ds + dp) + dq) / Y.J;
+            sd[ln] = div;
+            if (A.divU) (A.divU + e * np)[on] = div;
+        }
+        __syncthreads();
+        {
+            if (first) baseW = floor0[qi + 8 * wv];
+            double acc = 0.0, top = 0.0;
+            #pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const double x = sd[mf3_at(qi, wv, 4 * q + a.k)];
+                acc = __builtin_amdgcn_mfma_f64_4x4x4f64(C.Cup[row * n1 + 4 * q + a.k], x, acc, 0, 0, 0);
+                top = __builtin_amdgcn_mfma_f64_4x4x4f64(C.tu[4 * q + a.k], x, top, 0, 0, 0);
+            }
+            const double wval = __builtin_fma(-Y.h, acc, baseW);
+            baseW = __builtin_fma(-Y.h, top, C.sr * baseW);
+            (w + e * np)[qn] = wval;
+            sw[ql] = wval;
+        }
+    }
+    __syncthreads();
+    {
+        const size_t e = (size_t)hE + (size_t)A.nH * (A.nL - 1);
+        Mf3Lag ML;
+        mf3_load_lag(ML, L.lL, L.lR, tl);
+        const double wt = mf3_trace(ML, sw, wv, tl);
+        if (mf3_face(wv, tl, sdn, node)) (A.tr + (e * 18 + 1) * n2)[ot] = wt;
+    }
+}
+
 // ---------------------------------------------------------------- stage
 // RiemannSolver (:2738-2778) with in = the primary side's state
 __device__ __forceinline__ void hpe_riemann(double bIn, double wIn, double pIn, double bEx, double wEx, double pEx,
@@ -486,6 +654,126 @@ __global__ __launch_bounds__(HShape<N>::threads) void k_hpe_stage(HpeArgs A)
     }
 }
 
+// N = 7 on the matrix cores (Mf3Ops): wavefront wv owns plane k = wv for s and
+// p and plane j = wv for q.  The element's own face values are formed from
+// the node values it has loaded anyway (the same instructions as in
+// k_hpe_columns_mf, so both sides of a face still see the same values).
+// Bound: HBM, 786 MB at 24x21x12 (164 us at the rate of a large copy, which
+// writes half of its bytes; this reads four in five).  Measured there: 174.0 us for
+// k_hpe_stage<7> (214 registers, one workgroup a CU), 139.9 here (84, two).
+__global__ __launch_bounds__(512, 4) void k_hpe_stage_mf(HpeArgs A)
+{
+    constexpr int n1 = 8, n2 = 64, np = 512, nl = kMf3Size;
+    __shared__ HNodal<7> L;
+    __shared__ double fl[9 * nl];             // [dir s,p,q][eq u,v,b][node]
+    __shared__ double sq[5 * nl];             // u, v, b, w, p
+    __shared__ double F[6 * 3 * n2];          // [side][eq][node]
+    const size_t e = blockIdx.x;
+    const int tl = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned on = 64 * wv + lane_node<7>(tl);
+    const int i = lane_node<7>(tl) % n1, j = lane_node<7>(tl) / n1, k = wv, ln = mf3_at(i, j, k);
+    const size_t NE = (size_t)A.nE, nEp = NE * np;
+    int sdn, node;
+    const bool has = mf3_face(wv, tl, sdn, node);
+    const int a = node % n1, bq = node / n1;
+    // loads first: nodal constants, face data, node values, the register,
+    // then the neighbours' face values addressed by the face data
+    HNodalRegs<7, 512> R;
+    hnodal_fetch<7, 512>(R, A.nodal, threadIdx.x);
+    const int2 info = (A.side + e * 6)[sdn];
+    double fd[6];
+    const unsigned of = sdn * 6 * n2 + node;
+    #pragma unroll
+    for (int c = 0; c < 6; ++c) fd[c] = (A.fdat + (e * 36 + c) * n2)[of];
+    double q5[5], geo[9];
+    #pragma unroll
+    for (int c = 0; c < 5; ++c) q5[c] = (A.sol + c * nEp + e * np)[on];
+    const double Bv = (A.Bvol + e * np)[on];
+    #pragma unroll
+    for (int c = 0; c < 9; ++c) geo[c] = (A.geo + c * nEp + e * np)[on];
+    const double Jv = (A.geo + 9 * nEp + e * np)[on];
+    double Gold[3] = {0.0, 0.0, 0.0};
+    asm volatile("" ::: "memory");  // the register after the others
+    if ((A.mode == 0 && !A.first) || A.mode == 2) {
+        #pragma unroll
+        for (int f = 0; f < 3; ++f) Gold[f] = (A.G + f * nEp + e * np)[on];
+    }
+    int na = a, nb = bq;
+    if (info.x >= 0) s3_map<7>(info.y, a, bq, na, nb);
+    // a boundary face node reads element 0's slot and ignores it
+    const size_t nbase = info.x >= 0 ? ((size_t)info.x * 6 + s3_nbr_side(info.y)) * 3 : 0;
+    const double *nbr = A.tr + nbase * n2 + na + n1 * nb;
+    const double bN = nbr[0], wN = nbr[n2], pN = nbr[2 * n2];
+    hnodal_put<7, 512>(L, R, threadIdx.x);
+    #pragma unroll
+    for (int c = 0; c < 5; ++c) sq[c * nl + ln] = q5[c];
+    const double Bw = Bv * q5[3];
+    #pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        fl[(3 * d + 0) * nl + ln] = geo[3 * d + 0] * q5[4];
+        fl[(3 * d + 1) * nl + ln] = geo[3 * d + 1] * q5[4];
+        fl[(3 * d + 2) * nl + ln] = geo[3 * d + 2] * Bw;
+    }
+    __syncthreads();
+    Mf3Lag ML;
+    mf3_load_lag(ML, L.lL, L.lR, tl);
+    const double bO = mf3_trace(ML, sq + 2 * nl, wv, tl), wO = mf3_trace(ML, sq + 3 * nl, wv, tl),
+                 pO = mf3_trace(ML, sq + 4 * nl, wv, tl);
+    double ub = 0.0, vb = 0.0;
+    if (__any(info.x == kSeaFloor)) {  // the whole wavefront forms them
+        ub = mf3_trace(ML, sq, wv, tl);
+        vb = mf3_trace(ML, sq + nl, wv, tl);
+    }
+    if (has) {
+        const double nx = fd[0], ny = fd[1], nz = fd[2], len = fd[3], Bf = fd[4], Wf = fd[5];
+        double f0, f1, f2, sgn = 1.0;
+        if (info.x >= 0) {
+            if (s3_primary(info.y)) {
+                hpe_riemann(bO, wO, pO, bN, wN, pN, nx, ny, nz, Bf, Wf, f0, f1, f2);
+            } else {
+                hpe_riemann(bN, wN, pN, bO, wO, pO, nx, ny, nz, Bf, Wf, f0, f1, f2);
+                sgn = -1.0;
+            }
+        } else {
+            double wE = 0.0;
+            if (info.x == kSeaFloor) wE = -(wO + 2.0 * (ub * nx + vb * ny)) / nz;
+            // NO_NORMAL_FLOW and SEA_FLOOR: zero exterior buoyancy, interior pressure
+            hpe_riemann(bO, wO, pO, 0.0, wE, pO, nx, ny, nz, Bf, Wf, f0, f1, f2);
+        }
+        F[(sdn * 3 + 0) * n2 + node] = sgn * (f0 * len);
+        F[(sdn * 3 + 1) * n2 + node] = sgn * (f1 * len);
+        F[(sdn * 3 + 2) * n2 + node] = sgn * (f2 * len);
+    }
+    Mf3Ops M;
+    mf3_load(M, L.D, tl);
+    #pragma unroll
+    for (int f = 0; f < 3; ++f) {
+        const double tq = mf3_q(M, fl + (6 + f) * nl, wv, tl);
+        fl[(6 + f) * nl + mf3_q_node(wv, tl)] = tq;  // read back after the barrier
+    }
+    __syncthreads();
+    #pragma unroll
+    for (int f = 0; f < 3; ++f) {
+        double ds = mf3_s(M, fl + f * nl, wv, tl), dp = mf3_p(M, fl + (3 + f) * nl, wv, tl), dq = fl[(6 + f) * nl + ln];
+        ds += (F[(1 * 3 + f) * n2 + j + n1 * k] * L.lR[i] + F[(3 * 3 + f) * n2 + j + n1 * k] * L.lL[i]) * L.iw[i];
+        dp += (F[(2 * 3 + f) * n2 + i + n1 * k] * L.lR[j] + F[(0 * 3 + f) * n2 + i + n1 * k] * L.lL[j]) * L.iw[j];
+        dq += (F[(5 * 3 + f) * n2 + i + n1 * j] * L.lR[k] + F[(4 * 3 + f) * n2 + i + n1 * j] * L.lL[k]) * L.iw[k];
+        const double tend = ((-ds - dp) - dq) / Jv;
+        double *G = A.G + f * nEp + e * np, *sol = A.sol + f * nEp + e * np;
+        if (A.mode == 1) {  // the time derivative alone
+            (A.tend + f * nEp + e * np)[on] = tend;
+        } else if (A.mode == 0) {  // RK3 stage
+            const double Gn = A.first ? tend : A.a * Gold[f] + tend;
+            G[on] = Gn;
+            sol[on] = q5[f] + A.gdt * Gn;
+        } else {  // AB2 step, G the previous tendency
+            const double Gn = 0.5 * (3.0 * tend - Gold[f]);
+            sol[on] = q5[f] + A.dt * Gn;
+            G[on] = tend;
+        }
+    }
+}
+
 #define HPE_DISPATCH_N(N_, CALL)                                                            \
     switch (N_) {                                                                           \
     case 1: { constexpr int NN = 1; CALL; } break;                                          \
@@ -531,8 +819,13 @@ int hpe_stage(self_hpe_s *h, int mode, int m, bool keepDivU)
     A.gdt = mode == 0 ? kRkG[m] * h->dt : 0.0;
     A.divU = keepDivU ? h->divU : nullptr;
     HPE_DISPATCH_N(h->N, {
-        hipLaunchKernelGGL((k_hpe_columns<NN>), dim3((unsigned)h->nH), dim3(HShape<NN>::threads), 0, h->stream, A);
-        hipLaunchKernelGGL((k_hpe_stage<NN>), dim3((unsigned)h->nE), dim3(HShape<NN>::threads), 0, h->stream, A);
+        if constexpr (NN == 7) {
+            hipLaunchKernelGGL(k_hpe_columns_mf, dim3((unsigned)h->nH), dim3(512), 0, h->stream, A);
+            hipLaunchKernelGGL(k_hpe_stage_mf, dim3((unsigned)h->nE), dim3(512), 0, h->stream, A);
+        } else {
+            hipLaunchKernelGGL((k_hpe_columns<NN>), dim3((unsigned)h->nH), dim3(HShape<NN>::threads), 0, h->stream, A);
+            hipLaunchKernelGGL((k_hpe_stage<NN>), dim3((unsigned)h->nE), dim3(HShape<NN>::threads), 0, h->stream, A);
+        }
     });
     SELF_HIP(hipGetLastError());
     return SELF_OK;
@@ -646,7 +939,26 @@ try {
             }
             for (int jj = 0; jj <= N; ++jj) I[kk * n1 + jj] *= 0.25 * (xiIp1 - xiI);
         }
-    std::vector<double> nod(3 * n1 * n1 + 3 * n1);
+    // running sums of the increments, their face values, a constant's face value
+    HpeColumn col{};
+    if (N == 7) {
+        for (int m = 0; m <= N; ++m) {
+            double run = 0.0;
+            for (int kk = N; kk >= 0; --kk) {
+                col.Cdn[kk * n1 + m] = run += Idn[kk * n1 + m];
+                col.td[m] += lagLeft[kk] * run;
+            }
+            run = 0.0;
+            for (int kk = 0; kk <= N; ++kk) {
+                col.Cup[kk * n1 + m] = run += Iup[kk * n1 + m];
+                col.tu[m] += lagRight[kk] * run;
+            }
+            col.sl += lagLeft[m];
+            col.sr += lagRight[m];
+        }
+    }
+    std::vector<double> nod(3 * n1 * n1 + 3 * n1 + sizeof(HpeColumn) / sizeof(double));
+    std::memcpy(nod.data() + 3 * n1 * n1 + 3 * n1, &col, sizeof(HpeColumn));
     std::memcpy(nod.data(), dMat, sizeof(double) * n1 * n1);
     std::memcpy(nod.data() + n1 * n1, qWeight, sizeof(double) * n1);
     std::memcpy(nod.data() + n1 * n1 + n1, lagLeft, sizeof(double) * n1);
