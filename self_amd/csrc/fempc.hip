@@ -6,6 +6,7 @@
 
 #include "fempc.hpp"
 #include "krylov.hpp"
+#include "reduce.hpp"
 
 namespace self {
 
@@ -13,32 +14,46 @@ namespace {
 
 constexpr int kPcThreads = 256;
 constexpr int kMaxWidth = 32;  // ELL slots per row (a node shared by up to 8 elements of the linear mesh)
-constexpr int kPcChunk = 8;    // ELL slots of a row loaded together
+constexpr int kPcChunk = 9;    // ELL slots of a row loaded together (a row of a quadrilateral mesh)
 
 __device__ __forceinline__ bool pc_skip(const PcState *st, const SolverState *outer)
 {
     return st->done || (outer && (outer->done || outer->innerExit));
 }
 
-// block sum of a double, result in thread 0 (fixed tree)
-__device__ __forceinline__ double pc_block_sum(double v)
+// block sum of a double, the same bits in every thread (fixed tree); lw: one
+// LDS slot a wavefront, not used again by the caller
+__device__ __forceinline__ double pc_block_sum(double v, double (&lw)[kPcThreads / 64])
 {
-    __shared__ double lw[kPcThreads / 64];
-    v = wave_sum(v);
+    v = wave_sum_dpp(v);
     if ((threadIdx.x & 63) == 0) lw[threadIdx.x >> 6] = v;
     __syncthreads();
-    double s = 0.0;
-    if (threadIdx.x == 0)
-        for (int q = 0; q < kPcThreads / 64; ++q) s += lw[q];
+    double s = lw[0];
+    #pragma unroll
+    for (int q = 1; q < kPcThreads / 64; ++q) s += lw[q];
     return s;
 }
 
-// one workgroup: fixed-order sum of the kPcParts partials
-__device__ __forceinline__ double pc_final_sum(const double *partials)
+// this thread's share of nParts partials
+__device__ __forceinline__ double pc_part(const double *partials, int nParts)
 {
     double v = 0.0;
-    for (int b = threadIdx.x; b < kPcParts; b += kPcThreads) v += partials[b];
-    return pc_block_sum(v);
+    for (int b = threadIdx.x; b < nParts; b += kPcThreads) v += partials[b];
+    return v;
+}
+
+// one workgroup: fixed-order sum of the partials
+__device__ __forceinline__ double pc_final_sum(const double *partials, int nParts)
+{
+    __shared__ double lw[kPcThreads / 64];
+    return pc_block_sum(pc_part(partials, nParts), lw);
+}
+
+// the workgroups a problem has rows for (more would sum the partials, and
+// leave more of them, for nothing)
+inline unsigned pc_grid(size_t n)
+{
+    return (unsigned)std::min<size_t>(kPcParts, (n + kPcThreads - 1) / kPcThreads);
 }
 
 // Solve_CGsemPreconditioner_2D (:704-711): r = b (MapFromOrigToPC), u = 0, |r|^2
@@ -55,15 +70,16 @@ __global__ __launch_bounds__(kPcThreads) void k_pc_start(const T *__restrict__ b
         x[i] = (T)0;
         acc += (double)bv * (double)bv;
     }
-    const double p = pc_block_sum(acc);
+    __shared__ double lw[kPcThreads / 64];
+    const double p = pc_block_sum(acc, lw);
     if (threadIdx.x == 0) partials[blockIdx.x] = p;
 }
 
-__global__ __launch_bounds__(kPcThreads) void k_pc_final_start(const double *partials, PcState *st,
+__global__ __launch_bounds__(kPcThreads) void k_pc_final_start(const double *partials, int nParts, PcState *st,
                                                                const SolverState *outer, int maxIters, double tol)
 {
     if (outer && (outer->done || outer->innerExit)) return;
-    const double S = pc_final_sum(partials);
+    const double S = pc_final_sum(partials, nParts);
     if (threadIdx.x == 0) {
         st->r0 = sqrt(S);
         st->rNorm = st->r0;
@@ -87,6 +103,10 @@ __global__ __launch_bounds__(kPcThreads) void k_pc_final_start(const double *par
 // stop test rNorm/r0 < TOL, num and c = num/den, :728-732) comes first:
 // every workgroup sums the partials itself in one fixed order, so all take
 // the same decision from the same bits; workgroup 0 records it.
+// Bound: latency, one memory round trip after another.  All that does not
+// depend on the decision is loaded before it: the state, the partials and the
+// row first, the gathered entries next, so two round trips are left of four.
+// 45x33, N = 5 (36 736 unknowns): 5.2 -> 4.6 us a launch.
 template <typename T>
 __global__ __launch_bounds__(kPcThreads) void k_pc_spmv(const T *__restrict__ r, const T *__restrict__ vOld,
                                                         T *__restrict__ vNew, T *__restrict__ z,
@@ -94,15 +114,46 @@ __global__ __launch_bounds__(kPcThreads) void k_pc_spmv(const T *__restrict__ r,
                                                         int width, size_t n, double *partials, PcState *st,
                                                         const SolverState *outer, int it)
 {
-    if (pc_skip(st, outer)) return;  // decided by an earlier launch: the same for every workgroup
     const bool first = it == 1;
+    // iteration 1 has no previous direction: it reads r in its place (and
+    // ignores it), so the same loads serve every iteration
+    const T *__restrict__ vPrev = first ? r : vOld;
+    const size_t i0 = (size_t)blockIdx.x * kPcThreads + threadIdx.x, stride = (size_t)gridDim.x * kPcThreads;
+    int cc[kPcChunk];
+    T vv[kPcChunk], rc[kPcChunk], vc[kPcChunk], ri, vi;
+    // the first kPcChunk slots of row i: column indices and values, then the
+    // gathered entries, all in flight together (slots past the width repeat the
+    // last one and are not added)
+    const auto slots = [&](int k0, size_t i) {
+        #pragma unroll
+        for (int u = 0; u < kPcChunk; ++u) {
+            const size_t kk = (size_t)min(k0 + u, width - 1) * n + i;
+            cc[u] = col[kk];
+            vv[u] = val[kk];
+        }
+    };
+    const auto gather = [&] {
+        #pragma unroll
+        for (int u = 0; u < kPcChunk; ++u) {
+            rc[u] = r[cc[u]];
+            vc[u] = vPrev[cc[u]];
+        }
+    };
+    const size_t ic = min(i0, n - 1);  // a thread without a row loads the last one
+    double part = first ? 0.0 : pc_part(partials + kPcParts, gridDim.x);
+    slots(0, ic);
+    ri = r[ic];
+    vi = vPrev[ic];
+    gather();
+    #pragma unroll
+    for (int u = 0; u < kPcChunk; ++u) asm volatile("" : "+v"(rc[u]), "+v"(vc[u]));
+    asm volatile("" : "+v"(ri), "+v"(vi), "+v"(part));
+    if (pc_skip(st, outer)) return;  // decided by an earlier launch: the same for every workgroup
+    __shared__ double lw[2][kPcThreads / 64];
     T beta = (T)0;
     if (!first) {
-        __shared__ double sS;
-        const double S0 = pc_final_sum(partials + kPcParts);
-        if (threadIdx.x == 0) sS = S0;
-        __syncthreads();
-        const double S = sS, rNorm = sqrt(S), den = st->numP[(it - 1) & 1];
+        const double S = pc_block_sum(part, lw[0]);
+        const double rNorm = sqrt(S), den = st->numP[(it - 1) & 1];
         const bool stop = rNorm / st->r0 < st->tol || it - 1 >= st->maxIters;
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             st->rNorm = rNorm;
@@ -117,84 +168,77 @@ __global__ __launch_bounds__(kPcThreads) void k_pc_spmv(const T *__restrict__ r,
         if (stop) return;
         beta = (T)(S / den);
     }
-    // iteration 1 has no previous direction: it reads r in its place (and
-    // ignores it), so the same loads serve every iteration
-    const T *__restrict__ vPrev = first ? r : vOld;
     double acc = 0.0;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        T ri = r[i], vi = vPrev[i];
+    for (size_t i = i0; i < n; i += stride) {
+        if (i != i0) {
+            slots(0, i);
+            ri = r[i];
+            vi = vPrev[i];
+            gather();
+        }
         T zi = (T)0;
-        // the row's slots kPcChunk at a time: their column indices and values
-        // first, then the gathered entries, all in flight together, then the
-        // multiply-adds in slot order (a loop that loads a slot's column and
-        // then its entry waits twice per slot); slots past the width repeat
-        // the last one and are not added
-        for (int k0 = 0; k0 < width; k0 += kPcChunk) {
-            int cc[kPcChunk];
-            T vv[kPcChunk], rc[kPcChunk], vc[kPcChunk];
-            #pragma unroll
-            for (int u = 0; u < kPcChunk; ++u) {
-                const size_t kk = (size_t)min(k0 + u, width - 1) * n + i;
-                cc[u] = col[kk];
-                vv[u] = val[kk];
-            }
-            #pragma unroll
-            for (int u = 0; u < kPcChunk; ++u) {
-                rc[u] = r[cc[u]];
-                vc[u] = vPrev[cc[u]];
-            }
-            #pragma unroll
-            for (int u = 0; u < kPcChunk; ++u) asm volatile("" : "+v"(rc[u]), "+v"(vc[u]));
+        for (int k0 = 0;;) {
             #pragma unroll
             for (int u = 0; u < kPcChunk; ++u) {
                 const T x = first ? rc[u] : __builtin_fma(beta, vc[u], rc[u]);
                 if (k0 + u < width) zi = __builtin_fma(vv[u], x, zi);
             }
+            k0 += kPcChunk;
+            if (k0 >= width) break;
+            slots(k0, i);
+            gather();
         }
-        asm volatile("" : "+v"(ri), "+v"(vi));
         const T vn = first ? ri : __builtin_fma(beta, vi, ri);
         vNew[i] = vn;
         z[i] = zi;
         acc += (double)vn * (double)zi;
     }
-    const double p = pc_block_sum(acc);
+    const double p = pc_block_sum(acc, lw[1]);
     if (threadIdx.x == 0) partials[blockIdx.x] = p;
 }
 
 // a = num / (v.z) (:723), each workgroup summing the product step's
-// partials itself; u += a v, r -= a z, |r|^2 (:724-727)
+// partials itself; u += a v, r -= a z, |r|^2 (:724-727).  Loads first, as in
+// k_pc_spmv.
 template <typename T>
 __global__ __launch_bounds__(kPcThreads) void k_pc_update(T *__restrict__ x, const T *__restrict__ v,
                                                           T *__restrict__ r, const T *__restrict__ z, size_t n,
                                                           double *partials, PcState *st,
                                                           const SolverState *outer, int it)
 {
+    const size_t i0 = (size_t)blockIdx.x * kPcThreads + threadIdx.x, ic = min(i0, n - 1);
+    double part = pc_part(partials, gridDim.x);
+    T xi = x[ic], vi = v[ic], ri = r[ic], zi = z[ic];
+    asm volatile("" : "+v"(xi), "+v"(vi), "+v"(ri), "+v"(zi), "+v"(part));
     if (pc_skip(st, outer)) return;
-    __shared__ double sS;
-    const double S0 = pc_final_sum(partials);
-    if (threadIdx.x == 0) sS = S0;
-    __syncthreads();
-    const double alpha = st->numP[it & 1] / sS;
+    __shared__ double lw[2][kPcThreads / 64];
+    const double alpha = st->numP[it & 1] / pc_block_sum(part, lw[0]);
     if (blockIdx.x == 0 && threadIdx.x == 0) st->alpha = alpha;
     const T a = (T)alpha;
     double acc = 0.0;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        x[i] = x[i] + a * v[i];
-        const T rv = r[i] - a * z[i];
+    for (size_t i = i0; i < n; i += (size_t)gridDim.x * kPcThreads) {
+        if (i != i0) {
+            xi = x[i];
+            vi = v[i];
+            ri = r[i];
+            zi = z[i];
+        }
+        x[i] = xi + a * vi;
+        const T rv = ri - a * zi;
         r[i] = rv;
         acc += (double)rv * (double)rv;
     }
-    const double p = pc_block_sum(acc);
+    const double p = pc_block_sum(acc, lw[1]);
     if (threadIdx.x == 0) partials[kPcParts + blockIdx.x] = p;
 }
 
 // the end of the last iteration issued (it = maxIters): rNorm and the
 // count; the loop ends there whatever the stop test says (:728-732)
-__global__ __launch_bounds__(kPcThreads) void k_pc_final_rnorm(const double *partials, PcState *st,
+__global__ __launch_bounds__(kPcThreads) void k_pc_final_rnorm(const double *partials, int nParts, PcState *st,
                                                                const SolverState *outer, int it)
 {
     if (pc_skip(st, outer)) return;
-    const double S = pc_final_sum(partials + kPcParts);
+    const double S = pc_final_sum(partials + kPcParts, nParts);
     if (threadIdx.x == 0) {
         const double den = st->numP[it & 1];
         st->rNorm = sqrt(S);
@@ -206,39 +250,87 @@ __global__ __launch_bounds__(kPcThreads) void k_pc_final_rnorm(const double *par
     }
 }
 
-// nIt = 0: the preconditioner returns r itself (:738-740)
+// the result; nIt = 0: the preconditioner returns r itself (:738-740)
 template <typename T>
-__global__ __launch_bounds__(kPcThreads) void k_pc_finish(T *__restrict__ x, const T *__restrict__ r, size_t n,
-                                                          const PcState *st, const SolverState *outer)
+__global__ __launch_bounds__(kPcThreads) void k_pc_finish(T *__restrict__ x, const T *__restrict__ u,
+                                                          const T *__restrict__ r, size_t n, const PcState *st,
+                                                          const SolverState *outer)
 {
     if (outer && (outer->done || outer->innerExit)) return;
-    if (st->maxIters > 0) return;
+    const T *__restrict__ q = st->maxIters > 0 ? u : r;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        x[i] = r[i];
+        x[i] = q[i];
 }
 
 template <typename T>
-int pc_apply(FemPC &pc, const T *b, T *x, T *r, T *z, T *v0, T *v1, const T *val, const SolverState *outer,
-             hipStream_t s)
+struct PcBuffers {
+    T *r, *z, *v[2], *u;
+    const T *val;
+};
+
+template <typename T>
+hipError_t pc_iterations(FemPC &pc, const PcBuffers<T> &B, const SolverState *outer, hipStream_t s)
 {
     const size_t n = pc.n;
-    const dim3 g(kPcParts), t(kPcThreads);
-    hipLaunchKernelGGL(k_pc_start<T>, g, t, 0, s, b, r, x, n, pc.partials, (const PcState *)pc.st, outer);
-    hipLaunchKernelGGL(k_pc_final_start, dim3(1), t, 0, s, (const double *)pc.partials, pc.st, outer, pc.maxIters,
-                       pc.tol);
-    T *v[2] = {v0, v1};
+    const dim3 g(pc_grid(n)), t(kPcThreads);
     for (int it = 1; it <= pc.maxIters; ++it) {
-        T *vNew = v[it & 1];
-        const T *vOld = v[(it + 1) & 1];
-        hipLaunchKernelGGL(k_pc_spmv<T>, g, t, 0, s, (const T *)r, vOld, vNew, z, (const int *)pc.col, val,
+        T *vNew = B.v[it & 1];
+        const T *vOld = B.v[(it + 1) & 1];
+        hipLaunchKernelGGL(k_pc_spmv<T>, g, t, 0, s, (const T *)B.r, vOld, vNew, B.z, (const int *)pc.col, B.val,
                            pc.width, n, pc.partials, pc.st, outer, it);
-        hipLaunchKernelGGL(k_pc_update<T>, g, t, 0, s, x, (const T *)vNew, r, (const T *)z, n, pc.partials, pc.st,
-                           outer, it);
+        hipLaunchKernelGGL(k_pc_update<T>, g, t, 0, s, B.u, (const T *)vNew, B.r, (const T *)B.z, n, pc.partials,
+                           pc.st, outer, it);
     }
     if (pc.maxIters > 0)
-        hipLaunchKernelGGL(k_pc_final_rnorm, dim3(1), t, 0, s, (const double *)pc.partials, pc.st, outer,
-                           pc.maxIters);
-    hipLaunchKernelGGL(k_pc_finish<T>, g, t, 0, s, x, (const T *)r, n, (const PcState *)pc.st, outer);
+        hipLaunchKernelGGL(k_pc_final_rnorm, dim3(1), t, 0, s, (const double *)pc.partials, (int)g.x, pc.st,
+                           outer, pc.maxIters);
+    return hipGetLastError();
+}
+
+// The two launches an iteration cost the host 6.2 us each, more than the
+// kernels take up to some 10^5 unknowns.
+// 45x33, N = 5, 60 applications of 50 iterations: 37.4 ms launched one by one,
+// 28.6 as graphs (32.2 with 512 workgroups instead of pc_grid's).
+// Where no graph can be had (memory, a stream that is being captured) the
+// launches are issued one by one.
+template <typename T>
+int pc_apply(FemPC &pc, const T *b, T *x, const PcBuffers<T> &B, const SolverState *outer, hipStream_t s)
+{
+    const size_t n = pc.n;
+    const dim3 g(pc_grid(n)), t(kPcThreads);
+    FemPC::Graph &G = pc.graph[sizeof(T) == 4][outer != nullptr];
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    SELF_HIP(hipStreamIsCapturing(s, &cap));
+    const bool useGraph = pc.maxIters > 0 && cap == hipStreamCaptureStatusNone;
+    if (useGraph && G.exec && G.outer != outer) {  // another solver's state
+        SELF_HIP(hipStreamSynchronize(s));
+        SELF_HIP(hipGraphExecDestroy(G.exec));
+        G.exec = nullptr;
+    }
+    if (useGraph && !G.exec && !G.failed) {
+        hipGraph_t gr = nullptr;
+        hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
+        if (e == hipSuccess) {
+            const hipError_t l = pc_iterations<T>(pc, B, outer, s);
+            e = hipStreamEndCapture(s, &gr);
+            if (e == hipSuccess) e = l;
+        }
+        if (e == hipSuccess) e = hipGraphInstantiate(&G.exec, gr, nullptr, nullptr, 0);
+        if (gr) (void)hipGraphDestroy(gr);
+        G.outer = outer;
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            G.exec = nullptr;
+            G.failed = true;
+        }
+    }
+    hipLaunchKernelGGL(k_pc_start<T>, g, t, 0, s, b, B.r, B.u, n, pc.partials, (const PcState *)pc.st, outer);
+    hipLaunchKernelGGL(k_pc_final_start, dim3(1), t, 0, s, (const double *)pc.partials, (int)g.x, pc.st, outer,
+                       pc.maxIters, pc.tol);
+    SELF_HIP(hipGetLastError());
+    if (useGraph && G.exec) SELF_HIP(hipGraphLaunch(G.exec, s));
+    else SELF_HIP(pc_iterations<T>(pc, B, outer, s));
+    hipLaunchKernelGGL(k_pc_finish<T>, g, t, 0, s, x, (const T *)B.u, (const T *)B.r, n, (const PcState *)pc.st, outer);
     SELF_HIP(hipGetLastError());
     return SELF_OK;
 }
@@ -247,7 +339,10 @@ int pc_apply(FemPC &pc, const T *b, T *x, T *r, T *z, T *v0, T *v1, const T *val
 
 FemPC::~FemPC()
 {
-    void *p[] = {col, val, val32, r, z, v[0], v[1], r32, z32, v32[0], v32[1], partials, st};
+    for (auto &a : graph)
+        for (Graph &g : a)
+            if (g.exec) (void)hipGraphExecDestroy(g.exec);
+    void *p[] = {col, val, val32, r, z, v[0], v[1], u, r32, z32, v32[0], v32[1], u32, partials, st};
     for (void *q : p)
         if (q) (void)hipFree(q);
 }
@@ -348,7 +443,7 @@ int FemPC::build(int N, size_t nE, const double *x, const double *y, const doubl
     const size_t ne = (size_t)width * nG;
     if ((rc = dev(&col, ne)) || (rc = dev(&val, ne)) || (rc = dev(&val32, ne)) || (rc = dev(&r, nG)) ||
         (rc = dev(&z, nG)) || (rc = dev(&v[0], nG)) || (rc = dev(&v[1], nG)) || (rc = dev(&r32, nG)) ||
-        (rc = dev(&z32, nG)) || (rc = dev(&v32[0], nG)) || (rc = dev(&v32[1], nG)) ||
+        (rc = dev(&z32, nG)) || (rc = dev(&v32[0], nG)) || (rc = dev(&v32[1], nG)) || (rc = dev(&u, nG)) || (rc = dev(&u32, nG)) ||
         (rc = dev(&partials, 2 * kPcParts)) || (rc = dev(&st, 1)))
         return rc;
     SELF_HIP(hipMemcpy(col, ellc.data(), sizeof(int) * ne, hipMemcpyHostToDevice));
@@ -360,12 +455,12 @@ int FemPC::build(int N, size_t nE, const double *x, const double *y, const doubl
 
 int FemPC::apply(const double *b, double *x, const SolverState *outer, hipStream_t s)
 {
-    return pc_apply<double>(*this, b, x, r, z, v[0], v[1], val, outer, s);
+    return pc_apply<double>(*this, b, x, {r, z, {v[0], v[1]}, u, val}, outer, s);
 }
 
 int FemPC::apply32(const float *b, float *x, const SolverState *outer, hipStream_t s)
 {
-    return pc_apply<float>(*this, b, x, r32, z32, v32[0], v32[1], val32, outer, s);
+    return pc_apply<float>(*this, b, x, {r32, z32, {v32[0], v32[1]}, u32, val32}, outer, s);
 }
 
 int FemPC::last_iterations(hipStream_t s, int &its)

@@ -17,7 +17,9 @@
 // launch's partials itself, in one fixed order, so all hold the same bits);
 // every kernel returns at once when the inner CG has converged or the outer
 // solver is done, so the host issues pcIterates iterations without reading
-// anything back.
+// anything back: as one graph launch, recorded by the first application over
+// the solver's own buffers (the right-hand side comes in by the start kernel,
+// the result leaves by the finish kernel).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -46,8 +48,15 @@ struct FemPC {
     int *col = nullptr;
     double *val = nullptr;
     float *val32 = nullptr;
-    double *r = nullptr, *z = nullptr, *v[2] = {nullptr, nullptr};
-    float *r32 = nullptr, *z32 = nullptr, *v32[2] = {nullptr, nullptr};
+    double *r = nullptr, *z = nullptr, *v[2] = {nullptr, nullptr}, *u = nullptr;
+    float *r32 = nullptr, *z32 = nullptr, *v32[2] = {nullptr, nullptr}, *u32 = nullptr;
+    // the iterations as a graph over the buffers above, by arithmetic (FP64,
+    // FP32) and by whether an outer solver's state can end them
+    struct Graph {
+        hipGraphExec_t exec = nullptr;
+        const SolverState *outer = nullptr;
+        bool failed = false;
+    } graph[2][2];
     double *partials = nullptr;  // [2][kPcParts]: product step (v.z), update (r.r)
     PcState *st = nullptr;
     size_t bytes = 0;
