@@ -287,6 +287,46 @@ hipError_t pc_iterations(FemPC &pc, const PcBuffers<T> &B, const SolverState *ou
     return hipGetLastError();
 }
 
+// The same launches as a graph, a chain of kernel nodes (built node by node: a
+// stream capture can fail beside another thread's allocations).
+template <typename T>
+hipError_t pc_graph(FemPC &pc, const PcBuffers<T> &B, const SolverState *outer, hipGraphExec_t *exec)
+{
+    hipGraph_t gr = nullptr;
+    hipError_t e = hipGraphCreate(&gr, 0);
+    hipGraphNode_t last = nullptr;
+    const auto node = [&](void *f, unsigned blocks, void **params) {
+        if (e != hipSuccess) return;
+        hipKernelNodeParams k{};
+        k.func = f;
+        k.gridDim = dim3(blocks);
+        k.blockDim = dim3(kPcThreads);
+        k.kernelParams = params;
+        hipGraphNode_t nd = nullptr;
+        e = hipGraphAddKernelNode(&nd, gr, last ? &last : nullptr, last ? 1 : 0, &k);
+        last = nd;
+    };
+    unsigned g = pc_grid(pc.n);
+    int nParts = (int)g;
+    const T *r = B.r, *z = B.z, *val = B.val;
+    const double *parts = pc.partials;
+    const int *col = pc.col;
+    T *rw = B.r, *zw = B.z, *u = B.u;
+    for (int it = 1; it <= pc.maxIters; ++it) {
+        T *vNew = B.v[it & 1];
+        const T *vOld = B.v[(it + 1) & 1], *v = vNew;
+        void *a[] = {&r, &vOld, &vNew, &zw, &col, &val, &pc.width, &pc.n, &pc.partials, &pc.st, &outer, &it};
+        node(reinterpret_cast<void *>(&k_pc_spmv<T>), g, a);
+        void *b[] = {&u, &v, &rw, &z, &pc.n, &pc.partials, &pc.st, &outer, &it};
+        node(reinterpret_cast<void *>(&k_pc_update<T>), g, b);
+    }
+    void *c[] = {&parts, &nParts, &pc.st, &outer, &pc.maxIters};
+    node(reinterpret_cast<void *>(&k_pc_final_rnorm), 1, c);
+    if (e == hipSuccess) e = hipGraphInstantiate(exec, gr, nullptr, nullptr, 0);
+    if (gr) (void)hipGraphDestroy(gr);
+    return e;
+}
+
 // The two launches an iteration cost the host 6.2 us each, more than the
 // kernels take up to some 10^5 unknowns.
 // 45x33, N = 5, 60 applications of 50 iterations: 37.4 ms launched one by one,
@@ -308,15 +348,7 @@ int pc_apply(FemPC &pc, const T *b, T *x, const PcBuffers<T> &B, const SolverSta
         G.exec = nullptr;
     }
     if (useGraph && !G.exec && !G.failed) {
-        hipGraph_t gr = nullptr;
-        hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
-        if (e == hipSuccess) {
-            const hipError_t l = pc_iterations<T>(pc, B, outer, s);
-            e = hipStreamEndCapture(s, &gr);
-            if (e == hipSuccess) e = l;
-        }
-        if (e == hipSuccess) e = hipGraphInstantiate(&G.exec, gr, nullptr, nullptr, 0);
-        if (gr) (void)hipGraphDestroy(gr);
+        const hipError_t e = pc_graph<T>(pc, B, outer, &G.exec);
         G.outer = outer;
         if (e != hipSuccess) {
             (void)hipGetLastError();
