@@ -291,7 +291,8 @@ int self_sw2d_synchronize(self_sw2d_t h);
  * waves), 2 (each workgroup prefetches its second group while computing the
  * first), 0 = default (1).  No reference counterpart. */
 int self_sw2d_set_groups(self_sw2d_t h, int groups);
-/* Fused form: run pairs of RK3 steps as one captured HIP graph (six stage
+/* Fused form: two or more RK3 steps of a model that fits the device run in one
+ * launch; of others, pairs of steps run as one captured HIP graph (six stage
  * launches), re-captured whenever a launch it holds would change (default
  * on); 0 launches every stage from the host.  No reference counterpart. */
 int self_sw2d_set_graph(self_sw2d_t h, int enable);
