@@ -552,6 +552,11 @@ __global__ __launch_bounds__(256) void k_adv_steps(AdvArgs A, AdvStepsArgs T)
                 // every lane is past its contractions: the flux arrays take the gradient and the volume flux
                 sx[lo + f * np + nd] = gx[f];
                 sy[lo + f * np + nd] = gy[f];
+                // the model's gradient is the last stage's, as the launched stages leave it
+                if (st + 1 == T.nStages) {
+                    A.grad[f * mstride + base] = gx[f];
+                    A.grad[(NQ + f) * mstride + base] = gy[f];
+                }
             }
         }
         sync();

@@ -65,3 +65,25 @@ def test_resident_steps_equal_launches(gpu_lib, case, monkeypatch):
     assert np.array_equal(a.GetTendency(), b.GetTendency())
     a.Trash()
     b.Trash()
+
+
+@pytest.mark.parametrize("case", [CASES[0], CASES[2], CASES[8], CASES[10], CASES[11]],
+                         ids=lambda c: "-".join(str(v) for v in c.values()))
+def test_gradient_after_steps(gpu_lib, case, monkeypatch):
+    """GetGradient after ForwardStepRK3 is the last stage's, as the launched
+    stages leave it: not that of an earlier time derivative."""
+    a, b = _model(**case), _model(**case)
+    monkeypatch.setenv("SELF_AMD_SPIN_LIMIT", "0")
+    for n in (1, 4):
+        b.ForwardStepRK3(0.1, n)
+        b.Synchronize()
+    want = b.GetGradient()
+    monkeypatch.delenv("SELF_AMD_SPIN_LIMIT")
+    a.GlobalTimeDerivative(0.1)
+    before = a.GetGradient()
+    for n in (1, 4):
+        a.ForwardStepRK3(0.1, n)
+    for g, w, o in zip(a.GetGradient(), want, before):
+        assert np.isfinite(w).all() and np.array_equal(g, w) and not np.array_equal(g, o)
+    a.Trash()
+    b.Trash()
