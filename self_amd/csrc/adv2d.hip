@@ -398,7 +398,8 @@ struct AdvStepsArgs {
     PersistArgs P;
     int nStages;
     unsigned tag0;          // tag of the first stage
-    double tn, dt;
+    int first;              // steps of the call before this launch's
+    double tn, dt;          // tn: start of the call
     double a[3], b[3], gc[3];
     double *cOut;
     ll_quad *llC, *llG;     // [nE][NQ][4 n1], [nE][2 NQ][4 n1]
@@ -481,8 +482,8 @@ __global__ __launch_bounds__(256) void k_adv_steps(AdvArgs A, AdvStepsArgs T)
     sync();
     send_c(T.tag0);
     int rk = 0;
-    double tStep = T.tn;
-    for (int st = 0, step = 0; st < T.nStages; ++st) {
+    double tStep = T.tn + (double)T.first * T.dt;
+    for (int st = 0, step = T.first; st < T.nStages; ++st) {
         #pragma clang fp contract(off)
         const unsigned tag = T.tag0 + st;
         const double time = tStep + (rk == 0 ? T.b[0] : rk == 1 ? T.b[1] : T.b[2]) * T.dt;
@@ -664,8 +665,6 @@ struct self_adv2d_s {
     bool trValid = false, ready = false, hasRelax = false;
     // several steps in one launch (k_adv_steps): second state, messages, launches in flight
     double *cAlt = nullptr;
-    ll_quad *ll = nullptr;
-    unsigned tag = 0;
     ResidentRuns runs;
 };
 
@@ -779,20 +778,19 @@ int resident_prepare(self_adv2d_s *h)
     ADV_DISPATCH(h->N, h->nq, fits = (resident_blocks<NN, QQ>(h, perCu, blocks)));
     h->runs.off = !fits;
     if (!fits) return SELF_OK;
+    h->runs.messageBytes = 3 * sizeof(ll_quad) * ll_quads(h);
     if (hipMalloc(reinterpret_cast<void **>(&h->cAlt), sizeof(double) * h->nq * h->nE * h->np) != hipSuccess ||
-        hipMalloc(reinterpret_cast<void **>(&h->ll), 3 * sizeof(ll_quad) * ll_quads(h)) != hipSuccess ||
+        hipMalloc(reinterpret_cast<void **>(&h->runs.messages), h->runs.messageBytes) != hipSuccess ||
         hipMalloc(reinterpret_cast<void **>(&h->runs.status), sizeof(int)) != hipSuccess) {
         (void)hipGetLastError();
         h->runs.off = true;
         return SELF_OK;
     }
-    SELF_HIP(hipMemsetAsync(h->ll, 0, 3 * sizeof(ll_quad) * ll_quads(h), h->stream));  // tags start at 1
-    SELF_HIP(hipMemsetAsync(h->runs.status, 0, sizeof(int), h->stream));
-    return SELF_OK;
+    return h->runs.clear(h->stream);
 }
 
 template <int N, int NQ>
-int launch_steps(self_adv2d_s *h, double tn, int nSteps)
+int launch_steps(self_adv2d_s *h, double tn, int first, int nSteps)
 {
     int perCu = 0;
     size_t blocks = 0;
@@ -801,7 +799,8 @@ int launch_steps(self_adv2d_s *h, double tn, int nSteps)
     AdvStepsArgs T{};
     T.P = h->runs.args();
     T.nStages = 3 * nSteps;
-    T.tag0 = h->tag + 1;
+    T.tag0 = h->runs.tag + 1;
+    T.first = first;
     T.tn = tn;
     T.dt = h->dt;
     for (int m = 0; m < 3; ++m) {
@@ -810,31 +809,29 @@ int launch_steps(self_adv2d_s *h, double tn, int nSteps)
         T.gc[m] = kRkG[m];
     }
     T.cOut = h->cAlt;
-    T.llC = h->ll;
-    T.llG = h->ll + ll_quads(h);
+    T.llC = h->runs.messages;
+    T.llG = h->runs.messages + ll_quads(h);
     T.bytesC = (unsigned)(sizeof(ll_quad) * ll_quads(h));
-    {
-        PersistGate gate(h->device, h->stream, (int)blocks, perCu);
-        if (gate.rc) return gate.rc;
-        hipLaunchKernelGGL((k_adv_steps<N, NQ>), dim3((unsigned)blocks), dim3(256), 0, h->stream, A, T);
-        SELF_HIP(hipGetLastError());
-        if (int rc = gate.launched()) return rc;
-    }
-    h->tag += 3u * (unsigned)nSteps;
-    h->runs.launched(nSteps, tn, h->c);
+    h->runs.pending.reserve(h->runs.pending.size() + 1);  // nothing fails between the launch and its record
+    PersistGate gate(h->device, h->stream, (int)blocks, perCu);
+    if (gate.rc) return gate.rc;
+    hipLaunchKernelGGL((k_adv_steps<N, NQ>), dim3((unsigned)blocks), dim3(256), 0, h->stream, A, T);
+    SELF_HIP(hipGetLastError());
+    h->runs.launched(first, nSteps, tn, h->c);
     std::swap(h->c, h->cAlt);
     h->trValid = false;
-    return SELF_OK;
+    return gate.launched();
 }
 
-int launched_steps(self_adv2d_s *h, double tn, int nSteps)
+// steps first .. nSteps - 1 of a call that begins at tn
+int launched_steps(self_adv2d_s *h, double tn, int first, int nSteps)
 {
     int rc = SELF_OK;
     if (!h->trValid) {
         if ((rc = launch_c_traces(h, h->tr[h->cur]))) return rc;
         h->trValid = true;
     }
-    for (int s = 0; s < nSteps && !rc; ++s) {
+    for (int s = first; s < nSteps && !rc; ++s) {
         const double t0 = tn + s * h->dt;
         for (int m = 0; m < 3 && !rc; ++m) rc = stage(h, t0 + kRkB[m] * h->dt, m, 0);
     }
@@ -852,7 +849,7 @@ int settle(self_adv2d_s *h)
     if (h->c != again[0].in) std::swap(h->c, h->cAlt);
     h->trValid = false;
     for (const auto &r : again)
-        if (int rc = launched_steps(h, r.t0, r.steps)) return rc;
+        if (int rc = launched_steps(h, r.t0, r.first, r.first + r.steps)) return rc;
     SELF_HIP(hipStreamSynchronize(h->stream));
     return SELF_OK;
 }
@@ -893,7 +890,7 @@ try {
     const size_t nE = h->nE, np = h->np, n1 = h->n1, nq = h->nq;
     auto fail = [&](hipError_t e) {
         void *p[] = {h->nodal, h->c, h->G, h->tend, h->grad, h->vel, h->velTr, h->fvel, h->metric, h->fnrm,
-                     h->tr[0], h->tr[1], h->trG, h->relax, h->rFac, h->side, h->pnode, h->cAlt, h->ll, h->runs.status};
+                     h->tr[0], h->tr[1], h->trG, h->relax, h->rFac, h->side, h->pnode, h->cAlt, h->runs.messages, h->runs.status};
         for (void *q : p)
             if (q) (void)hipFree(q);
         if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -954,7 +951,7 @@ int self_adv2d_destroy(self_adv2d_t h)
     (void)hipSetDevice(h->device);
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     void *p[] = {h->nodal, h->c, h->G, h->tend, h->grad, h->vel, h->velTr, h->fvel, h->metric, h->fnrm,
-                 h->tr[0], h->tr[1], h->trG, h->relax, h->rFac, h->side, h->pnode, h->cAlt, h->ll, h->runs.status};
+                 h->tr[0], h->tr[1], h->trG, h->relax, h->rFac, h->side, h->pnode, h->cAlt, h->runs.messages, h->runs.status};
     for (void *q : p)
         if (q) (void)hipFree(q);
     if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -1048,7 +1045,7 @@ try {
     SELF_HIP(hipSetDevice(h->device));
     int rc = SELF_OK;
     const bool resident = !h->runs.off && nSteps >= 1;
-    if (!resident || elapsed_ms || h->runs.pending.size() >= 64)
+    if (!resident || elapsed_ms)
         if ((rc = settle(h))) return rc;
     if (!resident && !h->trValid) {
         if ((rc = launch_c_traces(h, h->tr[h->cur]))) return rc;
@@ -1060,10 +1057,17 @@ try {
         SELF_HIP(hipEventCreate(&e1));
         SELF_HIP(hipEventRecord(e0, h->stream));
     }
-    if (resident && !h->runs.off) {
-        ADV_DISPATCH(h->N, h->nq, rc = (launch_steps<NN, QQ>(h, tn, nSteps)));
-    } else {
-        rc = launched_steps(h, tn, nSteps);
+    int s = 0;
+    while (resident && s < nSteps && !rc) {
+        if (h->runs.pending.size() >= 64) rc = settle(h);
+        if (rc || h->runs.off) break;
+        const int n = std::min(nSteps - s, kPersistMaxSteps);
+        ADV_DISPATCH(h->N, h->nq, rc = (launch_steps<NN, QQ>(h, tn, s, n)));
+        s += n;
+    }
+    if (!rc && s < nSteps) {
+        rc = settle(h);
+        if (!rc) rc = launched_steps(h, tn, s, nSteps);
     }
     if (elapsed_ms) {
         SELF_HIP(hipEventRecord(e1, h->stream));

@@ -438,8 +438,8 @@ struct CgsemOp final : DevOp {
     char *resBuf = nullptr;
     size_t resBytes = 0;
     int resLaunches = 0, resGaveUp = 0;
-    unsigned resTag = 0;
-    bool resident = true;
+    unsigned resTag = 0;            // of the last iteration settled
+    bool resDirty = false;          // messages of a launch not settled, or never cleared
     std::vector<double> kH;         // flux coefficient last set (host, local layout; empty = ONE)
     std::unique_ptr<FemPC> pc;      // CGsemPreconditioner_2D (self_cgsem2d_set_preconditioner)
 
@@ -553,8 +553,13 @@ struct CgsemOp final : DevOp {
                 resGaveUp = 4;
                 return SELF_OK;
             }
-            SELF_HIP(hipMemsetAsync(resBuf, 0, resBytes, s));  // tags start at 1
+            resDirty = true;
         }
+        if (resDirty) {  // tags start at 1
+            SELF_HIP(hipMemsetAsync(resBuf, 0, resBytes, s));
+            resTag = 0;
+        }
+        resDirty = true;
         CgResArgs A{};
         A.gid = gid;
         A.cs = cs;
@@ -590,7 +595,7 @@ struct CgsemOp final : DevOp {
     int resident_cg(KrylovWork &wk, bool precond, bool &taken, hipStream_t s) override
     {
         taken = false;
-        if (!resident || resGaveUp >= 4 || maxCopies > 4 || res_exch() >= (1u << 31)) return SELF_OK;
+        if (resGaveUp >= 4 || maxCopies > 4 || res_exch() >= (1u << 31)) return SELF_OK;
         int rc = SELF_OK;
         // As few nodes a thread as the device has workgroups for; one a thread
         // only on up to 7/8 of the CUs (64x64, N = 7: 7.8 us an iteration on 256
@@ -608,9 +613,10 @@ struct CgsemOp final : DevOp {
         gaveUp = h.done == kCgGaveUp;
         if (gaveUp) {  // beside much other work on the device it will happen again
             ++resGaveUp;
-            resTag = 0;
-            SELF_HIP(hipMemsetAsync(resBuf, 0, resBytes, s));
-        } else if (h.done != 3) {  // 3: nothing to solve, the launch returned at once
+            return SELF_OK;
+        }
+        resDirty = false;
+        if (h.done != 3) {  // 3: nothing to solve, the launch returned at once
             std::swap(wk.u, wk.z);
             resTag += (unsigned)h.iter;
         }

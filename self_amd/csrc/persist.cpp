@@ -71,6 +71,14 @@ unsigned persist_spin_limit()
     return 2000;
 }
 
+int ResidentRuns::clear(hipStream_t s)
+{
+    SELF_HIP(hipMemsetAsync(messages, 0, messageBytes, s));
+    SELF_HIP(hipMemsetAsync(status, 0, sizeof(int), s));
+    tag = 0;
+    return SELF_OK;
+}
+
 int ResidentRuns::settle(hipStream_t s, std::vector<Run> &again)
 {
     again.clear();
@@ -82,7 +90,7 @@ int ResidentRuns::settle(hipStream_t s, std::vector<Run> &again)
     done.swap(pending);
     if (bad == 0) return SELF_OK;
     if (++gaveUp >= 4) off = true;
-    SELF_HIP(hipMemsetAsync(status, 0, sizeof(int), s));
+    if (int rc = clear(s)) return rc;
     size_t first = 0;
     while (first < done.size() && done[first].launch != bad) ++first;
     SELF_REQUIRE(first < done.size(), SELF_ERR_HIP, "a resident launch gave up and cannot be found (%d)", bad);

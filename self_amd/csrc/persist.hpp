@@ -148,23 +148,42 @@ int persist_blocks_per_cu(const void *kernel, int threads);
 int persist_cus(int device);
 unsigned persist_spin_limit();
 
-// Launches of resident time steps that are not yet known to have finished.  One
-// that gave up left its input as it was and made the later ones return at
-// once: settle() waits for them and lists the runs to do over by ordinary
-// launches.  After several such launches `off` is set: beside much other work
-// on the device it happens again.
+// Steps of one launch at most: the launches between two settlings stay
+// countable, and 3 x steps in an int.
+constexpr int kPersistMaxSteps = 1 << 16;
+
+// Launches of resident time steps that are not yet known to have finished, and
+// the messages they exchange.  A launch that gave up left its input as it was
+// and made the later ones return at once: settle() waits for them and lists the
+// runs to do over by ordinary launches.  After several such launches `off` is
+// set: beside much other work on the device it happens again.
+// The tags of stages count on over the launches.  That a word holds the wanted
+// tag or an older one of the last two is true only while every launch writes all
+// its messages; after one that gave up, words of any earlier stage are left, and
+// 16 bits of tag come round again after 65 536 stages (kPersistMaxSteps steps
+// are a multiple of it).  So settle() clears the messages then and the tags
+// begin again.
 struct ResidentRuns {
     struct Run {
-        int launch, steps;
+        int launch, first, steps;  // first: steps of the call before this run
         double t0;
         double *in;  // the state the run began with
     };
     int *status = nullptr;
+    ll_quad *messages = nullptr;
+    size_t messageBytes = 0;
+    unsigned tag = 0;              // of the last stage launched; the cleared messages' is 0
     int launches = 0, gaveUp = 0;
     bool off = false;
     std::vector<Run> pending;
     PersistArgs args() const { return {status, launches + 1, persist_spin_limit()}; }
-    void launched(int steps, double t0, double *in) { pending.push_back({++launches, steps, t0, in}); }
+    // call it as soon as the launch is queued: its messages will have been written
+    void launched(int first, int steps, double t0, double *in)
+    {
+        tag += 3u * (unsigned)steps;
+        pending.push_back({++launches, first, steps, t0, in});
+    }
+    int clear(hipStream_t s);      // messages and status, before the first launch
     int settle(hipStream_t s, std::vector<Run> &again);
 };
 

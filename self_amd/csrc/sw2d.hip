@@ -1265,9 +1265,6 @@ struct self_sw2d_s {
     // several steps in one launch (k_sw_steps): second state buffer, messages,
     // launches in flight (off also where the buffers could not be had)
     double *qAlt = nullptr;
-    ll_quad *ll = nullptr;
-    unsigned tag = 0;
-    bool llClear = false;
     ResidentRuns runs;
 };
 
@@ -1291,7 +1288,7 @@ void free_all(self_sw2d_s *h)
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (h->qAlt) (void)hipFree(h->qAlt);
-    if (h->ll) (void)hipFree(h->ll);
+    if (h->runs.messages) (void)hipFree(h->runs.messages);
     if (h->runs.status) (void)hipFree(h->runs.status);
 }
 
@@ -1536,10 +1533,9 @@ size_t ll_quads(const self_sw2d_s *h) { return (size_t)h->members * h->nE * 8 * 
 void persist_free(self_sw2d_s *h)
 {
     if (h->qAlt) { (void)hipFree(h->qAlt); h->bytes -= sizeof(double) * 3 * h->members * h->nE * h->np; }
-    if (h->ll) { (void)hipFree(h->ll); h->bytes -= 2 * sizeof(ll_quad) * ll_quads(h); }
+    if (h->runs.messages) { (void)hipFree(h->runs.messages); h->bytes -= h->runs.messageBytes; }
     h->qAlt = nullptr;
-    h->ll = nullptr;
-    h->llClear = false;
+    h->runs.messages = nullptr;
 }
 
 // Buffers of the resident form, had once: at creation (a single state, the
@@ -1554,21 +1550,22 @@ int steps_ready(self_sw2d_s *h, bool &ok, int &perCu, size_t &blocks)
     blocks = (size_t)grid_fused<N>(h->nE, 1) * h->members;
     if (perCu < 1 || sizeof(ll_quad) * ll_quads(h) >= (1u << 31) || blocks > (size_t)perCu * persist_cus(h->device))
         return SELF_OK;
+    ok = true;
+    if (h->runs.messages) return SELF_OK;  // the buffers come and go together
     const size_t nq = 3 * (size_t)h->members * h->nE * h->np;
-    if ((!h->qAlt && dalloc(h, &h->qAlt, nq) != SELF_OK) || (!h->ll && dalloc(h, &h->ll, 2 * ll_quads(h)) != SELF_OK) ||
+    h->runs.messageBytes = 2 * sizeof(ll_quad) * ll_quads(h);
+    if (dalloc(h, &h->qAlt, nq) != SELF_OK || dalloc(h, &h->runs.messages, 2 * ll_quads(h)) != SELF_OK ||
         (!h->runs.status && dalloc(h, &h->runs.status, 1) != SELF_OK)) {
         (void)hipGetLastError();  // no memory for it: the ordinary launches need none
         persist_free(h);
         h->runs.off = true;
+        ok = false;
         return SELF_OK;
     }
-    if (!h->llClear) {  // tags start at 1
-        SELF_HIP(hipMemsetAsync(h->ll, 0, 2 * sizeof(ll_quad) * ll_quads(h), h->stream));
-        SELF_HIP(hipMemsetAsync(h->runs.status, 0, sizeof(int), h->stream));
-        h->llClear = true;
-        h->tag = 0;
+    if (int rc = h->runs.clear(h->stream)) {
+        persist_free(h);
+        return rc;
     }
-    ok = true;
     return SELF_OK;
 }
 
@@ -1585,24 +1582,21 @@ int launch_steps(self_sw2d_s *h, int nSteps, bool &taken)
     SWStepsArgs T{};
     T.P = h->runs.args();
     T.nStages = 3 * nSteps;
-    T.tag0 = h->tag + 1;
+    T.tag0 = h->runs.tag + 1;
     for (int m = 0; m < 3; ++m) { T.a[m] = kRkA[m]; T.gc[m] = kRkG[m]; }
     T.dt = h->d.dt;
     T.qOut = h->qAlt;
-    T.ll = h->ll;
-    T.llBytes = (unsigned)(sizeof(ll_quad) * ll_quads(h));
-    {
-        PersistGate gate(h->device, h->stream, (int)blocks, perCu);
-        if (gate.rc) return gate.rc;
-        hipLaunchKernelGGL((k_sw_steps<N, MIXED>), dim3((unsigned)blocks), dim3(256), 0, h->stream, A, T);
-        SELF_HIP(hipGetLastError());
-        if (int rc = gate.launched()) return rc;
-    }
-    h->tag += 3u * (unsigned)nSteps;
-    h->runs.launched(nSteps, 0.0, h->q);
+    T.ll = h->runs.messages;
+    T.llBytes = (unsigned)(h->runs.messageBytes / 2);
+    h->runs.pending.reserve(h->runs.pending.size() + 1);  // nothing fails between the launch and its record
+    PersistGate gate(h->device, h->stream, (int)blocks, perCu);
+    if (gate.rc) return gate.rc;
+    hipLaunchKernelGGL((k_sw_steps<N, MIXED>), dim3((unsigned)blocks), dim3(256), 0, h->stream, A, T);
+    SELF_HIP(hipGetLastError());
+    h->runs.launched(0, nSteps, 0.0, h->q);
     std::swap(h->q, h->qAlt);
     h->trValid = false;
-    return SELF_OK;
+    return gate.launched();
 }
 
 int steps_prepare(self_sw2d_s *h)
@@ -2128,13 +2122,11 @@ int self_sw2d_forward_step_rk3(self_sw2d_t h, double tn, int nSteps)
     int s = 0;
     if (h->d.form == SELF_FUSED && h->useGraph && !h->runs.off && nSteps >= 2 &&
         fused_groups(h->groups, h->nE, 0) == 1) {
-        // at most kMaxSteps a launch; launches in flight stay countable
-        constexpr int kMaxSteps = 1 << 16;
         bool taken = true;
         while (s < nSteps && taken) {
             if (h->runs.pending.size() >= 64 && (rc = settle(h))) return rc;
             if (h->runs.off) break;
-            const int n = std::min(nSteps - s, kMaxSteps);
+            const int n = std::min(nSteps - s, kPersistMaxSteps);
             if ((rc = steps_persistent(h, n, taken))) return rc;
             if (taken) s += n;
         }

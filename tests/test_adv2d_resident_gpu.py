@@ -9,9 +9,9 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-def _model(N, nX, nY, nq, periodic=True, warp=0.0, relax=False, inflow=False):
+def _model(N, nX, nY, nq, periodic=True, warp=0.0, relax=False, inflow=False, dt=2e-5):
     from self_amd.advection import Advection, AdvectionParams
-    p = AdvectionParams(polyDeg=N, nXElem=nX, nYElem=nY, nTracers=nq, dt=2e-5, kappa=2e-3, warp=warp,
+    p = AdvectionParams(polyDeg=N, nXElem=nX, nYElem=nY, nTracers=nq, dt=dt, kappa=2e-3, warp=warp,
                         periodicX=periodic, periodicY=periodic)
     edges = None
     if inflow:
@@ -85,5 +85,25 @@ def test_gradient_after_steps(gpu_lib, case, monkeypatch):
         a.ForwardStepRK3(0.1, n)
     for g, w, o in zip(a.GetGradient(), want, before):
         assert np.isfinite(w).all() and np.array_equal(g, w) and not np.array_equal(g, o)
+    a.Trash()
+    b.Trash()
+
+
+def test_tags_come_round_after_a_launch_gave_up(gpu_lib, monkeypatch):
+    """65536 steps are a multiple of the 65536 stages after which a message's
+    tag is the same again: the first messages of a launch that gave up must not
+    be taken for those of the launch after it.  More steps than one launch takes
+    too, with an inflow that depends on the time."""
+    case = dict(N=2, nX=9, nY=11, nq=1, periodic=False, inflow=True, dt=1e-8)
+    a, b = _model(**case), _model(**case)
+    b.ForwardStepRK3(0.2, 65536 + 3)
+    b.ForwardStepRK3(0.3, 2)
+    monkeypatch.setenv("SELF_AMD_SPIN_LIMIT", "0")
+    a.ForwardStepRK3(0.2, 65536 + 3)
+    a.Synchronize()
+    monkeypatch.delenv("SELF_AMD_SPIN_LIMIT")
+    a.ForwardStepRK3(0.3, 2)
+    want = b.GetSolution()
+    assert np.isfinite(want).all() and np.array_equal(a.GetSolution(), want)
     a.Trash()
     b.Trash()

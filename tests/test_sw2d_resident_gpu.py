@@ -120,3 +120,24 @@ def test_models_in_flight_together_equal_alone(gpu_lib):
             w.ForwardStepRK3(0.0, 4)
         assert np.array_equal(g, w.GetSolution())
         w.Trash()
+
+
+def test_tags_come_round_after_a_launch_gave_up(gpu_lib, monkeypatch):
+    """65536 steps are a multiple of the 65536 stages after which a message's
+    tag is the same again: the first messages of a launch that gave up must not
+    be taken for those of the launch after it."""
+    case = dict(N=3, nX=5, nY=7, precision="fp64", warp=0.03)
+    a, b = _model(**case), _model(**case)
+    for m in (a, b):
+        gpu_lib.check(gpu_lib.lib().self_sw2d_set_params(m._h, 1.0, 1e-7, 0.0))
+    b.ForwardStepRK3(0.0, 65536)
+    b.ForwardStepRK3(0.0, 2)
+    monkeypatch.setenv("SELF_AMD_SPIN_LIMIT", "0")
+    a.ForwardStepRK3(0.0, 65536)
+    a.Synchronize()
+    monkeypatch.delenv("SELF_AMD_SPIN_LIMIT")
+    a.ForwardStepRK3(0.0, 2)
+    want = b.GetSolution()
+    assert np.isfinite(want).all() and np.array_equal(a.GetSolution(), want)
+    a.Trash()
+    b.Trash()
