@@ -305,13 +305,14 @@ def hpe_bytes_per_element_stage(N):
     reads u, v, b, six cofactor terms and J at every node, the column
     height, and the four normal values on six faces, and writes p, w and
     the face values of b, w, p; the stage kernel reads p, w, u, v, b, the
-    background buoyancy, nine cofactor terms and J, its own and the
-    neighbour's face values, the face data (normal, |n|, background) and
-    the RK register, and writes u, v, b and the register."""
+    background buoyancy, nine cofactor terms and J, its own (N = 7 forms
+    them from the node values instead) and the neighbour's face values, the
+    face data (normal, |n|, background) and the RK register, and writes u,
+    v, b and the register."""
     n1 = N + 1
     np_, n2 = n1 ** 3, n1 * n1
     col = 12 * np_ + 43 * n2
-    stage = 25 * np_ + 72 * n2
+    stage = 25 * np_ + (54 if N == 7 else 72) * n2
     return 8 * col, 8 * stage
 
 
@@ -330,15 +331,16 @@ def bench_hpe(steps=10, warm=2, nX=32, nY=32, nL=16, N=7):
     E = m.nElems
     dof = E * (N + 1) ** 3
     bcol, bst = hpe_bytes_per_element_stage(N)
+    kcol, kst = ("k_hpe_columns_mf", "k_hpe_stage_mf") if N == 7 else (f"k_hpe_columns<{N}>", f"k_hpe_stage<{N}>")
     m.Trash()
     stage_ms = ms / steps / 3.0
     return {"workload": f"hydrostatic primitive equations {nX}x{nY} columns x {nL} layers N={N}, walled, "
                         f"buoyancy anomaly at rest, dt={info['dt']}", "steps": steps,
             "ms_per_step": ms / steps, "stage_ms": stage_ms, "dof_stage_per_s": dof * 3 * steps / (ms * 1e-3),
-            "kernel_ms": {"k_hpe_columns": col_ms, "k_hpe_stage": st_ms},
-            "algorithmic_bytes_per_stage": {"k_hpe_columns": bcol * E, "k_hpe_stage": bst * E},
-            "achieved_GBs": {"k_hpe_columns": round(bcol * E / (col_ms * 1e-3) / 1e9, 1),
-                             "k_hpe_stage": round(bst * E / (st_ms * 1e-3) / 1e9, 1),
+            "kernel_ms": {kcol: col_ms, kst: st_ms},
+            "algorithmic_bytes_per_stage": {kcol: bcol * E, kst: bst * E},
+            "achieved_GBs": {kcol: round(bcol * E / (col_ms * 1e-3) / 1e9, 1),
+                             kst: round(bst * E / (st_ms * 1e-3) / 1e9, 1),
                              "stage": round((bcol + bst) * E / (stage_ms * 1e-3) / 1e9, 1)},
             "finite": ok}
 

@@ -808,6 +808,31 @@ HpeArgs args_of(self_hpe_s *h)
     return A;
 }
 
+// The two kernels of a time derivative and update; N = 7 has its own.
+int launch_columns(self_hpe_s *h, const HpeArgs &A)
+{
+    HPE_DISPATCH_N(h->N, {
+        if constexpr (NN == 7)
+            hipLaunchKernelGGL(k_hpe_columns_mf, dim3((unsigned)h->nH), dim3(512), 0, h->stream, A);
+        else
+            hipLaunchKernelGGL((k_hpe_columns<NN>), dim3((unsigned)h->nH), dim3(HShape<NN>::threads), 0, h->stream, A);
+    });
+    SELF_HIP(hipGetLastError());
+    return SELF_OK;
+}
+
+int launch_stage(self_hpe_s *h, const HpeArgs &A)
+{
+    HPE_DISPATCH_N(h->N, {
+        if constexpr (NN == 7)
+            hipLaunchKernelGGL(k_hpe_stage_mf, dim3((unsigned)h->nE), dim3(512), 0, h->stream, A);
+        else
+            hipLaunchKernelGGL((k_hpe_stage<NN>), dim3((unsigned)h->nE), dim3(HShape<NN>::threads), 0, h->stream, A);
+    });
+    SELF_HIP(hipGetLastError());
+    return SELF_OK;
+}
+
 // one GlobalTimeDerivative followed by the update of `mode` (0 RK3 stage m,
 // 1 tendency only, 2 AB2)
 int hpe_stage(self_hpe_s *h, int mode, int m, bool keepDivU)
@@ -818,17 +843,8 @@ int hpe_stage(self_hpe_s *h, int mode, int m, bool keepDivU)
     A.a = mode == 0 ? kRkA[m] : 0.0;
     A.gdt = mode == 0 ? kRkG[m] * h->dt : 0.0;
     A.divU = keepDivU ? h->divU : nullptr;
-    HPE_DISPATCH_N(h->N, {
-        if constexpr (NN == 7) {
-            hipLaunchKernelGGL(k_hpe_columns_mf, dim3((unsigned)h->nH), dim3(512), 0, h->stream, A);
-            hipLaunchKernelGGL(k_hpe_stage_mf, dim3((unsigned)h->nE), dim3(512), 0, h->stream, A);
-        } else {
-            hipLaunchKernelGGL((k_hpe_columns<NN>), dim3((unsigned)h->nH), dim3(HShape<NN>::threads), 0, h->stream, A);
-            hipLaunchKernelGGL((k_hpe_stage<NN>), dim3((unsigned)h->nE), dim3(HShape<NN>::threads), 0, h->stream, A);
-        }
-    });
-    SELF_HIP(hipGetLastError());
-    return SELF_OK;
+    if (int rc = launch_columns(h, A)) return rc;
+    return launch_stage(h, A);
 }
 
 void free_all(self_hpe_s *h)
@@ -1152,13 +1168,10 @@ int self_hpe_kernel_times(self_hpe_t h, int nSteps, double *avg_ms)
             A.gdt = kRkG[m] * h->dt;
             A.divU = nullptr;
             SELF_HIP(hipEventRecord(ev[0], h->stream));
-            HPE_DISPATCH_N(h->N, hipLaunchKernelGGL((k_hpe_columns<NN>), dim3((unsigned)h->nH),
-                                                    dim3(HShape<NN>::threads), 0, h->stream, A));
+            if (int rc = launch_columns(h, A)) return rc;
             SELF_HIP(hipEventRecord(ev[1], h->stream));
-            HPE_DISPATCH_N(h->N, hipLaunchKernelGGL((k_hpe_stage<NN>), dim3((unsigned)h->nE),
-                                                    dim3(HShape<NN>::threads), 0, h->stream, A));
+            if (int rc = launch_stage(h, A)) return rc;
             SELF_HIP(hipEventRecord(ev[2], h->stream));
-            SELF_HIP(hipGetLastError());
             SELF_HIP(hipEventSynchronize(ev[2]));
             float a = 0, b = 0;
             SELF_HIP(hipEventElapsedTime(&a, ev[0], ev[1]));

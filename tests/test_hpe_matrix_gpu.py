@@ -47,3 +47,15 @@ def test_derivative_and_steps_match_the_oracle(gpu_lib, case):
     so, sg = orc.view(orc.sol, 5), gpu.GetSolution()
     for f in range(3):
         assert rel_l2(sg[:, f], so[:, f]) < 1e-11, f
+
+
+@pytest.mark.parametrize("N", [4, 7])
+def test_kernel_times_are_of_the_kernels_a_step_runs(gpu_lib, N):
+    """KernelTimes advances the model as that many steps do, bit for bit: it
+    times the same kernels."""
+    case = dict(N=N, n=(2, 2, 3), periodic=(False, True), warp=0.02, dp=True)
+    _, a = _pair(case, dt=2e-3)
+    _, b = _pair(case, dt=2e-3)
+    a.ForwardStepRK3(3)
+    assert min(b.KernelTimes(3)) > 0.0
+    assert np.array_equal(a.GetSolution(), b.GetSolution())
