@@ -783,6 +783,10 @@ int resident_prepare(self_adv2d_s *h)
         hipMalloc(reinterpret_cast<void **>(&h->runs.messages), h->runs.messageBytes) != hipSuccess ||
         hipMalloc(reinterpret_cast<void **>(&h->runs.status), sizeof(int)) != hipSuccess) {
         (void)hipGetLastError();
+        if (h->cAlt) (void)hipFree(h->cAlt);
+        if (h->runs.messages) (void)hipFree(h->runs.messages);
+        h->cAlt = nullptr;
+        h->runs.messages = nullptr;
         h->runs.off = true;
         return SELF_OK;
     }

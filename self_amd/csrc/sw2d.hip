@@ -2568,7 +2568,7 @@ int self_sw2d_synchronize(self_sw2d_t h)
 int self_sw2d_device_bytes(self_sw2d_t h, size_t *bytes)
 {
     SELF_REQUIRE(h && bytes, SELF_ERR_ARG, "null argument");
-    *bytes = h->bytes;
+    *bytes = h->bytes + sizeof(double) * h->stage.cap;
     return SELF_OK;
 }
 
