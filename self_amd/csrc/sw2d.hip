@@ -1538,8 +1538,9 @@ void persist_free(self_sw2d_s *h)
     h->runs.messages = nullptr;
 }
 
-// Buffers of the resident form, had once: at creation (a single state, the
-// usual case) or at the first call after the members changed.  ok: the model's
+// Buffers of the resident form, had once: with the geometry (a single state, the
+// usual case), or by the first steps after the members changed or the form was
+// switched on; a model that launches every stage from the host needs none.  ok: the model's
 // workgroups are all resident at once and the buffers are there.
 template <int N, bool MIXED>
 int steps_ready(self_sw2d_s *h, bool &ok, int &perCu, size_t &blocks)
@@ -1752,7 +1753,6 @@ try {
     if (e == hipSuccess && h->plv32) e = hipMemsetAsync(h->plv32, 0, nfield * sizeof(float), h->stream);
     if (e == hipSuccess) e = hipEventCreate(&h->ev0);
     if (e == hipSuccess) e = hipEventCreate(&h->ev1);
-    if (e == hipSuccess && (rc = steps_prepare(h))) return fail(rc);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     if (e != hipSuccess) return fail(hip_fail(e, "create", __FILE__, __LINE__));
     *out = h;
@@ -1897,7 +1897,7 @@ try {
     SELF_HIP(hipMemcpy(h->edges, edges, sizeof(int) * 6 * nEd, hipMemcpyHostToDevice));
     h->geomSet = true;
     h->trValid = false;
-    return SELF_OK;
+    return h->useGraph ? steps_prepare(h) : SELF_OK;
 }
 SELF_CATCH_ALL
 

@@ -1,6 +1,8 @@
 """Fields to the host in one piece, in several with a ragged last one, and
-without device memory for a staging buffer: the same bytes, and what the buffer
-holds is counted."""
+without device memory for a staging buffer: the same bytes.  What a model
+allocates is counted, and a request's reservation covers its model."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -49,3 +51,41 @@ def test_device_bytes_count_the_staging_buffer(gpu_lib, monkeypatch):
     monkeypatch.delenv("SELF_AMD_STAGE_DOUBLES")
     m.GetSolution()
     assert m.DeviceBytes() == before + n
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("nX,N", [(32, 7), (64, 3)])
+def test_a_request_reserves_what_its_model_holds(gpu_lib, precision, nX, N):
+    """The server's models launch their stages from the host: they allocate no
+    buffers of the resident form.  Built here with the server's calls."""
+    from self_amd import _lib as L
+    from self_amd import serving as S
+    lib, check = L.lib(), L.check
+    srv = S.Server(workers=1)
+    spec = S.make_inputs(S.Spec(S.REQ_SW2D, nX, N, 7, precision, 2))
+    res, out = srv.wait(srv.submit(spec))
+    srv.close()
+    assert res.status == 0 and np.isfinite(out).all()
+    m = sw2d_model(N=N, nX=nX, nY=nX, precision=precision)
+    h, held = C.c_void_p(), C.c_size_t()
+    d = L.SWDesc(N, m.nElems, m.mesh.nEdges, {"fp64": L.FP64, "mixed": L.MIXED}[precision], L.FUSED, 1.0, 1e-4, 0.0)
+    check(lib.self_sw2d_create(C.byref(d), C.byref(h)))
+    check(lib.self_sw2d_set_graph(h, 0))
+    g, ns = m.mesh, m.dgStorage
+    check(lib.self_sw2d_set_nodal(h, L.ptr(ns.flat("dMatS")), L.ptr(ns.flat("dMatP")), L.ptr(ns.qWeight),
+                                  L.ptr(ns.qWeight), L.ptr(ns.lagWest), L.ptr(ns.lagEast), L.ptr(ns.lagSouth),
+                                  L.ptr(ns.lagNorth)))
+    check(lib.self_sw2d_set_geometry(h, L.ptr(g.edges, L.ip), L.ptr(g.dxds), L.ptr(g.dxdp), L.ptr(g.dyds),
+                                     L.ptr(g.dydp), L.ptr(g.J), L.ptr(g.nHat), L.ptr(g.nLen)))
+    sol = np.ascontiguousarray(m.GetSolution())
+    check(lib.self_sw2d_set_field(h, 0, L.ptr(sol)))
+    check(lib.self_sw2d_forward_step_rk3(h, 0.0, 4))
+    check(lib.self_sw2d_get_field(h, 0, L.ptr(sol)))
+    check(lib.self_sw2d_device_bytes(h, C.byref(held)))
+    check(lib.self_sw2d_destroy(h))
+    nodes = g.nElems * (N + 1) ** 2
+    resident = 3 * 8 * nodes + 2 * 16 * g.nElems * 8 * (N + 1) + 4  # second state, messages, status
+    m.GetSolution()
+    assert m.DeviceBytes() == held.value + resident
+    assert held.value <= res.bytes
+    m.Trash()
