@@ -287,6 +287,10 @@ int self_sw2d_calculate_bathymetry_gradient(self_sw2d_t h);
  * (:1754-1825).  -5 for any other value. */
 int self_sw2d_set_variant(self_sw2d_t h, int variant);
 int self_sw2d_synchronize(self_sw2d_t h);
+/* Launches of several steps at once so far, and how many of them gave up
+ * waiting (beside other work on the device) and were run again by a launch per
+ * stage; waits for those in flight.  No reference counterpart. */
+int self_sw2d_resident_counts(self_sw2d_t h, int *launches, int *gaveUp);
 /* Element groups per workgroup of the fused stage kernel: 1 (one round of
  * waves), 2 (each workgroup prefetches its second group while computing the
  * first), 0 = default (1).  No reference counterpart. */
@@ -430,6 +434,8 @@ int self_adv2d_global_time_derivative(self_adv2d_t h, double t);
  * (nullable) is the device time of the steps. */
 int self_adv2d_forward_step_rk3(self_adv2d_t h, double tn, int nSteps, double *elapsed_ms);
 int self_adv2d_synchronize(self_adv2d_t h);
+/* As self_sw2d_resident_counts. */
+int self_adv2d_resident_counts(self_adv2d_t h, int *launches, int *gaveUp);
 /* WritePickup (:2040-2103) / ReadPickup (:2107-2171) of the handle's
  * fields to / from `path` (see self_adv2d_pickup_write). */
 int self_adv2d_write_pickup(self_adv2d_t h, const char *path);
@@ -648,6 +654,10 @@ int self_cgsem2d_solve(self_cgsem2d_t h, int method, int precond, double tol, in
  * (nullable): device time of the whole batch. */
 int self_cgsem2d_solve_batched(self_cgsem2d_t *problems, int nProblems, int precond, double tol, int maxIters,
                                int *ioerr, int *iterations, double *elapsed_ms);
+/* CG solves in one launch so far, and how many of them gave up waiting (beside
+ * other work on the device) and were done by launched iterations.  No
+ * reference counterpart. */
+int self_cgsem2d_resident_counts(self_cgsem2d_t h, int *launches, int *gaveUp);
 /* Restarted FGMRES(mInner) (IterativeSolvers_Class.f90:656-822 control
  * flow) whose operator and preconditioner applications run in FP32 while
  * the basis, Gram-Schmidt (ortho 0 modified, 1 classical twice), Givens

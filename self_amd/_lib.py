@@ -56,6 +56,13 @@ def lib():
     return _lib
 
 
+def resident_counts(fn, h):
+    """(launches, launches that gave up) of a handle's resident form."""
+    n, g = C.c_int(), C.c_int()
+    check(fn(h, C.byref(n), C.byref(g)))
+    return n.value, g.value
+
+
 def check(rc, allow=()):
     if rc != SELF_OK and rc not in allow:
         msg = lib().self_last_error().decode(errors="replace")
@@ -122,6 +129,7 @@ _SIGS = {
     "self_sw2d_calculate_bathymetry_gradient": ([C.c_void_p], C.c_int),
     "self_sw2d_kernel_times": ([C.c_void_p, C.c_double, C.c_int, dp, ip], C.c_int),
     "self_sw2d_synchronize": ([C.c_void_p], C.c_int),
+    "self_sw2d_resident_counts": ([C.c_void_p, ip, ip], C.c_int),
     "self_sw2d_device_bytes": ([C.c_void_p, szp], C.c_int),
     "self_linop_dense_create": ([C.c_int, dp, dp, C.POINTER(C.c_void_p)], C.c_int),
     "self_linop_elliptic1d_create": ([C.c_int, C.c_int, C.c_double, C.POINTER(C.c_void_p)], C.c_int),
@@ -143,6 +151,7 @@ _SIGS = {
     "self_cgsem2d_residual": ([C.c_void_p, dp], C.c_int),
     "self_cgsem2d_solve": ([C.c_void_p, C.c_int, C.c_int, C.c_double, C.c_int, C.c_int, C.c_int, ip, ip, dp,
                             C.c_int, dp], C.c_int),
+    "self_cgsem2d_resident_counts": ([C.c_void_p, ip, ip], C.c_int),
     "self_cgsem2d_solve_batched": ([C.POINTER(C.c_void_p), C.c_int, C.c_int, C.c_double, C.c_int, ip, ip, dp],
                                    C.c_int),
     "self_cgsem2d_mask": ([C.c_void_p, dp], C.c_int),
@@ -166,6 +175,7 @@ _SIGS = {
     "self_adv2d_global_time_derivative": ([C.c_void_p, C.c_double], C.c_int),
     "self_adv2d_forward_step_rk3": ([C.c_void_p, C.c_double, C.c_int, dp], C.c_int),
     "self_adv2d_synchronize": ([C.c_void_p], C.c_int),
+    "self_adv2d_resident_counts": ([C.c_void_p, ip, ip], C.c_int),
     "self_nodal3d_build": ([C.c_int, C.c_int, C.c_int, dp, dp, dp, dp, dp], C.c_int),
     "self_rolloff_filter1d": ([C.c_int, C.c_int, dp, dp, dp], C.c_int),
     "self_hexmesh_counts": ([C.c_int] * 6 + [ip, ip], C.c_int),

@@ -163,3 +163,7 @@ class Advection:
 
     def Synchronize(self):
         L.check(L.lib().self_adv2d_synchronize(self._h))
+
+    def ResidentCounts(self):
+        """(launches of several steps at once, how many of them gave up)."""
+        return L.resident_counts(L.lib().self_adv2d_resident_counts, self._h)

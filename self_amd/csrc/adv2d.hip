@@ -1048,7 +1048,7 @@ try {
     SELF_REQUIRE(h && nSteps >= 0, SELF_ERR_ARG, "bad arguments");
     SELF_HIP(hipSetDevice(h->device));
     int rc = SELF_OK;
-    const bool resident = !h->runs.off && nSteps >= 1;
+    const bool resident = !h->runs.off && nSteps >= 1 && h->runs.ups.tries();
     if (!resident || elapsed_ms)
         if ((rc = settle(h))) return rc;
     if (!resident && !h->trValid) {
@@ -1064,7 +1064,7 @@ try {
     int s = 0;
     while (resident && s < nSteps && !rc) {
         if (h->runs.pending.size() >= 64) rc = settle(h);
-        if (rc || h->runs.off) break;
+        if (rc || h->runs.ups.rest > 0) break;
         const int n = std::min(nSteps - s, kPersistMaxSteps);
         ADV_DISPATCH(h->N, h->nq, rc = (launch_steps<NN, QQ>(h, tn, s, n)));
         s += n;
@@ -1081,10 +1081,10 @@ try {
         *elapsed_ms = ms;
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
-        const int gaveUp = h->runs.gaveUp;
+        const int gaveUp = h->runs.ups.total;
         const auto t0 = std::chrono::steady_clock::now();
         if (!rc) rc = settle(h);
-        if (h->runs.gaveUp != gaveUp)  // the steps ran (again) in there
+        if (h->runs.ups.total != gaveUp)  // the steps ran (again) in there
             *elapsed_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     }
     return rc;
@@ -1118,6 +1118,16 @@ try {
     if (!rc) rc = self_adv2d_set_field(h, 3, rFac.data());
     if (!rc) rc = self_adv2d_set_field(h, 1, vel.data());
     return rc;
+}
+SELF_CATCH_ALL
+
+int self_adv2d_resident_counts(self_adv2d_t h, int *launches, int *gaveUp)
+try {
+    SELF_REQUIRE(h && launches && gaveUp, SELF_ERR_ARG, "null argument");
+    if (int rc = settle(h)) return rc;
+    *launches = h->runs.ups.launches;
+    *gaveUp = h->runs.ups.total;
+    return SELF_OK;
 }
 SELF_CATCH_ALL
 

@@ -437,7 +437,8 @@ struct CgsemOp final : DevOp {
     int maxCopies = 0;              // copies of the most shared DOF
     char *resBuf = nullptr;
     size_t resBytes = 0;
-    int resLaunches = 0, resGaveUp = 0;
+    GiveUps resUps;
+    bool resOff = false;            // no memory for it
     unsigned resTag = 0;            // of the last iteration settled
     bool resDirty = false;          // messages of a launch not settled, or never cleared
     std::vector<double> kH;         // flux coefficient last set (host, local layout; empty = ONE)
@@ -550,7 +551,7 @@ struct CgsemOp final : DevOp {
             resBytes = res_exch() + kResRed + sizeof(CgResOut) + 64;
             if (dev(&resBuf, resBytes) != SELF_OK) {  // no memory for it: the two-launch form needs none
                 (void)hipGetLastError();
-                resGaveUp = 4;
+                resOff = true;
                 return SELF_OK;
             }
             resDirty = true;
@@ -579,7 +580,7 @@ struct CgsemOp final : DevOp {
         A.tag0 = resTag;
         A.out = reinterpret_cast<CgResOut *>(resBuf + res_exch() + kResRed);
         A.P.status = reinterpret_cast<int *>(resBuf + resBytes - 64);
-        A.P.launch = ++resLaunches;
+        A.P.launch = ++resUps.launches;
         A.P.limit = persist_spin_limit();
         PersistGate gate(device, s, blocks, 1);
         if (gate.rc) return gate.rc;
@@ -595,7 +596,7 @@ struct CgsemOp final : DevOp {
     int resident_cg(KrylovWork &wk, bool precond, bool &taken, hipStream_t s) override
     {
         taken = false;
-        if (resGaveUp >= 4 || maxCopies > 4 || res_exch() >= (1u << 31)) return SELF_OK;
+        if (resOff || maxCopies > 4 || res_exch() >= (1u << 31) || !resUps.tries()) return SELF_OK;
         int rc = SELF_OK;
         // As few nodes a thread as the device has workgroups for; one a thread
         // only on up to 7/8 of the CUs (64x64, N = 7: 7.8 us an iteration on 256
@@ -611,10 +612,11 @@ struct CgsemOp final : DevOp {
     int resident_cg_end(KrylovWork &wk, const SolverState &h, bool &gaveUp, hipStream_t s) override
     {
         gaveUp = h.done == kCgGaveUp;
-        if (gaveUp) {  // beside much other work on the device it will happen again
-            ++resGaveUp;
+        if (gaveUp) {
+            resUps.gaveUp();
             return SELF_OK;
         }
+        resUps.finished();
         resDirty = false;
         if (h.done != 3) {  // 3: nothing to solve, the launch returned at once
             std::swap(wk.u, wk.z);
@@ -1330,6 +1332,14 @@ try {
     return SELF_OK;
 }
 SELF_CATCH_ALL
+
+int self_cgsem2d_resident_counts(self_cgsem2d_t h, int *launches, int *gaveUp)
+{
+    SELF_REQUIRE(h && launches && gaveUp, SELF_ERR_ARG, "null argument");
+    *launches = h->op.resUps.launches;
+    *gaveUp = h->op.resUps.total;
+    return SELF_OK;
+}
 
 int self_cgsem2d_solve_batched(self_cgsem2d_t *problems, int nProblems, int precond, double tol, int maxIters,
                                int *ioerr, int *iterations, double *elapsed_ms)

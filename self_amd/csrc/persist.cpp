@@ -88,8 +88,11 @@ int ResidentRuns::settle(hipStream_t s, std::vector<Run> &again)
     SELF_HIP(hipStreamSynchronize(s));
     std::vector<Run> done;
     done.swap(pending);
-    if (bad == 0) return SELF_OK;
-    if (++gaveUp >= 4) off = true;
+    if (bad == 0) {
+        ups.finished();
+        return SELF_OK;
+    }
+    ups.gaveUp();
     if (int rc = clear(s)) return rc;
     size_t first = 0;
     while (first < done.size() && done[first].launch != bad) ++first;

@@ -148,6 +148,26 @@ int persist_blocks_per_cu(const void *kernel, int threads);
 int persist_cus(int device);
 unsigned persist_spin_limit();
 
+// Whether a resident form is tried.  Beside much other work on the device a
+// launch that gave up will be followed by others, and each costs a wait to its
+// bound (about 2 ms); after four in a row the ordinary launches serve the next
+// 256 calls (8 us of waiting a call at worst), then the form is tried again.
+struct GiveUps {
+    int launches = 0, total = 0, inRow = 0, rest = 0;
+    bool tries()  // once a call
+    {
+        if (rest == 0) return true;
+        --rest;
+        return false;
+    }
+    void finished() { inRow = 0; }
+    void gaveUp()
+    {
+        ++total;
+        if (++inRow >= 4) rest = 256;
+    }
+};
+
 // Steps of one launch at most: the launches between two settlings stay
 // countable, and 3 x steps in an int.
 constexpr int kPersistMaxSteps = 1 << 16;
@@ -155,8 +175,7 @@ constexpr int kPersistMaxSteps = 1 << 16;
 // Launches of resident time steps that are not yet known to have finished, and
 // the messages they exchange.  A launch that gave up left its input as it was
 // and made the later ones return at once: settle() waits for them and lists the
-// runs to do over by ordinary launches.  After several such launches `off` is
-// set: beside much other work on the device it happens again.
+// runs to do over by ordinary launches.
 // The tags of stages count on over the launches.  That a word holds the wanted
 // tag or an older one of the last two is true only while every launch writes all
 // its messages; after one that gave up, words of any earlier stage are left, and
@@ -173,15 +192,15 @@ struct ResidentRuns {
     ll_quad *messages = nullptr;
     size_t messageBytes = 0;
     unsigned tag = 0;              // of the last stage launched; the cleared messages' is 0
-    int launches = 0, gaveUp = 0;
-    bool off = false;
+    GiveUps ups;
+    bool off = false;              // the model does not fit, or there was no memory for its buffers
     std::vector<Run> pending;
-    PersistArgs args() const { return {status, launches + 1, persist_spin_limit()}; }
+    PersistArgs args() const { return {status, ups.launches + 1, persist_spin_limit()}; }
     // call it as soon as the launch is queued: its messages will have been written
     void launched(int first, int steps, double t0, double *in)
     {
         tag += 3u * (unsigned)steps;
-        pending.push_back({++launches, first, steps, t0, in});
+        pending.push_back({++ups.launches, first, steps, t0, in});
     }
     int clear(hipStream_t s);      // messages and status, before the first launch
     int settle(hipStream_t s, std::vector<Run> &again);

@@ -2121,11 +2121,11 @@ int self_sw2d_forward_step_rk3(self_sw2d_t h, double tn, int nSteps)
     SELF_REQUIRE(nSteps >= 0, SELF_ERR_ARG, "negative step count");
     int s = 0;
     if (h->d.form == SELF_FUSED && h->useGraph && !h->runs.off && nSteps >= 2 &&
-        fused_groups(h->groups, h->nE, 0) == 1) {
+        fused_groups(h->groups, h->nE, 0) == 1 && h->runs.ups.tries()) {
         bool taken = true;
         while (s < nSteps && taken) {
             if (h->runs.pending.size() >= 64 && (rc = settle(h))) return rc;
-            if (h->runs.off) break;
+            if (h->runs.ups.rest > 0) break;
             const int n = std::min(nSteps - s, kPersistMaxSteps);
             if ((rc = steps_persistent(h, n, taken))) return rc;
             if (taken) s += n;
@@ -2161,10 +2161,10 @@ int self_sw2d_forward_step_rk3_timed(self_sw2d_t h, double tn, int nSteps, doubl
     float ms = 0.0f;
     SELF_HIP(hipEventElapsedTime(&ms, h->ev0, h->ev1));
     *elapsed_ms = ms;
-    const int gaveUp = h->runs.gaveUp;
+    const int gaveUp = h->runs.ups.total;
     const auto t0 = std::chrono::steady_clock::now();
     rc = settle(h);
-    if (h->runs.gaveUp != gaveUp)  // the steps ran (again) in there
+    if (h->runs.ups.total != gaveUp)  // the steps ran (again) in there
         *elapsed_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     return rc;
 }
@@ -2564,6 +2564,16 @@ int self_sw2d_synchronize(self_sw2d_t h)
     SELF_HIP(hipStreamSynchronize(h->stream));
     return settle(h);
 }
+
+int self_sw2d_resident_counts(self_sw2d_t h, int *launches, int *gaveUp)
+try {
+    SELF_REQUIRE(h && launches && gaveUp, SELF_ERR_ARG, "null argument");
+    if (int rc = settle(h)) return rc;
+    *launches = h->runs.ups.launches;
+    *gaveUp = h->runs.ups.total;
+    return SELF_OK;
+}
+SELF_CATCH_ALL
 
 int self_sw2d_device_bytes(self_sw2d_t h, size_t *bytes)
 {

@@ -210,6 +210,10 @@ class CGsemElliptic2D:
         L.check(L.lib().self_cgsem2d_apply_preconditioner(self._h, L.ptr(self._arr(b)), L.ptr(out), C.byref(it)))
         return out, it.value
 
+    def ResidentCounts(self):
+        """(CG solves in one launch, how many of them gave up)."""
+        return L.resident_counts(L.lib().self_cgsem2d_resident_counts, self._h)
+
     def SolveGMRESMixed(self, tolerance=1e-10, maxCycles=50, mInner=30, precond="fem", ortho=MGS):
         """Restarted FGMRES(mInner) with FP32 operator and preconditioner
         applications and FP64 basis, orthogonalisation and restart

@@ -294,6 +294,10 @@ class ShallowWater:
     def Synchronize(self):
         L.check(L.lib().self_sw2d_synchronize(self._h))
 
+    def ResidentCounts(self):
+        """(launches of several steps at once, how many of them gave up)."""
+        return L.resident_counts(L.lib().self_sw2d_resident_counts, self._h)
+
     def DeviceBytes(self):
         b = C.c_size_t()
         L.check(L.lib().self_sw2d_device_bytes(self._h, C.byref(b)))

@@ -37,7 +37,13 @@ CASES = [dict(N=N, nX=5 + N % 3, nY=4, nq=1 + N % 4) for N in range(1, 9)] + [
     dict(N=4, nX=31, nY=17, nq=3, relax=True, warp=0.02),
     dict(N=2, nX=9, nY=11, nq=2, periodic=False, inflow=True),
     dict(N=5, nX=60, nY=50, nq=1),
+    dict(N=1, nX=13, nY=12, nq=3, warp=0.02),
+    dict(N=2, nX=12, nY=9, nq=4, relax=True),
 ]
+
+
+def _workgroups(case):
+    return -(-case["nX"] * case["nY"] // (256 // (case["N"] + 1) ** 2))
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(v) for v in c.values()))
@@ -57,9 +63,14 @@ def test_resident_steps_equal_launches(gpu_lib, case, monkeypatch):
     monkeypatch.delenv("SELF_AMD_SPIN_LIMIT")
     assert np.isfinite(want).all() and not np.array_equal(want, _model(**case).GetSolution())
     assert np.array_equal(got, want)
+    # a model of one workgroup may find its messages at the first poll
+    assert a.ResidentCounts() == (3, 0)
+    if _workgroups(case) > 1:
+        assert b.ResidentCounts() == (3, 1)
     b.ForwardStepRK3(t, 3)  # the form is taken up again
     a.ForwardStepRK3(t, 3)
     assert np.array_equal(a.GetSolution(), b.GetSolution())
+    assert b.ResidentCounts() == (4, 1 if _workgroups(case) > 1 else b.ResidentCounts()[1])
     a.GlobalTimeDerivative(t)
     b.GlobalTimeDerivative(t)
     assert np.array_equal(a.GetTendency(), b.GetTendency())
@@ -67,7 +78,7 @@ def test_resident_steps_equal_launches(gpu_lib, case, monkeypatch):
     b.Trash()
 
 
-@pytest.mark.parametrize("case", [CASES[0], CASES[2], CASES[8], CASES[10], CASES[11]],
+@pytest.mark.parametrize("case", [CASES[14], CASES[2], CASES[8], CASES[10], CASES[11]],
                          ids=lambda c: "-".join(str(v) for v in c.values()))
 def test_gradient_after_steps(gpu_lib, case, monkeypatch):
     """GetGradient after ForwardStepRK3 is the last stage's, as the launched
@@ -79,10 +90,12 @@ def test_gradient_after_steps(gpu_lib, case, monkeypatch):
         b.Synchronize()
     want = b.GetGradient()
     monkeypatch.delenv("SELF_AMD_SPIN_LIMIT")
+    assert _workgroups(case) == 1 or b.ResidentCounts() == (2, 2)
     a.GlobalTimeDerivative(0.1)
     before = a.GetGradient()
     for n in (1, 4):
         a.ForwardStepRK3(0.1, n)
+    assert a.ResidentCounts() == (2, 0)
     for g, w, o in zip(a.GetGradient(), want, before):
         assert np.isfinite(w).all() and np.array_equal(g, w) and not np.array_equal(g, o)
     a.Trash()
@@ -102,6 +115,7 @@ def test_tags_come_round_after_a_launch_gave_up(gpu_lib, monkeypatch):
     a.ForwardStepRK3(0.2, 65536 + 3)
     a.Synchronize()
     monkeypatch.delenv("SELF_AMD_SPIN_LIMIT")
+    assert a.ResidentCounts() == (2, 1)  # the second returned at once
     a.ForwardStepRK3(0.3, 2)
     want = b.GetSolution()
     assert np.isfinite(want).all() and np.array_equal(a.GetSolution(), want)

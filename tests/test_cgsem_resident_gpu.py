@@ -36,17 +36,29 @@ def _solve(m, precond, tol, iters, start=None):
 
 SHAPES = [(2, 7, 9), (3, 4, 4), (3, 21, 13), (4, 11, 6), (5, 3, 2), (5, 30, 17), (6, 8, 8), (7, 5, 7),
           (7, 63, 57), (8, 9, 5), (9, 6, 6), (10, 4, 5), (11, 5, 3), (7, 80, 61), (3, 150, 131), (5, 122, 101),
-          (7, 128, 127), (10, 75, 60), (7, 130, 128)]
+          (7, 128, 127), (10, 75, 60), (7, 130, 128), (2, 23, 19)]
+
+
+def _workgroups(N, nX, nY):  # at one node a thread
+    return -(-nX * nY // (1024 // (N + 1) ** 2))
+
+
+def _counted(m, launches, gaveUp, several):
+    n, g = m.ResidentCounts()
+    # a problem of one workgroup may find its messages at the first poll
+    assert n == launches and (g == gaveUp or not several), (n, g)
 
 
 @pytest.mark.parametrize("N,nX,nY", SHAPES)
 def test_one_launch_follows_the_launched_iterations(gpu_lib, N, nX, nY, monkeypatch):
     m = _model(N, nX, nY, warp=0.03 if nX < 40 else 0.0, boundary=True)
-    for precond in ("jacobi", "none"):
+    fits = nX * nY * (N + 1) ** 2 <= 1 << 20
+    for k, precond in enumerate(("jacobi", "none")):
         a, ia, _, ra = _solve(m, precond, 1e-300, 12)
         monkeypatch.setenv("SELF_AMD_SPIN_LIMIT", "0")
         b, ib, _, rb = _solve(m, precond, 1e-300, 12)
         monkeypatch.delenv("SELF_AMD_SPIN_LIMIT")
+        _counted(m, 2 * k + 2 if fits else 0, k + 1 if fits else 0, _workgroups(N, nX, nY) > 1)
         assert ia == ib == 12
         assert rel_l2(a, b) < 1e-12
         assert np.allclose(ra[:13], rb[:13], rtol=1e-10, atol=0)
@@ -62,12 +74,14 @@ def test_solutions_and_stop(gpu_lib, N, nX, nY, monkeypatch):
     monkeypatch.setenv("SELF_AMD_SPIN_LIMIT", "0")
     b, ib, iob, _ = _solve(m, "jacobi", 1e-11, 20000)
     monkeypatch.delenv("SELF_AMD_SPIN_LIMIT")
+    _counted(m, 3, 1, _workgroups(N, nX, nY) > 1)
     assert ioa == iob and abs(ia - ib) <= 2 + ib // 100
     assert ra[ia] / ra[0] < 1e-11 <= ra[ia - 1] / ra[0]
     assert rel_l2(a, b) < 1e-7
     # begun at the solution: few iterations, and the form is still taken
     c, it, _, _ = _solve(m, "jacobi", 1e-3, 100, start=a)
     assert np.isfinite(c).all() and it <= 100
+    _counted(m, 4, 1, _workgroups(N, nX, nY) > 1)
     m.Trash()
 
 

@@ -77,6 +77,8 @@ def test_resident_steps_equal_stage_launches(gpu_lib, case):
     assert all(np.isfinite(w).all() for w in want)
     for g, w in zip(got, want):
         assert np.array_equal(g, w)
+    assert b.ResidentCounts() == (0, 0)
+    assert a.ResidentCounts() == ((0, 0) if case["nX"] == 65 else (3, 0))  # every call of two steps or more
     a.Trash()
     b.Trash()
 
@@ -95,10 +97,43 @@ def test_steps_run_again_where_a_launch_gives_up(gpu_lib, case, monkeypatch):
     a.ForwardStepRK3(0.0, 2)  # returns at once behind the one that gave up
     for g, w in zip(_states(a, members), _states(b, members)):
         assert np.array_equal(g, w)
+    assert a.ResidentCounts() == (3, 1)
     a.ForwardStepRK3(0.0, 6)  # and the form is taken up again
     b.ForwardStepRK3(0.0, 6)
     for g, w in zip(_states(a, members), _states(b, members)):
         assert np.array_equal(g, w)
+    assert a.ResidentCounts() == (4, 1)
+    a.Trash()
+    b.Trash()
+
+
+def test_the_form_rests_after_four_launches_in_a_row_gave_up(gpu_lib, monkeypatch):
+    case = CASES[4]
+    a, b = _model(**case), _model(**case)
+    b.SetGraph(False)
+
+    def step(n):
+        for _ in range(n):
+            a.ForwardStepRK3(0.0, 2)
+            b.ForwardStepRK3(0.0, 2)
+
+    monkeypatch.setenv("SELF_AMD_SPIN_LIMIT", "0")
+    for k in range(3):
+        step(1)
+        assert a.ResidentCounts() == (k + 1, k + 1)
+    monkeypatch.delenv("SELF_AMD_SPIN_LIMIT")
+    step(1)  # one that finishes: the count begins again
+    assert a.ResidentCounts() == (4, 3)
+    monkeypatch.setenv("SELF_AMD_SPIN_LIMIT", "0")
+    for k in range(4):
+        step(1)
+        assert a.ResidentCounts() == (k + 5, k + 4)
+    monkeypatch.delenv("SELF_AMD_SPIN_LIMIT")
+    step(256)
+    assert a.ResidentCounts() == (8, 7)
+    step(1)
+    assert a.ResidentCounts() == (9, 7)
+    assert np.array_equal(a.GetSolution(), b.GetSolution())
     a.Trash()
     b.Trash()
 
@@ -136,6 +171,7 @@ def test_tags_come_round_after_a_launch_gave_up(gpu_lib, monkeypatch):
     a.ForwardStepRK3(0.0, 65536)
     a.Synchronize()
     monkeypatch.delenv("SELF_AMD_SPIN_LIMIT")
+    assert a.ResidentCounts() == (1, 1)
     a.ForwardStepRK3(0.0, 2)
     want = b.GetSolution()
     assert np.isfinite(want).all() and np.array_equal(a.GetSolution(), want)
