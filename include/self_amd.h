@@ -655,8 +655,8 @@ int self_cgsem2d_solve(self_cgsem2d_t h, int method, int precond, double tol, in
 int self_cgsem2d_solve_batched(self_cgsem2d_t *problems, int nProblems, int precond, double tol, int maxIters,
                                int *ioerr, int *iterations, double *elapsed_ms);
 /* CG solves in one launch so far, and how many of them gave up waiting (beside
- * other work on the device) and were done by launched iterations.  No
- * reference counterpart. */
+ * other work on the device) and were done by launched iterations, with the
+ * same result.  No reference counterpart. */
 int self_cgsem2d_resident_counts(self_cgsem2d_t h, int *launches, int *gaveUp);
 /* Restarted FGMRES(mInner) (IterativeSolvers_Class.f90:656-822 control
  * flow) whose operator and preconditioner applications run in FP32 while

@@ -23,8 +23,12 @@
 // -> 12.0 there, 10.5 -> 9.5 at 100x100 N = 5.
 //
 // The recurrences, the copies' summation order (GlobalSum) and the stop test
-// are those of the launched form; the dot products are summed in another fixed
-// order, which depends on the problem's shape only.
+// are those of the launched form for larger problems; the dot products are
+// summed in another fixed order, which depends on the problem's shape only.  So
+// that a result does not depend on whether the launch was resident (other work
+// on the device, memory for its messages), a problem of a resident shape that
+// does not run it takes three launches an iteration that form the same values
+// in the same order (k_cg_ord_*), bit for bit.
 #pragma once
 
 #include "dg2d_device.hpp"
@@ -64,14 +68,87 @@ struct CgMfOps {
     double a[Mf<N>::K], b[Mf<N>::K], at[Mf<N>::K], bt[Mf<N>::K];
 };
 
+template <int N>
+__device__ __forceinline__ void cg_mf_ops(CgMfOps<N> &M, const double *Dl, int tl)
+{
+    constexpr int n1 = N + 1;
+    const MfLane<N> a(tl);
+    #pragma unroll
+    for (int q = 0; q < Mf<N>::K; ++q) {
+        const int m = 4 * q + a.k;
+        M.a[q] = Dl[(4 * a.bi + a.c) + n1 * m];
+        M.b[q] = Dl[(4 * a.bj + a.c) + n1 * m];
+        M.at[q] = Dl[m + n1 * (4 * a.bi + a.c)];
+        M.bt[q] = Dl[m + n1 * (4 * a.bj + a.c)];
+    }
+}
+
+// the element operator at one node of an element (in: the lane has one)
+template <int N, int S, bool WL, typename F12, typename F22>
+__device__ __forceinline__ double cg_element_product(const CgMfOps<N> &M, const double *Dl, double *usE, double *f1E,
+                                                     double *f2E, double v, double g11, F12 g12of, F22 g22of, bool in,
+                                                     int tl, int i, int j)
+{
+    #pragma clang fp contract(off)
+    constexpr int n1 = N + 1;
+    constexpr bool MF = Mf<N>::on;
+    const int ns = i + S * j;
+    if (in) usE[ns] = v;
+    if constexpr (WL) wave_sync();
+    else __syncthreads();
+    double ds = 0.0, dp = 0.0;
+    if constexpr (MF) {
+        const MfLane<N> a(tl);
+        #pragma unroll
+        for (int q = 0; q < Mf<N>::K; ++q) {
+            const int m = 4 * q + a.k;
+            ds = __builtin_amdgcn_mfma_f64_4x4x4f64(M.a[q], usE[m + S * (4 * a.bj + a.c)], ds, 0, 0, 0);
+            dp = __builtin_amdgcn_mfma_f64_4x4x4f64(usE[(4 * a.bi + a.c) + S * m], M.b[q], dp, 0, 0, 0);
+        }
+    } else {
+        #pragma unroll
+        for (int m = 0; m < n1; ++m) {
+            ds = __builtin_fma(Dl[i + n1 * m], usE[m + S * j], ds);
+            dp = __builtin_fma(Dl[j + n1 * m], usE[i + S * m], dp);
+        }
+    }
+    if (in) {
+        const double g12 = g12of(), g22 = g22of();
+        f1E[ns] = __builtin_fma(g11, ds, g12 * dp);
+        f2E[ns] = __builtin_fma(g12, ds, g22 * dp);
+    }
+    if constexpr (WL) wave_sync();
+    else __syncthreads();
+    double s1 = 0.0, s2 = 0.0;
+    if constexpr (MF) {
+        const MfLane<N> a(tl);
+        #pragma unroll
+        for (int q = 0; q < Mf<N>::K; ++q) {
+            const int m = 4 * q + a.k;
+            s1 = __builtin_amdgcn_mfma_f64_4x4x4f64(M.at[q], f1E[m + S * (4 * a.bj + a.c)], s1, 0, 0, 0);
+            s2 = __builtin_amdgcn_mfma_f64_4x4x4f64(f2E[(4 * a.bi + a.c) + S * m], M.bt[q], s2, 0, 0, 0);
+        }
+    } else {
+        #pragma unroll
+        for (int m = 0; m < n1; ++m) {
+            s1 = __builtin_fma(Dl[m + n1 * i], f1E[m + S * j], s1);
+            s2 = __builtin_fma(Dl[m + n1 * j], f2E[i + S * m], s2);
+        }
+    }
+    return -(s1 + s2);
+}
+
+// row stride of an element's arrays in LDS: at N = 7 an odd one, or the matrix
+// operands' eight rows fall on four banks
+template <int N>
+constexpr int kCgRow = N == 7 ? N + 2 : N + 1;
+
 template <int N, int K>
 __global__ __launch_bounds__(kCgResThreads) void k_cg_resident(CgResArgs A)
 {
     constexpr int n1 = N + 1, np = n1 * n1, T = kCgResThreads, epb = T / np, W = T / 64;
-    constexpr bool MF = Mf<N>::on, WL = 64 % np == 0;
-    // row stride of an element's arrays in LDS: at N = 7 an odd one, or the
-    // matrix operands' eight rows fall on four banks
-    constexpr int S = N == 7 ? n1 + 1 : n1, ne = S * n1;
+    constexpr bool WL = 64 % np == 0;
+    constexpr int S = kCgRow<N>, ne = S * n1;
     // four nodes a thread: the solution, the inverse diagonal and as many of the
     // geometric factors as there is room for live in LDS (128 KB at N = 7)
     constexpr bool UD = K > 2;
@@ -96,23 +173,13 @@ __global__ __launch_bounds__(kCgResThreads) void k_cg_resident(CgResArgs A)
     if (stop) return;
     const int b = xcd_block(blockIdx.x, gridDim.x), nB = gridDim.x;
     int tl;
-    const int le = lane_element<N>(t, tl), nd = lane_node<N>(tl), i = nd % n1, j = nd / n1, ns = i + S * j;
+    const int le = lane_element<N>(t, tl), nd = lane_node<N>(tl), i = nd % n1, j = nd / n1;
     const int ls = le < epb ? le : 0;
     // where a wavefront holds whole elements its flux takes the values' place
     // (a wavefront's LDS operations are done in order)
     double *usE = us + ls * ne, *f1E = WL ? usE : f1 + ls * ne, *f2E = f2 + ls * ne;
     CgMfOps<N> M;
-    if constexpr (MF) {
-        const MfLane<N> a(tl);
-        #pragma unroll
-        for (int q = 0; q < Mf<N>::K; ++q) {
-            const int m = 4 * q + a.k;
-            M.a[q] = Dl[(4 * a.bi + a.c) + n1 * m];
-            M.b[q] = Dl[(4 * a.bj + a.c) + n1 * m];
-            M.at[q] = Dl[m + n1 * (4 * a.bi + a.c)];
-            M.bt[q] = Dl[m + n1 * (4 * a.bj + a.c)];
-        }
-    }
+    if constexpr (Mf<N>::on) cg_mf_ops<N>(M, Dl, tl);
     // corner lanes: entry (k epb + le) 4 + which of the table
     const bool isCorner = le < epb && (i == 0 || i == N) && (j == 0 || j == N);
     const int cEntry = isCorner ? ls * 4 + (i ? 1 : 0) + (j ? 2 : 0) : NC;
@@ -182,53 +249,17 @@ __global__ __launch_bounds__(kCgResThreads) void k_cg_resident(CgResArgs A)
         #pragma unroll
         for (int k = 0; k < K; ++k) {
             v[k] = __builtin_fma(beta, v[k], dinv(k) * r[k]);  // beta = 0, v = 0 in the first iteration
-            if (le < epb) usE[ns] = v[k];
-            if constexpr (WL) wave_sync();
-            else __syncthreads();
-            double ds = 0.0, dp = 0.0;
-            if constexpr (MF) {
-                const MfLane<N> a(tl);
-                #pragma unroll
-                for (int q = 0; q < Mf<N>::K; ++q) {
-                    const int m = 4 * q + a.k;
-                    ds = __builtin_amdgcn_mfma_f64_4x4x4f64(M.a[q], usE[m + S * (4 * a.bj + a.c)], ds, 0, 0, 0);
-                    dp = __builtin_amdgcn_mfma_f64_4x4x4f64(usE[(4 * a.bi + a.c) + S * m], M.b[q], dp, 0, 0, 0);
-                }
-            } else {
-                #pragma unroll
-                for (int m = 0; m < n1; ++m) {
-                    ds = __builtin_fma(Dl[i + n1 * m], usE[m + S * j], ds);
-                    dp = __builtin_fma(Dl[j + n1 * m], usE[i + S * m], dp);
-                }
-            }
-            if (le < epb) {
-                double g12, g22;
-                if constexpr (GL > 1) g12 = gl[1][k * T + t];
-                else g12 = g12r[k];
-                if constexpr (GL > 0) g22 = gl[0][k * T + t];
-                else g22 = g22r[k];
-                f1E[ns] = __builtin_fma(g11[k], ds, g12 * dp);
-                f2E[ns] = __builtin_fma(g12, ds, g22 * dp);
-            }
-            if constexpr (WL) wave_sync();
-            else __syncthreads();
-            double s1 = 0.0, s2 = 0.0;
-            if constexpr (MF) {
-                const MfLane<N> a(tl);
-                #pragma unroll
-                for (int q = 0; q < Mf<N>::K; ++q) {
-                    const int m = 4 * q + a.k;
-                    s1 = __builtin_amdgcn_mfma_f64_4x4x4f64(M.at[q], f1E[m + S * (4 * a.bj + a.c)], s1, 0, 0, 0);
-                    s2 = __builtin_amdgcn_mfma_f64_4x4x4f64(f2E[(4 * a.bi + a.c) + S * m], M.bt[q], s2, 0, 0, 0);
-                }
-            } else {
-                #pragma unroll
-                for (int m = 0; m < n1; ++m) {
-                    s1 = __builtin_fma(Dl[m + n1 * i], f1E[m + S * j], s1);
-                    s2 = __builtin_fma(Dl[m + n1 * j], f2E[i + S * m], s2);
-                }
-            }
-            L[k] = -(s1 + s2);
+            L[k] = cg_element_product<N, S, WL>(
+                M, Dl, usE, f1E, f2E, v[k], g11[k],
+                [&] {
+                    if constexpr (GL > 1) return gl[1][k * T + t];
+                    else return g12r[k];
+                },
+                [&] {
+                    if constexpr (GL > 0) return gl[0][k * T + t];
+                    else return g22r[k];
+                },
+                le < epb, tl, i, j);
             acc = __builtin_fma(v[k], L[k], acc);
             // a store past the buffer's end is dropped
             ll_store1(exch, (16u * (unsigned)(((b * K + k) * epb + le) * np + nd)) | (kNoMsg & ~(unsigned)bits(k, 0)), L[k], tag);
@@ -368,6 +399,132 @@ __global__ void k_cg_res_commit(SolverState *st, const CgResOut *out, const int 
     st->rNorm = out->rNorm;
     st->iter = out->iter;
     st->done = out->done;
+}
+
+// ---- the same iteration as three launches.  A thread has the resident form's
+// nodes, so every sum has its order; vectors are indexed by degree of freedom,
+// written by the owner copies (the direction to another array than it is read
+// from).  Rows 0, 1, 2 of the partial sums: v.Av, r.r, r.w, an entry a workgroup.
+struct CgOrdArgs {
+    const int *gid, *cs, *ci;
+    const double *G3, *D, *dinv;
+    double *r, *u, *vNew, *L;
+    const double *vOld;
+    double *partials;  // rows of kRedBlocks
+    SolverState *st;
+    int nE, it;
+};
+
+// sum of 16 wavefronts' values, one after another (thread 0's result counts)
+__device__ __forceinline__ double cg_ord_block(double v, double (&part)[kCgResThreads / 64])
+{
+    v = wave_sum_dpp(v);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double p = part[0];
+    #pragma unroll
+    for (int q = 1; q < kCgResThreads / 64; ++q) p += part[q];
+    return p;
+}
+
+// sum of nB workgroups' values in every thread; the first 256 threads call with
+// on = true
+__device__ __forceinline__ double cg_ord_fold(const double *row, int nB, bool on, double (&fold)[4])
+{
+    if (on) {
+        const int t = threadIdx.x;
+        const double x = wave_sum_dpp(t < nB ? row[t] : 0.0);
+        if ((t & 63) == 0) fold[t >> 6] = x;
+    }
+    __syncthreads();
+    return (fold[0] + fold[1]) + (fold[2] + fold[3]);
+}
+
+template <int N, int K>
+__global__ __launch_bounds__(kCgResThreads) void k_cg_ord_direction(CgOrdArgs A)
+{
+    #pragma clang fp contract(off)
+    constexpr int n1 = N + 1, np = n1 * n1, T = kCgResThreads, epb = T / np, S = kCgRow<N>, ne = S * n1;
+    constexpr bool WL = 64 % np == 0;
+    __shared__ double Dl[np], us[epb * ne], f1[WL ? 1 : epb * ne], f2[epb * ne], part[T / 64];
+    if (A.st->done) return;  // nothing writes it during this kernel
+    const int t = threadIdx.x;
+    if (t < np) Dl[t] = A.D[t];
+    __syncthreads();
+    int tl;
+    const int b = xcd_block(blockIdx.x, gridDim.x);
+    const int le = lane_element<N>(t, tl), nd = lane_node<N>(tl), i = nd % n1, j = nd / n1, ls = le < epb ? le : 0;
+    double *usE = us + ls * ne, *f1E = WL ? usE : f1 + ls * ne, *f2E = f2 + ls * ne;
+    CgMfOps<N> M;
+    if constexpr (Mf<N>::on) cg_mf_ops<N>(M, Dl, tl);
+    const double beta = A.it == 1 ? 0.0 : A.st->beta;
+    const size_t nLocal = (size_t)A.nE * np;
+    double acc = 0.0;
+    for (int k = 0; k < K; ++k) {
+        const int e = (b * K + k) * epb + le;
+        const bool act = le < epb && e < A.nE;
+        const size_t l = act ? (size_t)e * np + nd : 0;
+        const int g = act ? A.gid[l] : -1, gc = max(g, 0);
+        const double g11 = act ? A.G3[l] : 0.0, g12 = act ? A.G3[nLocal + l] : 0.0,
+                     g22 = act ? A.G3[2 * nLocal + l] : 0.0;
+        const double r = g >= 0 ? A.r[gc] : 0.0, vo = g >= 0 && A.it > 1 ? A.vOld[gc] : 0.0;
+        const double d = g >= 0 ? (A.dinv ? A.dinv[gc] : 1.0) : 0.0;
+        const double v = __builtin_fma(beta, vo, d * r);
+        const double L = cg_element_product<N, S, WL>(
+            M, Dl, usE, f1E, f2E, v, g11, [&] { return g12; }, [&] { return g22; }, le < epb, tl, i, j);
+        acc = __builtin_fma(v, L, acc);
+        if (act) A.L[l] = L;
+        if (g >= 0 && A.ci[A.cs[gc]] == (int)l) A.vNew[g] = v;
+    }
+    acc = cg_ord_block(acc, part);
+    if (t == 0) A.partials[b] = acc;
+}
+
+template <int N, int K>
+__global__ __launch_bounds__(kCgResThreads) void k_cg_ord_update(CgOrdArgs A)
+{
+    #pragma clang fp contract(off)
+    constexpr int n1 = N + 1, np = n1 * n1, T = kCgResThreads, epb = T / np;
+    __shared__ double part0[T / 64], part1[T / 64], fold[4];
+    if (A.st->done) return;
+    const int t = threadIdx.x, b = xcd_block(blockIdx.x, gridDim.x);
+    const double vz = cg_ord_fold(A.partials, gridDim.x, t < 256, fold);
+    const double alpha = A.st->numP[A.it & 1] / vz;
+    int tl;
+    const int le = lane_element<N>(t, tl), nd = lane_node<N>(tl);
+    double a0 = 0.0, a1 = 0.0;
+    for (int k = 0; k < K; ++k) {
+        const int e = (b * K + k) * epb + le;
+        if (le >= epb || e >= A.nE) continue;
+        const size_t l = (size_t)e * np + nd;
+        const int g = A.gid[l];
+        if (g < 0) continue;
+        const int c0 = A.cs[g], n = A.cs[g + 1] - c0;
+        if (A.ci[c0] != (int)l) continue;
+        double z = A.L[l] + (n > 1 ? A.L[A.ci[c0 + 1]] : 0.0);
+        if (n > 2) z = (z + A.L[A.ci[c0 + 2]]) + (n > 3 ? A.L[A.ci[c0 + 3]] : 0.0);
+        A.u[g] = __builtin_fma(alpha, A.vNew[g], A.u[g]);
+        const double r = __builtin_fma(-alpha, z, A.r[g]);
+        A.r[g] = r;
+        a0 = __builtin_fma(r, r, a0);
+        a1 = __builtin_fma(r, (A.dinv ? A.dinv[g] : 1.0) * r, a1);
+    }
+    a0 = cg_ord_block(a0, part0);
+    a1 = cg_ord_block(a1, part1);
+    if (t == 0) {
+        A.partials[kRedBlocks + b] = a0;
+        A.partials[2 * kRedBlocks + b] = a1;
+    }
+}
+
+// one workgroup of 256: the end of iteration A.it from nB workgroups' sums
+__global__ __launch_bounds__(256) void k_cg_ord_end(CgOrdArgs A, int nB)
+{
+    __shared__ double fold0[4], fold1[4];
+    if (A.st->done) return;
+    const double S0 = cg_ord_fold(A.partials + kRedBlocks, nB, true, fold0);
+    const double S1 = cg_ord_fold(A.partials + 2 * kRedBlocks, nB, true, fold1);
+    if (threadIdx.x == 0) cg_end_apply(A.st, A.it, S0, S1);
 }
 
 }  // namespace self

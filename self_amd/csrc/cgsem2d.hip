@@ -538,18 +538,81 @@ struct CgsemOp final : DevOp {
     static constexpr size_t kResRed = (size_t)kCgResReplicas * (16 * 256 + 32 * 256);
     size_t res_exch() const { return 16 * nLocal; }
 
-    template <int NN, int K>
-    int resident_launch(KrylovWork &wk, bool precond, int most, bool &taken, hipStream_t s)
+    // Nodes a thread of the resident form, 0 where the problem does not fit it:
+    // as few as the device has workgroups for, one only on up to 7/8 of the CUs
+    // (64x64, N = 7: 7.8 us an iteration on 256 workgroups, 7.1 on 128 with two;
+    // 56x56 on 196: 6.3 against 6.4 on 98).  Its workgroups in `blocks`.
+    template <int NN>
+    int resident_nodes(int &blocks)
     {
         constexpr int epb = kCgResThreads / ((NN + 1) * (NN + 1));
-        const void *f = reinterpret_cast<const void *>(&k_cg_resident<NN, K>);
-        const int blocks = (int)((nE + (size_t)epb * K - 1) / ((size_t)epb * K));
+        int device = 0;
+        if (maxCopies > 4 || res_exch() >= (1u << 31) || hipGetDevice(&device) != hipSuccess) return 0;
+        const int cus = persist_cus(device);
+        const auto fits = [&](const void *f, int K, int most) {
+            blocks = (int)((nE + (size_t)epb * K - 1) / ((size_t)epb * K));
+            return persist_blocks_per_cu(f, kCgResThreads) >= 1 && blocks <= most;
+        };
+        if (fits(reinterpret_cast<const void *>(&k_cg_resident<NN, 1>), 1, 7 * cus / 8)) return 1;
+        if (fits(reinterpret_cast<const void *>(&k_cg_resident<NN, 2>), 2, cus)) return 2;
+        if (fits(reinterpret_cast<const void *>(&k_cg_resident<NN, 4>), 4, cus)) return 4;
+        return 0;
+    }
+
+    bool resident_shape() override
+    {
+        int K = 0, blocks = 0;
+        CG_DISPATCH_N(N, if constexpr (NN > 1) K = (resident_nodes<NN>(blocks)););
+        return K > 0;
+    }
+
+    template <int NN, int K>
+    int ordered_launch(const CgOrdArgs &A, int blocks, hipStream_t s)
+    {
+        hipLaunchKernelGGL((k_cg_ord_direction<NN, K>), dim3((unsigned)blocks), dim3(kCgResThreads), 0, s, A);
+        hipLaunchKernelGGL((k_cg_ord_update<NN, K>), dim3((unsigned)blocks), dim3(kCgResThreads), 0, s, A);
+        hipLaunchKernelGGL(k_cg_ord_end, dim3(1), dim3(256), 0, s, A, blocks);
+        SELF_HIP(hipGetLastError());
+        return SELF_OK;
+    }
+
+    int cg_iteration_ordered(KrylovWork &wk, bool precond, int it, hipStream_t s) override
+    {
+        CgOrdArgs A{};
+        A.gid = gid;
+        A.cs = cs;
+        A.ci = ci;
+        A.G3 = G3;
+        A.D = D;
+        A.dinv = precond ? dinv : nullptr;
+        A.r = wk.r;
+        A.u = wk.u;
+        A.vNew = (it & 1) ? wk.v : wk.vB;
+        A.vOld = (it & 1) ? wk.vB : wk.v;
+        A.L = Lbuf;
+        A.partials = wk.slot.partials;
+        A.st = wk.st;
+        A.nE = (int)nE;
+        A.it = it;
+        int rc = SELF_ERR_STATE;
+        CG_DISPATCH_N(N, if constexpr (NN > 1) {
+            int blocks = 0;
+            const int K = resident_nodes<NN>(blocks);
+            if (K == 1) rc = (ordered_launch<NN, 1>(A, blocks, s));
+            else if (K == 2) rc = (ordered_launch<NN, 2>(A, blocks, s));
+            else if (K == 4) rc = (ordered_launch<NN, 4>(A, blocks, s));
+        });
+        return rc;
+    }
+
+    template <int NN, int K>
+    int resident_launch(KrylovWork &wk, bool precond, int blocks, bool &taken, hipStream_t s)
+    {
         int device = 0;
         SELF_HIP(hipGetDevice(&device));
-        if (persist_blocks_per_cu(f, kCgResThreads) < 1 || blocks > most * persist_cus(device) / 8) return SELF_OK;
         if (!resBuf) {
             resBytes = res_exch() + kResRed + sizeof(CgResOut) + 64;
-            if (dev(&resBuf, resBytes) != SELF_OK) {  // no memory for it: the two-launch form needs none
+            if (dev(&resBuf, resBytes) != SELF_OK) {  // no memory for it: the launched iterations need none
                 (void)hipGetLastError();
                 resOff = true;
                 return SELF_OK;
@@ -596,15 +659,14 @@ struct CgsemOp final : DevOp {
     int resident_cg(KrylovWork &wk, bool precond, bool &taken, hipStream_t s) override
     {
         taken = false;
-        if (resOff || maxCopies > 4 || res_exch() >= (1u << 31) || !resUps.tries()) return SELF_OK;
+        if (resOff || !resUps.tries()) return SELF_OK;
         int rc = SELF_OK;
-        // As few nodes a thread as the device has workgroups for; one a thread
-        // only on up to 7/8 of the CUs (64x64, N = 7: 7.8 us an iteration on 256
-        // workgroups, 7.1 on 128 with two; 56x56 on 196: 6.3 against 6.4 on 98).
         CG_DISPATCH_N(N, if constexpr (NN > 1) {
-            rc = (resident_launch<NN, 1>(wk, precond, 7, taken, s));
-            if (!rc && !taken) rc = (resident_launch<NN, 2>(wk, precond, 8, taken, s));
-            if (!rc && !taken) rc = (resident_launch<NN, 4>(wk, precond, 8, taken, s));
+            int blocks = 0;
+            const int K = resident_nodes<NN>(blocks);
+            if (K == 1) rc = (resident_launch<NN, 1>(wk, precond, blocks, taken, s));
+            else if (K == 2) rc = (resident_launch<NN, 2>(wk, precond, blocks, taken, s));
+            else if (K == 4) rc = (resident_launch<NN, 4>(wk, precond, blocks, taken, s));
         });
         return rc;
     }
@@ -1403,17 +1465,24 @@ try {
             taken[p] = t;
         }
         for (int p = 0; p < nProblems; ++p) {
-            if (!taken[p]) continue;
+            CgsemOp &op = hs[p]->op;
+            KrylovWork &wk = hs[p]->wk;
             bool done = false;
-            if (int rc = krylov_cg_resident_end(hs[p]->op, hs[p]->wk, done, hs[p]->op.stream)) return rc;
-            if (done) {
-                KrylovResult res;
-                if (int rc = krylov_cg_finish(hs[p]->op, hs[p]->wk, kStopNormRel, tol, hs[p]->op.xg, res, hs[p]->op.stream))
-                    return rc;
-                ioerr[p] = res.ioerr;
-                iterations[p] = res.iterations;
-                solved[p] = 1;
+            if (taken[p])
+                if (int rc = krylov_cg_resident_end(op, wk, done, op.stream)) return rc;
+            if (!done) {
+                if (!op.resident_shape()) continue;
+                // as its single solve would: the launches with the resident form's bits
+                int rc = taken[p] ? krylov_cg_begin(op, wk, precond == 1, kStopNormRel, tol, maxIters, op.xg, op.stream)
+                                  : SELF_OK;
+                if (!rc) rc = krylov_cg_ordered(op, wk, precond == 1, maxIters, op.stream);
+                if (rc) return rc;
             }
+            KrylovResult res;
+            if (int rc = krylov_cg_finish(op, wk, kStopNormRel, tol, op.xg, res, op.stream)) return rc;
+            ioerr[p] = res.ioerr;
+            iterations[p] = res.iterations;
+            solved[p] = 1;
         }
         for (int p = 0; p < nProblems; ++p)
             if (solved[p]) SELF_HIP(hipStreamSynchronize(hs[p]->op.stream));

@@ -562,6 +562,19 @@ int krylov_cg_resident_end(DevOp &op, KrylovWork &wk, bool &done, hipStream_t s)
     return SELF_OK;
 }
 
+int krylov_cg_ordered(DevOp &op, KrylovWork &wk, bool precond, int maxIters, hipStream_t s)
+{
+    for (int it0 = 1; it0 <= maxIters; it0 += kChunk) {
+        const int it1 = std::min(it0 + kChunk - 1, maxIters);
+        for (int it = it0; it <= it1; ++it)
+            if (int rc = op.cg_iteration_ordered(wk, precond, it, s)) return rc;
+        SolverState h{};
+        if (int rc = read_state(wk, h, s)) return rc;
+        if (h.done) break;
+    }
+    return SELF_OK;
+}
+
 int krylov_cg_finish(DevOp &op, KrylovWork &wk, int stopRule, double tol, double *sol, KrylovResult &res,
                      hipStream_t s)
 {
@@ -595,6 +608,10 @@ int run_cg(DevOp &op, KrylovWork &wk, bool precond, int stopRule, double tol, in
         if ((rc = krylov_cg_resident_end(op, wk, done, s))) return rc;
         if (done) return krylov_cg_finish(op, wk, stopRule, tol, sol, res, s);
         if ((rc = krylov_cg_begin(op, wk, precond, stopRule, tol, maxIters, sol, s))) return rc;
+    }
+    if (op.resident_shape()) {
+        if ((rc = krylov_cg_ordered(op, wk, precond, maxIters, s))) return rc;
+        return krylov_cg_finish(op, wk, stopRule, tol, sol, res, s);
     }
     const double *dinv = precond ? op.inv_diag() : nullptr;
     for (int it0 = 1; it0 <= maxIters; it0 += kChunk) {

@@ -201,7 +201,13 @@ struct DevOp {
     // the operator has one and the problem fits it (resident_cg launches it and
     // sets taken).  resident_cg_end, with the state read after it, says whether
     // the launch gave up (its input is untouched) and otherwise leaves the
-    // solution in wk.u.
+    // solution in wk.u.  A problem that fits (resident_shape) and is not or not
+    // to the end solved so takes cg_iteration_ordered, which has its bits.
+    virtual bool resident_shape() { return false; }
+    virtual int cg_iteration_ordered(KrylovWork &wk, bool precond, int it, hipStream_t s)
+    {
+        return SELF_ERR_STATE;
+    }
     virtual int resident_cg(KrylovWork &wk, bool precond, bool &taken, hipStream_t s)
     {
         taken = false;
@@ -287,6 +293,8 @@ int krylov_cg_finish(DevOp &op, KrylovWork &wk, int stopRule, double tol, double
 // launch of DevOp::resident_cg (waits for it); done is false where it gave up
 // and the solve has to begin again.
 int krylov_cg_resident_end(DevOp &op, KrylovWork &wk, bool &done, hipStream_t s);
+// All iterations of a solve begun by krylov_cg_begin by DevOp::cg_iteration_ordered.
+int krylov_cg_ordered(DevOp &op, KrylovWork &wk, bool precond, int maxIters, hipStream_t s);
 
 // Mixed precision: FP32 PCG inner solves, FP64 residual and iterative
 // refinement to |b - A x| / |b - A x0| <= tol.

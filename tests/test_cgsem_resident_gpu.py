@@ -1,14 +1,16 @@
-"""The CGSEM CG as one launch per solve against its two launches an iteration
-(which a launch whose first unsuccessful poll gives up falls back to): every
-degree, one, two and four nodes a thread, ragged last workgroups, curved
-elements, prescribed boundary values, no preconditioner, a start at the
-solution, and sizes past the device's (which stay with the launches).
+"""The CGSEM CG as one launch per solve against the launched iterations that a
+launch whose first unsuccessful poll gives up falls back to: every degree, one,
+two and four nodes a thread, ragged last workgroups, curved elements,
+prescribed boundary values, no preconditioner, a start at the solution, and
+sizes past the device's (which stay with the launches of large problems).
 
-After a fixed number of iterations the two differ by the rounding of their
-sums only: 12 iterations amplify 1e-16 by far less than 1e4 on these
-well-scaled problems, so 1e-12 relative.  Converged solutions to a relative
-residual of 1e-11 differ by at most that times the condition number (< 1e4
-here after the diagonal's scaling): 1e-7."""
+The two sum in one order and are bitwise equal (the bounds of the first two
+tests are those of any order: 12 iterations amplify 1e-16 by far less than 1e4
+on these well-scaled problems, so 1e-12 relative; solutions to a relative
+residual of 1e-11 differ by at most that times the condition number, < 1e4 here
+after the diagonal's scaling: 1e-7).  The operator is checked against another
+kernel's: the recursion's residual is that of the solution (Residual), up to
+the rounding of 12 iterations."""
 import numpy as np
 import pytest
 
@@ -62,6 +64,7 @@ def test_one_launch_follows_the_launched_iterations(gpu_lib, N, nX, nY, monkeypa
         assert ia == ib == 12
         assert rel_l2(a, b) < 1e-12
         assert np.allclose(ra[:13], rb[:13], rtol=1e-10, atol=0)
+        assert abs(np.linalg.norm(m.Residual()) - rb[12]) < 1e-12 * rb[0]
     m.Trash()
 
 
@@ -92,3 +95,35 @@ def test_nothing_to_solve(gpu_lib):
     u, it, _, _ = _solve(m, "jacobi", 1e-10, 50)
     assert it == 0 and not u.any()
     m.Trash()
+
+
+@pytest.mark.parametrize("N,nX,nY", [s for s in SHAPES if s[1] * s[2] * (s[0] + 1) ** 2 <= 1 << 20])
+def test_a_solve_that_gave_up_has_the_same_bits(gpu_lib, N, nX, nY, monkeypatch):
+    """A result must not depend on what else the device does: the launched
+    iterations of a problem of a resident shape sum in the resident order."""
+    m = _model(N, nX, nY, warp=0.03 if nX < 40 else 0.0, boundary=True)
+    for precond, tol, iters in (("jacobi", 1e-300, 40), ("none", 1e-300, 9), ("jacobi", 0.3, 200)):
+        a, ia, ioa, ra = _solve(m, precond, tol, iters)
+        monkeypatch.setenv("SELF_AMD_SPIN_LIMIT", "0")
+        b, ib, iob, rb = _solve(m, precond, tol, iters)
+        monkeypatch.delenv("SELF_AMD_SPIN_LIMIT")
+        assert (ia, ioa) == (ib, iob) and np.array_equal(a, b) and np.array_equal(ra, rb)
+    m.Trash()
+
+
+def test_a_batch_that_gave_up_has_the_single_solves_bits(gpu_lib, monkeypatch):
+    from self_amd.krylov import SolveBatched
+    shapes = [(7, 33, 31), (3, 21, 13), (5, 30, 17), (7, 80, 61), (2, 23, 19)]
+    ms = [_model(*s, boundary=True) for s in shapes]
+    want = [_solve(m, "jacobi", 1e-9, 5000)[:2] for m in ms]
+    for limit in ("2000", "0"):
+        monkeypatch.setenv("SELF_AMD_SPIN_LIMIT", limit)
+        for m in ms:
+            m.SetSolution(np.zeros_like(m.mesh.x))
+        _, its, _ = SolveBatched(ms, precond="jacobi", tolerance=1e-9, maxIters=5000)
+        for m, i, (u, it) in zip(ms, its, want):
+            assert i == it and np.array_equal(m.GetSolution(), u)
+    monkeypatch.delenv("SELF_AMD_SPIN_LIMIT")
+    assert [m.ResidentCounts()[1] for m in ms] == [1] * len(ms)
+    for m in ms:
+        m.Trash()
