@@ -475,10 +475,11 @@ int self_hexmesh_structured(int nX, int nY, int nZ, int N, int periodicX, int pe
 
 /* ---------------------------------------------------------- autotuning
  * The process-wide table of tuned launch configurations, keyed by model
- * kind ("sw2d", "sw2d_ensemble"), dimension, degree N, arithmetic (0 FP64,
- * 1 mixed) and size class floor(log2(elements)); entries hold four
- * configuration integers and the time per step that chose them.  No
- * reference counterpart. */
+ * kind ("sw2d", "sw2d_ensemble"; for models that do not fit the device, which
+ * launch every stage, "sw2d_launched", "sw2d_ensemble_launched"), dimension,
+ * degree N, arithmetic (0 FP64, 1 mixed) and size class
+ * floor(log2(elements)); entries hold four configuration integers and the
+ * time per step that chose them.  No reference counterpart. */
 int self_tune_count(int *n);
 /* entry index: kind (NUL-terminated, kindLen bytes), key4 = dim, N, dtype,
  * sizeClass; cfg4; ms per step */

@@ -1600,11 +1600,11 @@ int launch_steps(self_sw2d_s *h, int nSteps, bool &taken)
     return gate.launched();
 }
 
-int steps_prepare(self_sw2d_s *h)
+int steps_prepare(self_sw2d_s *h, bool &ok)
 {
     int rc = SELF_OK, perCu = 0;
     size_t blocks = 0;
-    bool ok = false;
+    ok = false;
     if (h->d.form != SELF_FUSED) return SELF_OK;
     if (h->d.precision == SELF_MIXED) {
         SELF_DISPATCH_N(h->d.N, (rc = steps_ready<NN, true>(h, ok, perCu, blocks)));
@@ -1897,7 +1897,8 @@ try {
     SELF_HIP(hipMemcpy(h->edges, edges, sizeof(int) * 6 * nEd, hipMemcpyHostToDevice));
     h->geomSet = true;
     h->trValid = false;
-    return h->useGraph ? steps_prepare(h) : SELF_OK;
+    bool ok = false;
+    return h->useGraph ? steps_prepare(h, ok) : SELF_OK;
 }
 SELF_CATCH_ALL
 
@@ -2487,13 +2488,20 @@ try {
         *groups = 1;
         return SELF_OK;
     }
-    // the table holds the choice for this degree, arithmetic and size
-    // class once any model of that key has been tuned
-    const char *kind = h->members > 1 ? "sw2d_ensemble" : "sw2d";
+    // The table holds the choice for this degree, arithmetic and size class once
+    // any model of that key has been tuned.  A size class holds models that fit
+    // the device and such that do not: groups = 1 with the graph on are resident
+    // steps for the first, stage launches for the second, and neither's choice or
+    // time is the other's.  Entries of the first kind carry a 1 in their third
+    // integer: those of files written before there were resident steps do not.
+    bool fits = false;
+    if ((rc = steps_prepare(h, fits))) return rc;
+    const char *kind = h->members > 1 ? (fits ? "sw2d_ensemble" : "sw2d_ensemble_launched")
+                                      : (fits ? "sw2d" : "sw2d_launched");
     const int dtype = h->d.precision == SELF_MIXED ? 1 : 0, sc = tune_size_class(h->nE * (size_t)h->members);
     int cfg[4];
     double known = 0.0;
-    if (tune_lookup(kind, 2, h->d.N, dtype, sc, cfg, &known)) {
+    if (tune_lookup(kind, 2, h->d.N, dtype, sc, cfg, &known) && (!fits || cfg[2] == 1)) {
         h->groups = cfg[0];
         h->useGraph = cfg[1] != 0;
         *groups = cfg[0];
@@ -2552,7 +2560,7 @@ try {
     h->useGraph = bestGraph != 0;
     *groups = bestG;
     if (ms_per_step) *ms_per_step = best / nSteps;
-    const int chosen[4] = {bestG, bestGraph, 0, 0};
+    const int chosen[4] = {bestG, bestGraph, fits ? 1 : 0, 0};
     tune_record(kind, 2, h->d.N, dtype, sc, chosen, best / nSteps);
     return SELF_OK;
 }

@@ -177,3 +177,30 @@ def test_tags_come_round_after_a_launch_gave_up(gpu_lib, monkeypatch):
     assert np.isfinite(want).all() and np.array_equal(a.GetSolution(), want)
     a.Trash()
     b.Trash()
+
+
+def test_tuning_keeps_resident_and_launched_models_apart(gpu_lib, tmp_path):
+    """64x64 elements at N = 7 fit the device, 65x64 of the same size class do
+    not: neither takes the other's choice, nor one written before there were
+    resident steps."""
+    from self_amd import shallow_water as SW
+    SW.clear_tuning_table()
+    big, fit = _model(N=7, nX=65, nY=64, precision="fp64"), _model(N=7, nX=64, nY=64, precision="fp64")
+    big.Autotune(4)
+    assert [t["kind"] for t in SW.tuning_table()] == ["sw2d_launched"]
+    fit.Autotune(4)
+    assert sorted(t["kind"] for t in SW.tuning_table()) == ["sw2d", "sw2d_launched"]
+    n = fit.ResidentCounts()[0]
+    assert n >= 2  # a trial's
+    fit.Autotune(4)  # from the table
+    assert fit.ResidentCounts() == (n, 0)
+    path = tmp_path / "t.txt"
+    path.write_text("sw2d 2 7 0 12 2 0 0 0 0.05\n")
+    SW.load_tuning_table(str(path))
+    fit.Autotune(4)
+    assert fit.ResidentCounts()[0] > n
+    kept = {t["kind"]: t["config"] for t in SW.tuning_table()}
+    assert kept["sw2d"][:3] == [1, 1, 1]
+    SW.clear_tuning_table()
+    big.Trash()
+    fit.Trash()
