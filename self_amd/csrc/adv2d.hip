@@ -1033,7 +1033,7 @@ try {
 SELF_CATCH_ALL
 
 int self_adv2d_global_time_derivative(self_adv2d_t h, double t)
-{
+try {
     SELF_REQUIRE(h, SELF_ERR_ARG, "null handle");
     SELF_HIP(hipSetDevice(h->device));
     int rc = settle(h);
@@ -1042,6 +1042,7 @@ int self_adv2d_global_time_derivative(self_adv2d_t h, double t)
     h->trValid = true;
     return stage(h, t, -1, 1);
 }
+SELF_CATCH_ALL
 
 int self_adv2d_forward_step_rk3(self_adv2d_t h, double tn, int nSteps, double *elapsed_ms)
 try {
@@ -1132,10 +1133,11 @@ try {
 SELF_CATCH_ALL
 
 int self_adv2d_synchronize(self_adv2d_t h)
-{
+try {
     SELF_REQUIRE(h, SELF_ERR_ARG, "null handle");
     SELF_HIP(hipStreamSynchronize(h->stream));
     return settle(h);
 }
+SELF_CATCH_ALL
 
 }  // extern "C"

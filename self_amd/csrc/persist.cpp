@@ -109,9 +109,11 @@ int ResidentRuns::settle(hipStream_t s, std::vector<Run> &again)
 // Where every launch takes a CU a workgroup, each needs only as many CUs as it
 // has.  Launches on one stream run one after another and count once.
 PersistGate::PersistGate(int device, hipStream_t stream, int blocks, int perCu)
-    : rc(SELF_OK), device_(device), stream_(stream), demand_((double)blocks / perCu), share_(1.0 / perCu)
+    : rc(SELF_OK), lock_(g_mutex), device_(device), stream_(stream), demand_((double)blocks / perCu), share_(1.0 / perCu)
 {
-    g_mutex.lock();
+    // room for this launch's records: nothing may throw once it is queued
+    g_flights.reserve(g_flights.size() + 1);
+    g_events.reserve(g_events.size() + g_flights.size() + 1);
     prune();
     std::map<hipStream_t, double> per;
     double largest = share_;
@@ -134,8 +136,6 @@ PersistGate::PersistGate(int device, hipStream_t stream, int blocks, int perCu)
         if (e != hipSuccess && rc == SELF_OK) rc = hip_fail(e, "hipStreamWaitEvent", __FILE__, __LINE__);
     }
 }
-
-PersistGate::~PersistGate() { g_mutex.unlock(); }
 
 int PersistGate::launched()
 {

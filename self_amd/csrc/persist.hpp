@@ -30,6 +30,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <vector>
 
 #include "common.hpp"
@@ -213,11 +214,11 @@ struct ResidentRuns {
 class PersistGate {
 public:
     PersistGate(int device, hipStream_t stream, int blocks, int perCu);
-    ~PersistGate();
     int rc;
     int launched();
 
 private:
+    std::lock_guard<std::mutex> lock_;
     int device_;
     hipStream_t stream_;
     double demand_, share_;

@@ -1996,7 +1996,7 @@ try {
 SELF_CATCH_ALL
 
 int self_sw2d_set_params(self_sw2d_t h, double g, double dt, double linearDrag)
-{
+try {
     SELF_REQUIRE(h, SELF_ERR_ARG, "null handle");
     if (int rs = settle(h)) return rs;
     h->d.g = g;
@@ -2010,40 +2010,45 @@ int self_sw2d_set_params(self_sw2d_t h, double g, double dt, double linearDrag)
     }
     return SELF_OK;
 }
+SELF_CATCH_ALL
 
 int self_sw2d_calculate_solution_at_boundaries(self_sw2d_t h)
-{
+try {
     int rc = check_ready(h);
     if (rc) return rc;
     return launch_traces(h, h->q, h->bsol, 3);
 }
+SELF_CATCH_ALL
 
 int self_sw2d_edge_flux(self_sw2d_t h, double t)
-{
+try {
     (void)t;  // no time-dependent boundary state in this model
     int rc = check_ready(h);
     if (rc) return rc;
     return launch_edge_flux(h);
 }
+SELF_CATCH_ALL
 
 int self_sw2d_mapped_time_derivative(self_sw2d_t h, double t)
-{
+try {
     (void)t;
     int rc = check_ready(h);
     if (rc) return rc;
     return launch_mapped(h);
 }
+SELF_CATCH_ALL
 
 int self_sw2d_global_time_derivative(self_sw2d_t h, double t)
-{
+try {
     (void)t;
     int rc = check_ready(h);
     if (rc) return rc;
     return gtd_plain(h);
 }
+SELF_CATCH_ALL
 
 int self_sw2d_check_mixed(self_sw2d_t h, double tol, double *relErr, int *switched)
-{
+try {
     int rc = check_ready(h);
     if (rc) return rc;
     SELF_REQUIRE(relErr && switched, SELF_ERR_ARG, "null argument");
@@ -2113,9 +2118,10 @@ int self_sw2d_check_mixed(self_sw2d_t h, double tol, double *relErr, int *switch
     }
     return SELF_OK;
 }
+SELF_CATCH_ALL
 
 int self_sw2d_forward_step_rk3(self_sw2d_t h, double tn, int nSteps)
-{
+try {
     (void)tn;
     int rc = check_ready(h, false);
     if (rc) return rc;
@@ -2143,9 +2149,10 @@ int self_sw2d_forward_step_rk3(self_sw2d_t h, double tn, int nSteps)
     for (; s < nSteps && !rc; ++s) rc = (h->d.form == SELF_FUSED) ? step_fused(h) : step_plain(h);
     return rc;
 }
+SELF_CATCH_ALL
 
 int self_sw2d_forward_step_rk3_timed(self_sw2d_t h, double tn, int nSteps, double *elapsed_ms)
-{
+try {
     int rc = check_ready(h);
     if (rc) return rc;
     SELF_REQUIRE(elapsed_ms, SELF_ERR_ARG, "null elapsed_ms");
@@ -2169,6 +2176,7 @@ int self_sw2d_forward_step_rk3_timed(self_sw2d_t h, double tn, int nSteps, doubl
         *elapsed_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     return rc;
 }
+SELF_CATCH_ALL
 
 int self_sw2d_kernel_times(self_sw2d_t h, double tn, int nSteps, double *avg_ms, int *nKernels)
 try {
@@ -2236,7 +2244,7 @@ try {
 SELF_CATCH_ALL
 
 int self_sw2d_calculate_bathymetry_gradient(self_sw2d_t h)
-{
+try {
     int rc = check_ready(h);
     if (rc) return rc;
     SWKernelArgs A = make_args(h);
@@ -2245,6 +2253,7 @@ int self_sw2d_calculate_bathymetry_gradient(self_sw2d_t h)
     SELF_HIP(hipGetLastError());
     return SELF_OK;
 }
+SELF_CATCH_ALL
 
 int self_sw2d_set_members(self_sw2d_t h, int members)
 try {
@@ -2367,13 +2376,14 @@ try {
 SELF_CATCH_ALL
 
 int self_sw2d_set_variant(self_sw2d_t h, int variant)
-{
+try {
     SELF_REQUIRE(h, SELF_ERR_ARG, "null handle");
     SELF_REQUIRE(variant == 0 || variant == 1, SELF_ERR_ARG, "unknown shallow-water variant %d", variant);
     if (int rs = settle(h)) return rs;
     h->variant = variant;
     return SELF_OK;
 }
+SELF_CATCH_ALL
 
 // ForwardStepRK3 nSteps times for several fused-form models at once, of
 // any degrees, one persistent launch per RK stage for all of them
@@ -2567,11 +2577,12 @@ try {
 SELF_CATCH_ALL
 
 int self_sw2d_synchronize(self_sw2d_t h)
-{
+try {
     SELF_REQUIRE(h, SELF_ERR_ARG, "null handle");
     SELF_HIP(hipStreamSynchronize(h->stream));
     return settle(h);
 }
+SELF_CATCH_ALL
 
 int self_sw2d_resident_counts(self_sw2d_t h, int *launches, int *gaveUp)
 try {

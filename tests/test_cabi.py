@@ -132,3 +132,15 @@ def test_tuning_table_file_round_trip_on_the_host(tmp_path):
     with pytest.raises(L.SelfError):
         SW.load_tuning_table(str(bad))
     SW.clear_tuning_table()
+
+
+def test_no_exception_leaves_an_entry_that_settles_launches():
+    """Settling launches in flight fills host vectors: every entry point that
+    does it (or calls one that does) catches what they throw."""
+    import re
+    for name in ("sw2d.hip", "adv2d.hip"):
+        src = open(os.path.join(ROOT, "self_amd", "csrc", name)).read()
+        bare = re.findall(r"^int (self_\w+)\([^)]*\)\n\{\n(.*?)^\}\n", src, re.S | re.M)
+        assert bare
+        for fn, body in bare:
+            assert not re.search(r"\b(settle|check_ready|steps_prepare)\(|std::vector", body), f"{name}: {fn}"
