@@ -327,12 +327,18 @@ hipError_t pc_graph(FemPC &pc, const PcBuffers<T> &B, const SolverState *outer, 
     return e;
 }
 
-// The two launches an iteration cost the host 6.2 us each, more than the
-// kernels take up to some 10^5 unknowns.
 // 45x33, N = 5, 60 applications of 50 iterations: 37.4 ms launched one by one,
-// 28.6 as graphs (32.2 with 512 workgroups instead of pc_grid's).
-// Where no graph can be had (memory, a stream that is being captured) the
-// launches are issued one by one.
+// 28.6 as graphs (32.2 with 512 workgroups instead of pc_grid's).  The host
+// issues a launch in 2.6 us (20 000 iterations that return at once: 106 ms, 82 as
+// a graph), less than the kernels take: it is the gap between dependent
+// launches that a graph shortens.
+// Building one takes as long as two to three applications' launches (2.2 ms at
+// 500 iterations), so the first application is launched one by one and the
+// second builds it.  Above kPcGraphIterations (35 MB of host memory a graph), where
+// no graph can be had and on a stream that is being captured the launches are
+// issued one by one too.
+constexpr int kPcGraphIterations = 8192;
+
 template <typename T>
 int pc_apply(FemPC &pc, const T *b, T *x, const PcBuffers<T> &B, const SolverState *outer, hipStream_t s)
 {
@@ -341,13 +347,13 @@ int pc_apply(FemPC &pc, const T *b, T *x, const PcBuffers<T> &B, const SolverSta
     FemPC::Graph &G = pc.graph[sizeof(T) == 4][outer != nullptr];
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     SELF_HIP(hipStreamIsCapturing(s, &cap));
-    const bool useGraph = pc.maxIters > 0 && cap == hipStreamCaptureStatusNone;
+    const bool useGraph = pc.maxIters > 0 && pc.maxIters <= kPcGraphIterations && cap == hipStreamCaptureStatusNone;
     if (useGraph && G.exec && G.outer != outer) {  // another solver's state
         SELF_HIP(hipStreamSynchronize(s));
         SELF_HIP(hipGraphExecDestroy(G.exec));
         G.exec = nullptr;
     }
-    if (useGraph && !G.exec && !G.failed) {
+    if (useGraph && !G.exec && !G.failed && G.applied) {
         const hipError_t e = pc_graph<T>(pc, B, outer, &G.exec);
         G.outer = outer;
         if (e != hipSuccess) {
@@ -356,6 +362,7 @@ int pc_apply(FemPC &pc, const T *b, T *x, const PcBuffers<T> &B, const SolverSta
             G.failed = true;
         }
     }
+    G.applied = true;
     hipLaunchKernelGGL(k_pc_start<T>, g, t, 0, s, b, B.r, B.u, n, pc.partials, (const PcState *)pc.st, outer);
     hipLaunchKernelGGL(k_pc_final_start, dim3(1), t, 0, s, (const double *)pc.partials, (int)g.x, pc.st, outer,
                        pc.maxIters, pc.tol);

@@ -17,7 +17,7 @@
 // launch's partials itself, in one fixed order, so all hold the same bits);
 // every kernel returns at once when the inner CG has converged or the outer
 // solver is done, so the host issues pcIterates iterations without reading
-// anything back: as one graph launch, built by the first application over
+// anything back: as one graph launch, built by the second application over
 // the solver's own buffers (the right-hand side comes in by the start kernel,
 // the result leaves by the finish kernel).
 #pragma once
@@ -55,7 +55,7 @@ struct FemPC {
     struct Graph {
         hipGraphExec_t exec = nullptr;
         const SolverState *outer = nullptr;
-        bool failed = false;
+        bool applied = false, failed = false;
     } graph[2][2];
     double *partials = nullptr;  // [2][kPcParts]: product step (v.z), update (r.r)
     PcState *st = nullptr;

@@ -53,3 +53,16 @@ def test_replays_equal_a_fresh_application_and_the_oracle(gpu_lib, N, nX, nY, it
     assert n == its + 2 and np.array_equal(x, h.ApplyPreconditioner(b)[0])
     g.Trash()
     h.Trash()
+
+
+def test_iterations_past_the_graph_s_bound(gpu_lib):
+    """8192 iterations are a graph, 8193 launches: the same bits, early end and all."""
+    g, h = _model(3, 9, 8), _model(3, 9, 8)
+    g.SetPreconditioner(pcIterates=8192, pcTolerance=0.2)
+    h.SetPreconditioner(pcIterates=8193, pcTolerance=0.2)
+    b = np.sin(5 * g.mesh.x) * (1 + g.mesh.y)
+    for _ in range(3):
+        (x, n), (y, m) = g.ApplyPreconditioner(b), h.ApplyPreconditioner(b)
+        assert 0 < n == m < 400 and np.array_equal(x, y)
+    g.Trash()
+    h.Trash()
