@@ -1,12 +1,15 @@
 // layout.hpp -- device fields [field][element][node] to the host's
-// [element][field][node] arrays.
+// [element][field][node] arrays, and plain arrays either way.
 //
-// The reordering runs on the device, through a bounded staging buffer kept by
-// the model, and each piece is copied straight into the caller's array.  A
-// host vector of the whole field, filled by the copy and reordered by memcpy,
-// costs three passes over fresh host pages: 44 ms for the 124 MB of a 24x21x12,
-// N = 7 hydrostatic state against 13 ms.  It is the way where the device has no
-// memory left for the buffer: reading a field must not fail for that.
+// Pieces travel through two halves of a pinned buffer kept by the model: while
+// one piece is on its way, the piece before is put in the caller's order, which
+// the copy out of the buffer does at no cost.  A copy from or to pageable memory
+// has the runtime pin or stage the caller's pages on each call, the slower the
+// fresher they are.  Measured, us, fresh pages (a hipMemcpy into a vector and a
+// memcpy; a reordering kernel and a copy into the caller's array; this): 6 KB of
+// three fields 12.8, 24.5, 12.2; 0.8 MB 415, 463, 114; 12.6 MB 1430, 954, 728;
+// 50 MB 15250, 4470, 3900.  Where no pinned memory is to be had, the vector
+// serves.
 #pragma once
 
 #include <algorithm>
@@ -18,81 +21,109 @@
 
 namespace self {
 
-// Most of the staging buffer: 32 MB.  SELF_AMD_STAGE_DOUBLES overrides it (a
-// test of the way without one sets 0, of several pieces a small number).
+// Most of one half: 4 MB (1 MB 5 to 10 % slower from 10 MB on, 512 KB 40 %).
+// SELF_AMD_STAGE_DOUBLES overrides it (a test of the way without the buffer
+// sets 0, of several pieces a small number).
 inline size_t stage_doubles()
 {
     const char *s = std::getenv("SELF_AMD_STAGE_DOUBLES");
     if (s && *s) return (size_t)std::strtoull(s, nullptr, 10);
-    return (size_t)4 << 20;
+    return (size_t)1 << 19;
 }
 
 struct HostStage {
     double *buf = nullptr;
-    size_t cap = 0;  // doubles
+    size_t cap = 0;                            // doubles
+    hipEvent_t done[2] = {nullptr, nullptr};   // the last copy of each half
     HostStage() = default;
     HostStage(const HostStage &) = delete;
     HostStage &operator=(const HostStage &) = delete;
-    ~HostStage() { release(); }
-    void release()
+    ~HostStage()
     {
-        if (buf) (void)hipFree(buf);
-        buf = nullptr;
-        cap = 0;
+        if (buf) (void)hipHostFree(buf);
+        for (hipEvent_t e : done)
+            if (e) (void)hipEventDestroy(e);
     }
-    // room for n values, if the device has it
+    // room for n values, if there is pinned memory for it
     bool reserve(size_t n)
     {
-        if (n <= cap) return true;
-        release();
-        if (hipMalloc(reinterpret_cast<void **>(&buf), sizeof(double) * n) != hipSuccess) {
-            (void)hipGetLastError();
+        hipError_t e = hipSuccess;
+        for (hipEvent_t &v : done)
+            if (!v && e == hipSuccess) e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
+        if (e == hipSuccess && n > cap) {
+            if (buf) (void)hipHostFree(buf);
             buf = nullptr;
-            return false;
+            cap = 0;
+            e = hipHostMalloc(reinterpret_cast<void **>(&buf), sizeof(double) * n, hipHostMallocDefault);
+            if (e == hipSuccess) cap = n;
+            else buf = nullptr;
         }
-        cap = n;
-        return true;
+        if (e != hipSuccess) (void)hipGetLastError();
+        return e == hipSuccess;
     }
 };
-
-// element-first copy of elements e0 .. e0 + n - 1; a thread per value
-template <typename T>
-__global__ __launch_bounds__(256) void k_elements_first(const T *__restrict__ src, T *__restrict__ dst, size_t nE,
-                                                        int nf, int np, size_t e0, size_t n)
-{
-    const size_t row = (size_t)nf * np, total = n * row;
-    for (size_t k = (size_t)blockIdx.x * 256 + threadIdx.x; k < total; k += (size_t)gridDim.x * 256) {
-        const size_t e = k / row, w = k - e * row, f = w / np, nd = w - f * np;
-        dst[k] = src[(f * nE + e0 + e) * np + nd];
-    }
-}
 
 // Work queued on s before the call is waited for; the copy is complete on return.
 inline int fields_to_host(const double *dev, double *host, size_t nE, int nf, int np, HostStage &st, hipStream_t s)
 {
-    const size_t row = (size_t)nf * np;
-    if (nf == 1) {  // the same layout
-        SELF_HIP(hipMemcpyAsync(host, dev, sizeof(double) * nE * row, hipMemcpyDeviceToHost, s));
-        SELF_HIP(hipStreamSynchronize(s));
-        return SELF_OK;
-    }
-    const size_t most = stage_doubles(), piece = std::min(nE, std::max<size_t>(1, most / row));
-    if (most == 0 || !st.reserve(piece * row)) {
+    const size_t row = (size_t)nf * np, most = stage_doubles();
+    const size_t piece = std::min(nE, std::max<size_t>(1, most / row)), n = piece ? (nE + piece - 1) / piece : 0;
+    const auto order = [&](const double *src, size_t e0, size_t m) {  // src: [field][m][node]
+        if (nf == 1) {
+            std::memcpy(host + e0 * row, src, sizeof(double) * m * row);
+            return;
+        }
+        for (size_t e = 0; e < m; ++e)
+            for (size_t f = 0; f < (size_t)nf; ++f)
+                std::memcpy(host + ((e0 + e) * nf + f) * np, src + (f * m + e) * np, sizeof(double) * np);
+    };
+    if (most == 0 || !st.reserve(std::min<size_t>(n, 2) * piece * row)) {
         std::vector<double> buf(nE * row);
         SELF_HIP(hipMemcpyAsync(buf.data(), dev, sizeof(double) * buf.size(), hipMemcpyDeviceToHost, s));
         SELF_HIP(hipStreamSynchronize(s));
-        for (size_t e = 0; e < nE; ++e)
-            for (size_t f = 0; f < (size_t)nf; ++f)
-                std::memcpy(host + (e * nf + f) * np, buf.data() + (f * nE + e) * np, sizeof(double) * np);
+        order(buf.data(), 0, nE);
         return SELF_OK;
     }
-    for (size_t e0 = 0; e0 < nE; e0 += piece) {
-        const size_t n = std::min(piece, nE - e0);
-        const unsigned grid = (unsigned)std::min<size_t>((n * row + 255) / 256, 4096);
-        hipLaunchKernelGGL(k_elements_first<double>, dim3(grid), dim3(256), 0, s, dev, st.buf, nE, nf, np, e0, n);
-        SELF_HIP(hipGetLastError());
-        SELF_HIP(hipMemcpyAsync(host + e0 * row, st.buf, sizeof(double) * n * row, hipMemcpyDeviceToHost, s));
+    const auto fetch = [&](size_t p) -> hipError_t {
+        const size_t e0 = p * piece, m = std::min(piece, nE - e0);
+        double *b = st.buf + (p & 1) * piece * row;
+        hipError_t e = hipSuccess;
+        if (m == nE)  // the whole field array
+            e = hipMemcpyAsync(b, dev, sizeof(double) * nE * row, hipMemcpyDeviceToHost, s);
+        else
+            for (size_t f = 0; f < (size_t)nf && e == hipSuccess; ++f)
+                e = hipMemcpyAsync(b + f * m * np, dev + (f * nE + e0) * np, sizeof(double) * m * np,
+                                   hipMemcpyDeviceToHost, s);
+        return e == hipSuccess && n > 1 ? hipEventRecord(st.done[p & 1], s) : e;
+    };
+    if (n > 0) SELF_HIP(fetch(0));
+    for (size_t p = 0; p < n; ++p) {
+        if (p + 1 < n) SELF_HIP(fetch(p + 1));
+        if (n > 1) SELF_HIP(hipEventSynchronize(st.done[p & 1]));
+        else SELF_HIP(hipStreamSynchronize(s));  // 7 us less than an event and a wait for it
+        order(st.buf + (p & 1) * piece * row, p * piece, std::min(piece, nE - p * piece));
+    }
+    return SELF_OK;
+}
+
+// n values to the device, after the work queued on s; the caller waits for s
+// before the stage is used again.
+inline int array_to_device(const double *host, double *dev, size_t n, HostStage &st, hipStream_t s)
+{
+    const size_t piece = std::min(n, stage_doubles());
+    if (piece == 0 || !st.reserve(piece < n ? 2 * piece : piece)) {
+        SELF_HIP(hipMemcpyAsync(dev, host, sizeof(double) * n, hipMemcpyHostToDevice, s));
         SELF_HIP(hipStreamSynchronize(s));
+        return SELF_OK;
+    }
+    size_t p = 0;
+    for (size_t k = 0; k < n; k += piece, ++p) {
+        const size_t m = std::min(piece, n - k);
+        double *b = st.buf + (p & 1) * piece;
+        if (p >= 2) SELF_HIP(hipEventSynchronize(st.done[p & 1]));
+        std::memcpy(b, host + k, sizeof(double) * m);
+        SELF_HIP(hipMemcpyAsync(dev + k, b, sizeof(double) * m, hipMemcpyHostToDevice, s));
+        if (n > piece) SELF_HIP(hipEventRecord(st.done[p & 1], s));
     }
     return SELF_OK;
 }

@@ -183,9 +183,9 @@ bool sw_groupable(const self_request &r)
 size_t estimate_bytes(const self_request &r)
 {
     const size_t n1 = r.N + 1, nE = (size_t)r.nX * r.nX, nodes = nE * n1 * n1;
-    // q, G, tend, bathy(3), plv, relax(4), metrics(5), the result's staging (3), traces, normals
+    // q, G, tend, bathy(3), plv, relax(4), metrics(5), traces, normals
     if (r.kind == SELF_REQ_SW2D)
-        return (size_t)(1.25 * (double)(nodes * 8 * 27 + nE * 4 * n1 * 8 * 18)) + (1u << 20);
+        return (size_t)(1.25 * (double)(nodes * 8 * 24 + nE * 4 * n1 * 8 * 18)) + (1u << 20);
     // CGSEM: local and global vectors, geometry, Krylov work vectors, messages of the one-launch solve (2)
     return (size_t)(1.25 * (double)(nodes * 8 * 24)) + (1u << 20);
 }

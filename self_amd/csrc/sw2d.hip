@@ -2597,7 +2597,7 @@ SELF_CATCH_ALL
 int self_sw2d_device_bytes(self_sw2d_t h, size_t *bytes)
 {
     SELF_REQUIRE(h && bytes, SELF_ERR_ARG, "null argument");
-    *bytes = h->bytes + sizeof(double) * h->stage.cap;
+    *bytes = h->bytes;
     return SELF_OK;
 }
 

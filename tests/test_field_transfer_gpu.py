@@ -1,6 +1,6 @@
 """Fields to the host in one piece, in several with a ragged last one, and
-without device memory for a staging buffer: the same bytes.  What a model
-allocates is counted, and a request's reservation covers its model."""
+without a pinned buffer: the same bytes, and no device memory for it.  A
+request's reservation covers its model."""
 import ctypes as C
 
 import numpy as np
@@ -42,15 +42,31 @@ def test_every_way_gives_the_same_bytes(gpu_lib, make, monkeypatch):
     assert np.array_equal(m.GetSolution(), want)
 
 
-def test_device_bytes_count_the_staging_buffer(gpu_lib, monkeypatch):
+def test_reading_a_field_takes_no_device_memory(gpu_lib):
     m = _sw2d()
     before = m.DeviceBytes()
-    monkeypatch.setenv("SELF_AMD_STAGE_DOUBLES", "0")
-    n = m.GetSolution().nbytes
-    assert m.DeviceBytes() == before
-    monkeypatch.delenv("SELF_AMD_STAGE_DOUBLES")
     m.GetSolution()
-    assert m.DeviceBytes() == before + n
+    assert m.DeviceBytes() == before
+
+
+def test_an_array_of_nodes_goes_there_and_back(gpu_lib, monkeypatch):
+    from test_cgsem_resident_gpu import _model as cgsem_model
+    m = cgsem_model(5, 9, 7, boundary=True)
+    rng = np.random.default_rng(3)
+    for most in (None, "0", "1", "700"):
+        if most is not None:
+            monkeypatch.setenv("SELF_AMD_STAGE_DOUBLES", most)
+        u = rng.standard_normal(m.mesh.x.shape)
+        m.SetSolution(u)
+        got = m.GetSolution()
+        monkeypatch.setenv("SELF_AMD_STAGE_DOUBLES", "0")
+        assert np.array_equal(m.GetSolution(), got)
+        monkeypatch.delenv("SELF_AMD_STAGE_DOUBLES")
+        inner = u[:, 1:-1, 1:-1]  # nodes of one element each
+        assert np.array_equal(got[:, 1:-1, 1:-1], inner)
+        m.SetSolution(got)  # copies of a shared node agree now, so this changes nothing
+        assert np.array_equal(m.GetSolution(), got)
+    m.Trash()
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
