@@ -655,7 +655,6 @@ struct self_adv2d_s {
     size_t nE = 0;
     double kappa = 0.0, dt = 0.0;
     hipStream_t stream = nullptr;
-    HostStage stage;
     double *nodal = nullptr, *c = nullptr, *G = nullptr, *tend = nullptr, *grad = nullptr, *vel = nullptr;
     double *velTr = nullptr, *fvel = nullptr, *metric = nullptr, *fnrm = nullptr, *tr[2] = {nullptr, nullptr};
     double *trG = nullptr, *relax = nullptr, *rFac = nullptr;
@@ -1028,7 +1027,7 @@ try {
         std::memset(data, 0, sizeof(double) * nq * nE * np);
         return SELF_OK;
     }
-    return fields_to_host(src, data, nE, (int)nq, (int)np, h->stage, h->stream);
+    return fields_to_host(src, data, nE, (int)nq, (int)np, h->stream);
 }
 SELF_CATCH_ALL
 

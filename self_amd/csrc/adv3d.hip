@@ -704,7 +704,6 @@ struct self_adv3d_s {
     size_t nE = 0, nSlots = 0;
     double dt = 0.0;
     hipStream_t stream = nullptr;
-    HostStage stage;
     double *nodal = nullptr, *c = nullptr, *G = nullptr, *tend = nullptr, *vel = nullptr, *geo = nullptr;
     double *fdat = nullptr, *nrm = nullptr, *bpos = nullptr, *tr[2] = {nullptr, nullptr}, *velTr = nullptr;
     double *relax = nullptr, *rFac = nullptr, *E1 = nullptr, *E2 = nullptr, *lim = nullptr;
@@ -1026,7 +1025,7 @@ try {
         SELF_HIP(hipMemcpy(data + 2 * nq * nE, h->lim, sizeof(double) * 3 * nq * nE, hipMemcpyDeviceToHost));
         return SELF_OK;
     }
-    return fields_to_host(field == 0 ? h->c : h->tend, data, nE, (int)nq, (int)np, h->stage, h->stream);
+    return fields_to_host(field == 0 ? h->c : h->tend, data, nE, (int)nq, (int)np, h->stream);
 }
 SELF_CATCH_ALL
 

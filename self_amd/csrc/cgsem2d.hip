@@ -848,7 +848,6 @@ struct self_cgsem2d_s {
     KrylovWork wk;
     int device = 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    HostStage stage;
     std::vector<double> resi;
 };
 
@@ -1262,7 +1261,7 @@ try {
     SELF_HIP(hipSetDevice(h->device));
     CgsemOp &op = h->op;
     // the element work array holds the host's values meanwhile
-    if (int rc = array_to_device(u, op.Lbuf, op.nLocal, h->stage, op.stream)) return rc;
+    if (int rc = array_to_device(u, op.Lbuf, op.nLocal, op.stream)) return rc;
     hipLaunchKernelGGL(k_cg_owners, dim3((unsigned)((op.nG + 255) / 256)), dim3(256), 0, op.stream,
                        (const double *)op.Lbuf, op.cs, op.ci, op.nG, op.xg);
     SELF_HIP(hipGetLastError());
@@ -1281,7 +1280,7 @@ try {
     hipLaunchKernelGGL(k_cg_unmask, dim3((unsigned)((op.nLocal + 255) / 256)), dim3(256), 0, op.stream,
                        (const double *)op.xg, op.gid, (const double *)op.uD, op.nLocal, op.Lbuf);
     SELF_HIP(hipGetLastError());
-    return fields_to_host(op.Lbuf, u, op.nLocal, 1, 1, h->stage, op.stream);
+    return fields_to_host(op.Lbuf, u, op.nLocal, 1, 1, op.stream);
 }
 SELF_CATCH_ALL
 

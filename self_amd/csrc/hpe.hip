@@ -64,7 +64,6 @@ struct self_hpe_s {
     size_t nE = 0, nH = 0, nL = 0;
     double dt = 0.0;
     hipStream_t stream = nullptr;
-    self::HostStage stage;
     double *nodal = nullptr, *sol = nullptr, *G = nullptr, *tend = nullptr, *geo = nullptr, *height = nullptr;
     double *nrm = nullptr, *fdat = nullptr, *tr = nullptr, *Bvol = nullptr, *divU = nullptr;
     int2 *side = nullptr;
@@ -1109,7 +1108,7 @@ try {
     }
     const int nf = field == 0 ? 5 : field == 1 ? 3 : 1;
     const double *src = field == 0 ? h->sol : field == 1 ? h->tend : h->divU;
-    return fields_to_host(src, data, nE, nf, (int)np, h->stage, h->stream);
+    return fields_to_host(src, data, nE, nf, (int)np, h->stream);
 }
 SELF_CATCH_ALL
 

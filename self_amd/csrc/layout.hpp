@@ -1,7 +1,7 @@
 // layout.hpp -- device fields [field][element][node] to the host's
 // [element][field][node] arrays, and plain arrays either way.
 //
-// Pieces travel through two halves of a pinned buffer kept by the model: while
+// Pieces travel through two halves of a pinned buffer: while
 // one piece is on its way, the piece before is put in the caller's order, which
 // the copy out of the buffer does at no cost.  A copy from or to pageable memory
 // has the runtime pin or stage the caller's pages on each call, the slower the
@@ -13,7 +13,6 @@
 #pragma once
 
 #include <algorithm>
-#include <cstdlib>
 #include <cstring>
 #include <vector>
 
@@ -24,47 +23,38 @@ namespace self {
 // Most of one half: 4 MB (1 MB 5 to 10 % slower from 10 MB on, 512 KB 40 %).
 // SELF_AMD_STAGE_DOUBLES overrides it (a test of the way without the buffer
 // sets 0, of several pieces a small number).
-inline size_t stage_doubles()
-{
-    const char *s = std::getenv("SELF_AMD_STAGE_DOUBLES");
-    if (s && *s) return (size_t)std::strtoull(s, nullptr, 10);
-    return (size_t)1 << 19;
-}
+size_t stage_doubles();
 
-struct HostStage {
-    double *buf = nullptr;
-    size_t cap = 0;                            // doubles
-    hipEvent_t done[2] = {nullptr, nullptr};   // the last copy of each half
-    HostStage() = default;
-    HostStage(const HostStage &) = delete;
-    HostStage &operator=(const HostStage &) = delete;
-    ~HostStage()
-    {
-        if (buf) (void)hipHostFree(buf);
-        for (hipEvent_t e : done)
-            if (e) (void)hipEventDestroy(e);
-    }
-    // room for n values, if there is pinned memory for it
-    bool reserve(size_t n)
-    {
-        hipError_t e = hipSuccess;
-        for (hipEvent_t &v : done)
-            if (!v && e == hipSuccess) e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
-        if (e == hipSuccess && n > cap) {
-            if (buf) (void)hipHostFree(buf);
-            buf = nullptr;
-            cap = 0;
-            e = hipHostMalloc(reinterpret_cast<void **>(&buf), sizeof(double) * n, hipHostMallocDefault);
-            if (e == hipSuccess) cap = n;
-            else buf = nullptr;
-        }
-        if (e != hipSuccess) (void)hipGetLastError();
-        return e == hipSuccess;
-    }
+// A pinned buffer for one transfer, from a small process-wide pool: a new one
+// costs 0.3 ms a MB on its first use.  Any thread, any stream of the current
+// device; a lease that ends before the transfer was seen to be over (an error
+// on the way) waits for the stream.
+struct StageBuffer {
+    double *p = nullptr;
+    size_t cap = 0;                           // doubles
+    int device = -1;
+    hipEvent_t done[2] = {nullptr, nullptr};  // the last copy of each half
+};
+
+class StageLease {
+public:
+    StageLease(size_t n, hipStream_t s);  // room for n values
+    ~StageLease();
+    StageLease(const StageLease &) = delete;
+    StageLease &operator=(const StageLease &) = delete;
+    bool ok() const { return b_.p != nullptr; }  // false: no pinned memory to be had
+    double *half(size_t p, size_t n) const { return b_.p + (p & 1) * n; }
+    hipEvent_t done(size_t p) const { return b_.done[p & 1]; }
+    void over() { over_ = true; }
+
+private:
+    StageBuffer b_;
+    hipStream_t s_;
+    bool over_ = false;
 };
 
 // Work queued on s before the call is waited for; the copy is complete on return.
-inline int fields_to_host(const double *dev, double *host, size_t nE, int nf, int np, HostStage &st, hipStream_t s)
+inline int fields_to_host(const double *dev, double *host, size_t nE, int nf, int np, hipStream_t s)
 {
     const size_t row = (size_t)nf * np, most = stage_doubles();
     const size_t piece = std::min(nE, std::max<size_t>(1, most / row)), n = piece ? (nE + piece - 1) / piece : 0;
@@ -77,7 +67,8 @@ inline int fields_to_host(const double *dev, double *host, size_t nE, int nf, in
             for (size_t f = 0; f < (size_t)nf; ++f)
                 std::memcpy(host + ((e0 + e) * nf + f) * np, src + (f * m + e) * np, sizeof(double) * np);
     };
-    if (most == 0 || !st.reserve(std::min<size_t>(n, 2) * piece * row)) {
+    StageLease st(most ? std::min<size_t>(n, 2) * piece * row : 0, s);
+    if (!st.ok()) {
         std::vector<double> buf(nE * row);
         SELF_HIP(hipMemcpyAsync(buf.data(), dev, sizeof(double) * buf.size(), hipMemcpyDeviceToHost, s));
         SELF_HIP(hipStreamSynchronize(s));
@@ -86,7 +77,7 @@ inline int fields_to_host(const double *dev, double *host, size_t nE, int nf, in
     }
     const auto fetch = [&](size_t p) -> hipError_t {
         const size_t e0 = p * piece, m = std::min(piece, nE - e0);
-        double *b = st.buf + (p & 1) * piece * row;
+        double *b = st.half(p, piece * row);
         hipError_t e = hipSuccess;
         if (m == nE)  // the whole field array
             e = hipMemcpyAsync(b, dev, sizeof(double) * nE * row, hipMemcpyDeviceToHost, s);
@@ -94,24 +85,25 @@ inline int fields_to_host(const double *dev, double *host, size_t nE, int nf, in
             for (size_t f = 0; f < (size_t)nf && e == hipSuccess; ++f)
                 e = hipMemcpyAsync(b + f * m * np, dev + (f * nE + e0) * np, sizeof(double) * m * np,
                                    hipMemcpyDeviceToHost, s);
-        return e == hipSuccess && n > 1 ? hipEventRecord(st.done[p & 1], s) : e;
+        return e == hipSuccess && n > 1 ? hipEventRecord(st.done(p), s) : e;
     };
     if (n > 0) SELF_HIP(fetch(0));
     for (size_t p = 0; p < n; ++p) {
         if (p + 1 < n) SELF_HIP(fetch(p + 1));
-        if (n > 1) SELF_HIP(hipEventSynchronize(st.done[p & 1]));
+        if (n > 1) SELF_HIP(hipEventSynchronize(st.done(p)));
         else SELF_HIP(hipStreamSynchronize(s));  // 7 us less than an event and a wait for it
-        order(st.buf + (p & 1) * piece * row, p * piece, std::min(piece, nE - p * piece));
+        order(st.half(p, piece * row), p * piece, std::min(piece, nE - p * piece));
     }
+    st.over();
     return SELF_OK;
 }
 
-// n values to the device, after the work queued on s; the caller waits for s
-// before the stage is used again.
-inline int array_to_device(const double *host, double *dev, size_t n, HostStage &st, hipStream_t s)
+// n values to the device, after the work queued on s; the copy is complete on return.
+inline int array_to_device(const double *host, double *dev, size_t n, hipStream_t s)
 {
     const size_t piece = std::min(n, stage_doubles());
-    if (piece == 0 || !st.reserve(piece < n ? 2 * piece : piece)) {
+    StageLease st(piece < n ? 2 * piece : piece, s);
+    if (!st.ok()) {
         SELF_HIP(hipMemcpyAsync(dev, host, sizeof(double) * n, hipMemcpyHostToDevice, s));
         SELF_HIP(hipStreamSynchronize(s));
         return SELF_OK;
@@ -119,12 +111,14 @@ inline int array_to_device(const double *host, double *dev, size_t n, HostStage 
     size_t p = 0;
     for (size_t k = 0; k < n; k += piece, ++p) {
         const size_t m = std::min(piece, n - k);
-        double *b = st.buf + (p & 1) * piece;
-        if (p >= 2) SELF_HIP(hipEventSynchronize(st.done[p & 1]));
+        double *b = st.half(p, piece);
+        if (p >= 2) SELF_HIP(hipEventSynchronize(st.done(p)));
         std::memcpy(b, host + k, sizeof(double) * m);
         SELF_HIP(hipMemcpyAsync(dev + k, b, sizeof(double) * m, hipMemcpyHostToDevice, s));
-        if (n > piece) SELF_HIP(hipEventRecord(st.done[p & 1], s));
+        if (n > piece) SELF_HIP(hipEventRecord(st.done(p), s));
     }
+    SELF_HIP(hipStreamSynchronize(s));
+    st.over();
     return SELF_OK;
 }
 

@@ -1234,7 +1234,6 @@ struct self_sw2d_s {
     self_sw2d_desc d{};
     int device = 0;
     hipStream_t stream = nullptr;
-    HostStage stage;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int n1 = 0, np = 0;
     size_t nE = 0;
@@ -1969,7 +1968,7 @@ try {
     SELF_HIP(hipStreamSynchronize(h->stream));
     const size_t nE = h->nE, np = h->np, n1 = h->n1;
     auto get_nodal = [&](const double *dev, int nf) -> int {
-        return fields_to_host(dev, data, nE, nf, (int)np, h->stage, h->stream);
+        return fields_to_host(dev, data, nE, nf, (int)np, h->stream);
     };
     switch (field) {
     case SELF_SW_SOLUTION: return get_nodal(h->q, 3);
@@ -2342,7 +2341,7 @@ try {
     SELF_HIP(hipSetDevice(h->device));
     SELF_HIP(hipStreamSynchronize(h->stream));
     const size_t nE = h->nE, np = h->np;
-    return fields_to_host(h->q + (size_t)member * 3 * nE * np, data, nE, 3, (int)np, h->stage, h->stream);
+    return fields_to_host(h->q + (size_t)member * 3 * nE * np, data, nE, 3, (int)np, h->stream);
 }
 SELF_CATCH_ALL
 
