@@ -780,7 +780,8 @@ int resident_prepare(self_adv2d_s *h)
     h->runs.messageBytes = 3 * sizeof(ll_quad) * ll_quads(h);
     if (hipMalloc(reinterpret_cast<void **>(&h->cAlt), sizeof(double) * h->nq * h->nE * h->np) != hipSuccess ||
         hipMalloc(reinterpret_cast<void **>(&h->runs.messages), h->runs.messageBytes) != hipSuccess ||
-        hipMalloc(reinterpret_cast<void **>(&h->runs.status), sizeof(int)) != hipSuccess) {
+        hipMalloc(reinterpret_cast<void **>(&h->runs.status), sizeof(int)) != hipSuccess ||
+        h->runs.alloc_host() != hipSuccess) {
         (void)hipGetLastError();
         if (h->cAlt) (void)hipFree(h->cAlt);
         if (h->runs.messages) (void)hipFree(h->runs.messages);
@@ -896,6 +897,7 @@ try {
                      h->tr[0], h->tr[1], h->trG, h->relax, h->rFac, h->side, h->pnode, h->cAlt, h->runs.messages, h->runs.status};
         for (void *q : p)
             if (q) (void)hipFree(q);
+        h->runs.free_host();
         if (h->stream) (void)hipStreamDestroy(h->stream);
         delete h;
         return hip_fail(e, "self_adv2d_create", __FILE__, __LINE__);
@@ -957,6 +959,7 @@ int self_adv2d_destroy(self_adv2d_t h)
                  h->tr[0], h->tr[1], h->trG, h->relax, h->rFac, h->side, h->pnode, h->cAlt, h->runs.messages, h->runs.status};
     for (void *q : p)
         if (q) (void)hipFree(q);
+    h->runs.free_host();
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
     return SELF_OK;

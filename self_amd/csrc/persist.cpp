@@ -75,17 +75,31 @@ int ResidentRuns::clear(hipStream_t s)
 {
     SELF_HIP(hipMemsetAsync(messages, 0, messageBytes, s));
     SELF_HIP(hipMemsetAsync(status, 0, sizeof(int), s));
+    *hostStatus = 0;
     tag = 0;
     return SELF_OK;
+}
+
+hipError_t ResidentRuns::alloc_host()
+{
+    if (hostStatus) return hipSuccess;
+    const hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&hostStatus), sizeof(int), hipHostMallocDefault);
+    if (e != hipSuccess) hostStatus = nullptr;
+    return e;
+}
+
+void ResidentRuns::free_host()
+{
+    if (hostStatus) (void)hipHostFree(hostStatus);
+    hostStatus = nullptr;
 }
 
 int ResidentRuns::settle(hipStream_t s, std::vector<Run> &again)
 {
     again.clear();
     if (pending.empty()) return SELF_OK;
-    int bad = 0;
-    SELF_HIP(hipMemcpyAsync(&bad, status, sizeof(int), hipMemcpyDeviceToHost, s));
     SELF_HIP(hipStreamSynchronize(s));
+    const int bad = *static_cast<volatile int *>(hostStatus);
     std::vector<Run> done;
     done.swap(pending);
     if (bad == 0) {

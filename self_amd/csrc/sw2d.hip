@@ -898,8 +898,8 @@ __global__ __launch_bounds__(256, 4 / G) void k_sw_stage_fused(SWKernelArgs A0)
 // vector instructions of all of them: 64x64, N = 7 takes 4.9 us a stage FP64
 // (stage kernel 10.1) and 4.5 mixed (10.1); 16x16, N = 3 2.1 (4.4); 70x70,
 // N = 6 5.7 (11.8).  A call starts with 10 to 16 us for loads and first traces,
-// so from two steps on it is the faster form (64x64, two steps: 44 against 60
-// us; 16x16, N = 3: 22 against 26).  Every value is formed by the stage
+// so from two steps on it is the faster form (two steps and the wait for them:
+// 64x64, N = 7 49 us against 85, 12x12, N = 3 27 against 40).  Every value is formed by the stage
 // kernel's expressions in its order: results are bitwise the same.
 struct SWStepsArgs {
     PersistArgs P;
@@ -1289,6 +1289,7 @@ void free_all(self_sw2d_s *h)
     if (h->qAlt) (void)hipFree(h->qAlt);
     if (h->runs.messages) (void)hipFree(h->runs.messages);
     if (h->runs.status) (void)hipFree(h->runs.status);
+    h->runs.free_host();
 }
 
 // fills A member by member (callers that compare argument blocks bytewise
@@ -1555,7 +1556,7 @@ int steps_ready(self_sw2d_s *h, bool &ok, int &perCu, size_t &blocks)
     const size_t nq = 3 * (size_t)h->members * h->nE * h->np;
     h->runs.messageBytes = 2 * sizeof(ll_quad) * ll_quads(h);
     if (dalloc(h, &h->qAlt, nq) != SELF_OK || dalloc(h, &h->runs.messages, 2 * ll_quads(h)) != SELF_OK ||
-        (!h->runs.status && dalloc(h, &h->runs.status, 1) != SELF_OK)) {
+        (!h->runs.status && dalloc(h, &h->runs.status, 1) != SELF_OK) || h->runs.alloc_host() != hipSuccess) {
         (void)hipGetLastError();  // no memory for it: the ordinary launches need none
         persist_free(h);
         h->runs.off = true;
@@ -2126,7 +2127,11 @@ try {
     if (rc) return rc;
     SELF_REQUIRE(nSteps >= 0, SELF_ERR_ARG, "negative step count");
     int s = 0;
-    if (h->d.form == SELF_FUSED && h->useGraph && !h->runs.off && nSteps >= 2 &&
+    // From two steps on, three where a workgroup holds 64 elements of N = 1 and most
+    // of the device's room is taken (65536 of them, calls of two steps: 100 us a call
+    // by launches, 110 resident; 32041: 65 and 49).
+    const int least = h->d.N == 1 && h->nE * (size_t)h->members > 32768 ? 3 : 2;
+    if (h->d.form == SELF_FUSED && h->useGraph && !h->runs.off && nSteps >= least &&
         fused_groups(h->groups, h->nE, 0) == 1 && h->runs.ups.tries()) {
         bool taken = true;
         while (s < nSteps && taken) {
