@@ -249,6 +249,7 @@ struct KrylovWork {
     double *V = nullptr, *Z = nullptr;  // GMRES bases (n x (m+1))
     double *small = nullptr;            // GMRES small matrices
     SolverState *st = nullptr;          // device
+    SolverState *stHost = nullptr;      // pinned, where the host reads it
     double *resi = nullptr;             // device residual history
     int resiLen = 0;
     RedSlot slot{};
