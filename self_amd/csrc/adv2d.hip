@@ -406,8 +406,13 @@ struct AdvStepsArgs {
     unsigned bytesC;        // of llC; llG has twice as many
 };
 
+// Workgroups a CU decide up to which size a model is resident: where two registers
+// stand between three and two of them, three are asked for.
 template <int N, int NQ>
-__global__ __launch_bounds__(256) void k_adv_steps(AdvArgs A, AdvStepsArgs T)
+constexpr int kAdvWaves = NQ == 1 && (N == 1 || N == 8) ? 3 : 1;
+
+template <int N, int NQ>
+__global__ __launch_bounds__(256, (kAdvWaves<N, NQ>)) void k_adv_steps(AdvArgs A, AdvStepsArgs T)
 {
     using S = Shape<N>;
     constexpr int n1 = S::n1, np = S::np, epb = S::epb, ns4 = 4 * n1, kSide = (ns4 + np - 1) / np;
@@ -416,7 +421,12 @@ __global__ __launch_bounds__(256) void k_adv_steps(AdvArgs A, AdvStepsArgs T)
     __shared__ double cs[epb * NQ * np], sx[epb * NQ * np], sy[epb * NQ * np], px[epb * NQ * np],
         py[epb * NQ * np], bf[epb * 4 * 2 * NQ * n1];
     __shared__ int stop;
-    if (threadIdx.x == 0) stop = persist_given_up(T.P);
+    // where the gradient goes is read when it is needed: no registers hold it meanwhile
+    __shared__ double *volatile grads[1];
+    if (threadIdx.x == 0) {
+        stop = persist_given_up(T.P);
+        grads[0] = A.grad;
+    }
     stage_nodal<N, false>(L, A.nodal, nullptr, nullptr);
     __syncthreads();
     if (stop) return;  // an earlier launch of this model gave up: leave the state to the host
@@ -550,14 +560,12 @@ __global__ __launch_bounds__(256) void k_adv_steps(AdvArgs A, AdvStepsArgs T)
                            bfE[((2 * 2 + 1) * NQ + f) * n1 + i], bfE[((0 * 2 + 1) * NQ + f) * n1 + i], y1[f], y2[f]);
                 gx[f] = (x1[f] + x2[f]) / J;
                 gy[f] = (y1[f] + y2[f]) / J;
-                // every lane is past its contractions: the flux arrays take the gradient and the volume flux
+                // Every lane is past its contractions: the arrays of the gradient's
+                // flux take the gradient (sx for its traces, py and sy until the next
+                // stage) and then the volume flux (sx, px).
                 sx[lo + f * np + nd] = gx[f];
+                py[lo + f * np + nd] = gx[f];
                 sy[lo + f * np + nd] = gy[f];
-                // the model's gradient is the last stage's, as the launched stages leave it
-                if (st + 1 == T.nStages) {
-                    A.grad[f * mstride + base] = gx[f];
-                    A.grad[(NQ + f) * mstride + base] = gy[f];
-                }
             }
         }
         sync();
@@ -640,8 +648,14 @@ __global__ __launch_bounds__(256) void k_adv_steps(AdvArgs A, AdvStepsArgs T)
         if (st + 1 < T.nStages) send_c(tag + 1);
     }
     if (act) {
+        // the model's gradient is the last stage's, as the launched stages leave it
+        double *grad = *grads;
         #pragma unroll
-        for (int f = 0; f < NQ; ++f) T.cOut[f * mstride + base] = c[f];
+        for (int f = 0; f < NQ; ++f) {
+            T.cOut[f * mstride + base] = c[f];
+            grad[f * mstride + base] = py[lo + f * np + nd];
+            grad[(NQ + f) * mstride + base] = sy[lo + f * np + nd];
+        }
     }
 }
 
@@ -780,7 +794,7 @@ int resident_prepare(self_adv2d_s *h)
     h->runs.messageBytes = 3 * sizeof(ll_quad) * ll_quads(h);
     if (hipMalloc(reinterpret_cast<void **>(&h->cAlt), sizeof(double) * h->nq * h->nE * h->np) != hipSuccess ||
         hipMalloc(reinterpret_cast<void **>(&h->runs.messages), h->runs.messageBytes) != hipSuccess ||
-        hipMalloc(reinterpret_cast<void **>(&h->runs.status), sizeof(int)) != hipSuccess ||
+        hipMalloc(reinterpret_cast<void **>(&h->runs.status), sizeof(PersistStatus)) != hipSuccess ||
         h->runs.alloc_host() != hipSuccess) {
         (void)hipGetLastError();
         if (h->cAlt) (void)hipFree(h->cAlt);
