@@ -258,6 +258,23 @@ __device__ __forceinline__ void trace3(const NodalLDS<N> &L, const double *qs, i
     }
 }
 
+// Node of lane tl.  At N = 3 and 7 the products are formed transposed: a result's
+// column, the fast lane index, is the node's first index, so that lanes next to
+// each other load nodes next to each other, 4 or 8 of them (N + 1 apart the other
+// way: a launched stage of 130x130, N = 3 mixed 13.1 against 12.4 us, a resident
+// one of 64x64, N = 7 mixed 4.4 against 4.3; the 3-D kernels and the conjugate
+// gradients, whose node values go through LDS or stay, are 2 % faster that way).
+template <int N>
+__device__ __forceinline__ int sw_node(int tl)
+{
+    if constexpr (Mf<N>::on) {
+        const MfLane<N> m(tl);
+        return (4 * m.bi + m.c) + (N + 1) * (4 * m.bj + m.k);
+    } else {
+        return tl;
+    }
+}
+
 // first side node (side (N+1) + k) of lane tl, or -1.  At N = 7 the quarter's
 // bits select the direction (bj: across p) and the half of the side (bi).
 template <int N>
@@ -271,12 +288,13 @@ __device__ __forceinline__ int lane_side(int tl)
         const MfLane<N> m(tl);
         return (m.k == 0 ? 3 : m.k == 1 ? 1 : m.k == 2 ? 0 : 2) * 4 + m.c;
     } else {
-        return tl < 4 * (N + 1) ? tl : -1;
+        // up to N = 2 every node is one, and another follows
+        return N <= 2 || tl < 4 * (N + 1) ? tl : -1;
     }
 }
 
-// the lane's operator entries: weak derivative in s (left operand) and in p
-// (right operand, transposed), end-point interpolation rows
+// the lane's operator entries: weak derivative in s (right operand, transposed)
+// and in p (left operand), end-point interpolation rows
 template <int N>
 struct MfOps {
     double s[Mf<N>::K], p[Mf<N>::K], lag[2];
@@ -315,8 +333,8 @@ __device__ __forceinline__ void mf_volume(const MfOps<N> &M, const double *sC, c
     #pragma unroll
     for (int q = 0; q < Mf<N>::K; ++q) {
         const int m = 4 * q + a.k;
-        t1 = __builtin_amdgcn_mfma_f64_4x4x4f64(M.s[q], sC[m + n1 * (4 * a.bj + a.c)], t1, 0, 0, 0);
-        t2 = __builtin_amdgcn_mfma_f64_4x4x4f64(pC[(4 * a.bi + a.c) + n1 * m], M.p[q], t2, 0, 0, 0);
+        t1 = __builtin_amdgcn_mfma_f64_4x4x4f64(sC[m + n1 * (4 * a.bj + a.c)], M.s[q], t1, 0, 0, 0);
+        t2 = __builtin_amdgcn_mfma_f64_4x4x4f64(M.p[q], pC[(4 * a.bi + a.c) + n1 * m], t2, 0, 0, 0);
     }
 }
 
@@ -562,7 +580,7 @@ __device__ __forceinline__ void sw_load(const SWKernelArgs &A, int e, int nd, in
     const size_t mstride = (size_t)A.nE * np;
     const size_t base = act ? (size_t)e * np + nd : 0;
     const int ec = act ? e : 0;
-    const int ns = max(w0, 0);
+    const int ns = N <= 2 ? w0 : max(w0, 0);
     const int sd0 = ns / n1, k0 = ns - sd0 * n1;
     const size_t es = (size_t)ec * 4 + sd0;
     P.Jv = 1.0; P.hRaw = 1.0;
@@ -677,7 +695,7 @@ __device__ __forceinline__ void sw_process(const SWKernelArgs &A, const NodalLDS
     sw_finish<MIXED>(A, act, P);
     constexpr int n1 = N + 1, np = n1 * n1;
     constexpr bool MF = Mf<N>::on;
-    const int nd = lane_node<N>(tl), w0 = lane_side<N>(tl);
+    const int nd = sw_node<N>(tl), w0 = lane_side<N>(tl);
     const int i = nd % n1, j = nd / n1;
     const size_t mstride = (size_t)A.nE * np, base = (size_t)e * np + nd;
 
@@ -708,7 +726,7 @@ __device__ __forceinline__ void sw_process(const SWKernelArgs &A, const NodalLDS
             #pragma unroll
             for (int f = 0; f < 3; ++f) tm[f] = mf_trace<N>(M, qsE + f * np, tl);
         }
-        for (int w = w0; w >= 0 && w < 4 * n1; w += np) {
+        for (int w = w0; (N <= 2 || w >= 0) && w < 4 * n1; w += np) {
             const int sd = w / n1, k = w - sd * n1;
             int2 info;
             double fn[3], oth[3], fl[3];
@@ -776,7 +794,7 @@ __device__ __forceinline__ void sw_process(const SWKernelArgs &A, const NodalLDS
             #pragma unroll
             for (int f = 0; f < 3; ++f) tm[f] = mf_trace<N>(M, qsE + f * np, tl);
         }
-        for (int w = w0; w >= 0 && w < 4 * n1; w += np) {
+        for (int w = w0; (N <= 2 || w >= 0) && w < 4 * n1; w += np) {
             const int sd = w / n1, k = w - sd * n1;
             const int2 info = (w == w0) ? P.info0 : A.side[(size_t)e * 4 + sd];
             if (info.x < 0) continue;
@@ -854,7 +872,7 @@ __device__ __forceinline__ void sw_stage_group(const SWKernelArgs &A0, int wg, S
     for (int g = 0; g < G; ++g) {
         e[g] = (wg * G + g) * epb + le;
         act[g] = le < epb && e[g] < A.nE;
-        sw_load<N, MIXED>(A, e[g], lane_node<N>(tl), lane_side<N>(tl), act[g], P[g]);
+        sw_load<N, MIXED>(A, e[g], sw_node<N>(tl), lane_side<N>(tl), act[g], P[g]);
     }
     nodal_put<N, MIXED, kLanes>(L, R, lane);
     if constexpr (WL) wave_sync();
@@ -952,7 +970,7 @@ __global__ __launch_bounds__(256, 4) void k_sw_steps(SWKernelArgs A, SWStepsArgs
     const int e = wg * epb + le;
     const bool act = le < epb && e < A.nE;
     constexpr bool MF = Mf<N>::on;
-    const int nd = lane_node<N>(tl), w0 = lane_side<N>(tl);
+    const int nd = sw_node<N>(tl), w0 = lane_side<N>(tl);
     const int i = nd % n1, j = nd / n1;
     const size_t mstride = (size_t)A.nE * np, base = (size_t)e * np + nd;
     SWPre P;
