@@ -28,8 +28,9 @@
 // sum_k Dhat(i,k) = -(l_E(i) - l_W(i))/w_i) and FP32 storage of the RK
 // tendency register, bathymetry gradient and Coriolis parameter.  State,
 // traces, metrics, normals and the RK accumulation stay FP64.  At N = 3 and 7
-// its contractions run on the FP64 matrix cores like the FP64 form's: they
-// are faster there than in FP32 on the vector pipe, deviations included (64x64,
+// its contractions are FP64 like the FP64 form's, on the matrix cores but for
+// the launched stage at N = 3: they are no slower there than in FP32 on the vector
+// pipe, deviations included (64x64,
 // N = 7: 5.5 -> 4.5 us a stage in k_sw_steps, 11.7 -> 10.1 us in the stage
 // kernel).
 
@@ -258,16 +259,24 @@ __device__ __forceinline__ void trace3(const NodalLDS<N> &L, const double *qs, i
     }
 }
 
+// The launched stage has its contractions on the matrix cores at N = 7.  At N = 3 it
+// is bound by its loads, and those of four elements in the instruction's layout
+// cost more than the vector pipe's FP64 sums (130x130: 12.6 us a stage mixed and
+// 13.4 FP64 against 11.2 and 12.7); the sums are the same to the bit, so the
+// resident form, which loads once a call, keeps the matrix cores at both.
+template <int N>
+constexpr bool kMfStage = N == 7;
+
 // Node of lane tl.  At N = 3 and 7 the products are formed transposed: a result's
 // column, the fast lane index, is the node's first index, so that lanes next to
 // each other load nodes next to each other, 4 or 8 of them (N + 1 apart the other
-// way: a launched stage of 130x130, N = 3 mixed 13.1 against 12.4 us, a resident
-// one of 64x64, N = 7 mixed 4.4 against 4.3; the 3-D kernels and the conjugate
+// way: a launched stage of 66x66, N = 7 FP64 12.2 us against 11.7, a resident one
+// of 64x64, N = 7 mixed 4.4 against 4.3; the 3-D kernels and the conjugate
 // gradients, whose node values go through LDS or stay, are 2 % faster that way).
-template <int N>
+template <int N, bool MF = Mf<N>::on>
 __device__ __forceinline__ int sw_node(int tl)
 {
-    if constexpr (Mf<N>::on) {
+    if constexpr (MF) {
         const MfLane<N> m(tl);
         return (4 * m.bi + m.c) + (N + 1) * (4 * m.bj + m.k);
     } else {
@@ -277,19 +286,19 @@ __device__ __forceinline__ int sw_node(int tl)
 
 // first side node (side (N+1) + k) of lane tl, or -1.  At N = 7 the quarter's
 // bits select the direction (bj: across p) and the half of the side (bi).
-template <int N>
+template <int N, bool MF = Mf<N>::on>
 __device__ __forceinline__ int lane_side(int tl)
 {
-    if constexpr (N == 7) {
+    if constexpr (!MF) {
+        // up to N = 2 every node is one, and another follows
+        return N <= 2 || tl < 4 * (N + 1) ? tl : -1;
+    } else if constexpr (N == 7) {
         const MfLane<N> m(tl);
         if (m.k >= 2) return -1;
         return (m.bj ? (m.k ? 2 : 0) : (m.k ? 1 : 3)) * 8 + 4 * m.bi + m.c;
-    } else if constexpr (N == 3) {
+    } else {
         const MfLane<N> m(tl);
         return (m.k == 0 ? 3 : m.k == 1 ? 1 : m.k == 2 ? 0 : 2) * 4 + m.c;
-    } else {
-        // up to N = 2 every node is one, and another follows
-        return N <= 2 || tl < 4 * (N + 1) ? tl : -1;
     }
 }
 
@@ -694,8 +703,8 @@ __device__ __forceinline__ void sw_process(const SWKernelArgs &A, const NodalLDS
 {
     sw_finish<MIXED>(A, act, P);
     constexpr int n1 = N + 1, np = n1 * n1;
-    constexpr bool MF = Mf<N>::on;
-    const int nd = sw_node<N>(tl), w0 = lane_side<N>(tl);
+    constexpr bool MF = kMfStage<N>, DEV = MIXED && !Mf<N>::on;
+    const int nd = sw_node<N, MF>(tl), w0 = lane_side<N, MF>(tl);
     const int i = nd % n1, j = nd / n1;
     const size_t mstride = (size_t)A.nE * np, base = (size_t)e * np + nd;
 
@@ -711,7 +720,7 @@ __device__ __forceinline__ void sw_process(const SWKernelArgs &A, const NodalLDS
     if constexpr (MF) mf_load<N>(M, L, tl);  // the nodal constants are complete after the first synchronization
     // ---- phase B: FP32 deviations of the contravariant fluxes (mixed), and
     // the Rusanov flux of each side node in the edge's primary orientation
-    if constexpr (MIXED && !MF) {
+    if constexpr (DEV) {
         if (act) {
             #pragma unroll
             for (int f = 0; f < 3; ++f) {
@@ -764,7 +773,7 @@ __device__ __forceinline__ void sw_process(const SWKernelArgs &A, const NodalLDS
                 mf_volume<N>(M, sCE + f * np, pCE + f * np, tl, t1, t2);
                 tend[f] = dg_lift64_field<N>(L, bfE, i, j, P.invJ, f, t1, t2);
             }
-        } else if constexpr (MIXED) {
+        } else if constexpr (DEV) {
             dg_divergence_dev32<N>(L, sCE, pCE, sDE, pDE, bfE, i, j, P.invJ, tend);
         } else dg_divergence64<N, (N <= 5 || N % 2 == 1)>(L, sCE, pCE, bfE, i, j, P.invJ, tend);
         sw_source(P.s, P.vort, A.g, P.hx, P.hy, P.dragH, A.hasRelax, P.r, src);
@@ -860,7 +869,13 @@ __device__ __forceinline__ void sw_stage_group(const SWKernelArgs &A0, int wg, S
     }
     NodalLDS<N> &L = U.Lw[WL ? threadIdx.x / 64 : 0];
     int tl;
-    const int le = lane_element<N>(threadIdx.x, tl);
+    int le;
+    if constexpr (kMfStage<N> || !Mf<N>::on) {
+        le = lane_element<N>(threadIdx.x, tl);
+    } else {
+        le = threadIdx.x / np;
+        tl = threadIdx.x - le * np;
+    }
     constexpr int kLanes = WL ? 64 : 256;
     const int lane = WL ? threadIdx.x % 64 : threadIdx.x;
     NodalRegs<N, MIXED, kLanes> R;
@@ -872,7 +887,7 @@ __device__ __forceinline__ void sw_stage_group(const SWKernelArgs &A0, int wg, S
     for (int g = 0; g < G; ++g) {
         e[g] = (wg * G + g) * epb + le;
         act[g] = le < epb && e[g] < A.nE;
-        sw_load<N, MIXED>(A, e[g], sw_node<N>(tl), lane_side<N>(tl), act[g], P[g]);
+        sw_load<N, MIXED>(A, e[g], sw_node<N, kMfStage<N>>(tl), lane_side<N, kMfStage<N>>(tl), act[g], P[g]);
     }
     nodal_put<N, MIXED, kLanes>(L, R, lane);
     if constexpr (WL) wave_sync();
