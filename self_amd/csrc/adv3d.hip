@@ -413,8 +413,14 @@ __global__ __launch_bounds__(Shape3<N>::threads) void k_adv3d_prologue(Adv3Args 
 // 41.1 at 16x16x8 and two tracers, 11.2 -> 8.1 at 8x8x8.  Three workgroups of
 // 512 threads a CU (80 registers): two gave 194.7, three 172.0, and 158.7 with
 // the element and wavefront numbers in scalar registers; four spill (215.5).
+// Wavefronts a SIMD that are asked for: more than four where a few registers more
+// would leave fewer than there is LDS for (16x16x12, N = 4, one tracer: 17.9 us a
+// stage with five, 16.3 with six).
 template <int N, int NQ, int PREC>
-__global__ __launch_bounds__(Shape3<N>::threads, (N == 7 && NQ == 1 && PREC == 0) ? 6 : 4) void k_adv3d_stage(Adv3Args A)
+constexpr int kAdv3Waves = NQ == 1 && PREC == 0 && (N == 7 || N == 4 || N == 3) ? 6 : 4;
+
+template <int N, int NQ, int PREC>
+__global__ __launch_bounds__(Shape3<N>::threads, (kAdv3Waves<N, NQ, PREC>)) void k_adv3d_stage(Adv3Args A)
 {
     using S = Shape3<N>;
     constexpr int n1 = S::n1, n2 = S::n2, np = S::np, epb = S::epb;
@@ -553,7 +559,16 @@ __global__ __launch_bounds__(Shape3<N>::threads, (N == 7 && NQ == 1 && PREC == 0
     #pragma unroll
     for (int q = 0; q < FQ; ++q) {
         int l2, sd, node;
-        if (!face(q, l2, sd, node)) continue;
+        if constexpr (MF) {
+            if (!face(q, l2, sd, node)) continue;
+        } else {  // from the number that is not clamped: formed again, not kept from the loads
+            const int w = t + q * S::threads;
+            if (w >= nF) continue;
+            l2 = w / (6 * n2);
+            const int rem = w - l2 * 6 * n2;
+            sd = rem / n2;
+            node = rem - sd * n2;
+        }
         const int e2 = blockIdx.x * epb + l2;
         if (e2 >= A.nE) continue;
         const int a = node % n1, b = node / n1;
