@@ -409,7 +409,7 @@ struct AdvStepsArgs {
 // Workgroups a CU decide up to which size a model is resident: where two registers
 // stand between three and two of them, three are asked for.
 template <int N, int NQ>
-constexpr int kAdvWaves = NQ == 1 && (N == 1 || N == 8) ? 3 : 1;
+constexpr int kAdvWaves = NQ == 1 && (N == 1 || N > 6) ? 3 : 1;
 
 template <int N, int NQ>
 __global__ __launch_bounds__(256, (kAdvWaves<N, NQ>)) void k_adv_steps(AdvArgs A, AdvStepsArgs T)
@@ -421,12 +421,7 @@ __global__ __launch_bounds__(256, (kAdvWaves<N, NQ>)) void k_adv_steps(AdvArgs A
     __shared__ double cs[epb * NQ * np], sx[epb * NQ * np], sy[epb * NQ * np], px[epb * NQ * np],
         py[epb * NQ * np], bf[epb * 4 * 2 * NQ * n1];
     __shared__ int stop;
-    // where the gradient goes is read when it is needed: no registers hold it meanwhile
-    __shared__ double *volatile grads[1];
-    if (threadIdx.x == 0) {
-        stop = persist_given_up(T.P);
-        grads[0] = A.grad;
-    }
+    if (threadIdx.x == 0) stop = persist_given_up(T.P);
     stage_nodal<N, false>(L, A.nodal, nullptr, nullptr);
     __syncthreads();
     if (stop) return;  // an earlier launch of this model gave up: leave the state to the host
@@ -561,10 +556,9 @@ __global__ __launch_bounds__(256, (kAdvWaves<N, NQ>)) void k_adv_steps(AdvArgs A
                 gx[f] = (x1[f] + x2[f]) / J;
                 gy[f] = (y1[f] + y2[f]) / J;
                 // Every lane is past its contractions: the arrays of the gradient's
-                // flux take the gradient (sx for its traces, py and sy until the next
-                // stage) and then the volume flux (sx, px).
+                // flux take the gradient (sx, sy, until the next stage) and the volume
+                // flux (py, px).
                 sx[lo + f * np + nd] = gx[f];
-                py[lo + f * np + nd] = gx[f];
                 sy[lo + f * np + nd] = gy[f];
             }
         }
@@ -587,13 +581,13 @@ __global__ __launch_bounds__(256, (kAdvWaves<N, NQ>)) void k_adv_steps(AdvArgs A
         if (act) {
             #pragma unroll
             for (int f = 0; f < NQ; ++f)
-                adv_volume_flux(c[f], u, v, A.kappa, gx[f], gy[f], met, sx[lo + f * np + nd], px[lo + f * np + nd]);
+                adv_volume_flux(c[f], u, v, A.kappa, gx[f], gy[f], met, py[lo + f * np + nd], px[lo + f * np + nd]);
         }
         sync();
         if (act) {
             #pragma unroll
             for (int f = 0; f < NQ; ++f)
-                dg_lines<N>(L, sx + lo + f * np + n1 * j, px + lo + f * np + i, i, j, x1[f], x2[f]);
+                dg_lines<N>(L, py + lo + f * np + n1 * j, px + lo + f * np + i, i, j, x1[f], x2[f]);
         }
         // ---- neighbours' gradients, upwind and diffusive flux
         #pragma unroll
@@ -649,12 +643,11 @@ __global__ __launch_bounds__(256, (kAdvWaves<N, NQ>)) void k_adv_steps(AdvArgs A
     }
     if (act) {
         // the model's gradient is the last stage's, as the launched stages leave it
-        double *grad = *grads;
         #pragma unroll
         for (int f = 0; f < NQ; ++f) {
             T.cOut[f * mstride + base] = c[f];
-            grad[f * mstride + base] = py[lo + f * np + nd];
-            grad[(NQ + f) * mstride + base] = sy[lo + f * np + nd];
+            A.grad[f * mstride + base] = sx[lo + f * np + nd];
+            A.grad[(NQ + f) * mstride + base] = sy[lo + f * np + nd];
         }
     }
 }
@@ -794,7 +787,7 @@ int resident_prepare(self_adv2d_s *h)
     h->runs.messageBytes = 3 * sizeof(ll_quad) * ll_quads(h);
     if (hipMalloc(reinterpret_cast<void **>(&h->cAlt), sizeof(double) * h->nq * h->nE * h->np) != hipSuccess ||
         hipMalloc(reinterpret_cast<void **>(&h->runs.messages), h->runs.messageBytes) != hipSuccess ||
-        hipMalloc(reinterpret_cast<void **>(&h->runs.status), sizeof(PersistStatus)) != hipSuccess ||
+        hipMalloc(reinterpret_cast<void **>(&h->runs.status), sizeof(int)) != hipSuccess ||
         h->runs.alloc_host() != hipSuccess) {
         (void)hipGetLastError();
         if (h->cAlt) (void)hipFree(h->cAlt);

@@ -389,10 +389,10 @@ __global__ __launch_bounds__(kCgResThreads) void k_cg_resident(CgResArgs A)
 // The launch's end in the solver state; done = kCgGaveUp where it gave up.
 constexpr int kCgGaveUp = 9;
 
-__global__ void k_cg_res_commit(SolverState *st, const CgResOut *out, const PersistStatus *status)
+__global__ void k_cg_res_commit(SolverState *st, const CgResOut *out, const int *status)
 {
     if (st->done) return;  // nothing to solve: the launch returned at once
-    if (status->launch != 0) {
+    if (*status != 0) {
         st->done = kCgGaveUp;
         return;
     }

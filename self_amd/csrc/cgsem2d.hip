@@ -643,7 +643,7 @@ struct CgsemOp final : DevOp {
         A.nE = (int)nE;
         A.tag0 = resTag;
         A.out = reinterpret_cast<CgResOut *>(resBuf + res_exch() + kResRed);
-        A.P.status = reinterpret_cast<PersistStatus *>(resBuf + resBytes - 64);
+        A.P.status = reinterpret_cast<int *>(resBuf + resBytes - 64);
         A.P.launch = ++resUps.launches;
         A.P.limit = persist_spin_limit();
         PersistGate gate(device, s, blocks, 1);
@@ -651,7 +651,7 @@ struct CgsemOp final : DevOp {
         hipLaunchKernelGGL((k_cg_resident<NN, K>), dim3((unsigned)blocks), dim3(kCgResThreads), 0, s, A);
         SELF_HIP(hipGetLastError());
         hipLaunchKernelGGL(k_cg_res_commit, dim3(1), dim3(1), 0, s, wk.st, (const CgResOut *)A.out,
-                           (const PersistStatus *)A.P.status);
+                           (const int *)A.P.status);
         SELF_HIP(hipGetLastError());
         taken = true;
         return gate.launched();

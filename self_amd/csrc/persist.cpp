@@ -74,7 +74,7 @@ unsigned persist_spin_limit()
 int ResidentRuns::clear(hipStream_t s)
 {
     SELF_HIP(hipMemsetAsync(messages, 0, messageBytes, s));
-    SELF_HIP(hipMemsetAsync(&status->launch, 0, sizeof(int), s));
+    SELF_HIP(hipMemsetAsync(status, 0, sizeof(int), s));
     *hostStatus = 0;
     tag = 0;
     return SELF_OK;
@@ -83,9 +83,8 @@ int ResidentRuns::clear(hipStream_t s)
 hipError_t ResidentRuns::alloc_host()
 {
     if (hostStatus) return hipSuccess;
-    hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&hostStatus), sizeof(int), hipHostMallocDefault);
+    const hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&hostStatus), sizeof(int), hipHostMallocDefault);
     if (e != hipSuccess) hostStatus = nullptr;
-    else if ((e = hipMemcpy(&status->host, &hostStatus, sizeof(int *), hipMemcpyHostToDevice)) != hipSuccess) free_host();
     return e;
 }
 

@@ -113,23 +113,17 @@ __device__ __forceinline__ bool ll_try1(const LLBuf &B, unsigned off, unsigned t
     return (wrong >> 16) == 0;
 }
 
-// In device memory, in one of a model's buffers: 0, or the number of the first
-// launch that gave up, and where to write it for the host too (or null).
-struct PersistStatus {
-    int launch;
-    int *host;
-};
-
 // One launch's bookkeeping, shared by the kernels' waits.
 struct PersistArgs {
-    PersistStatus *status;
+    int *status;      // 0, or the number of the first launch that gave up (device memory)
+    int *host;        // the same in pinned host memory, written only: the host's to read (or null)
     int launch;       // this launch's number (>= 1)
     unsigned limit;   // polls before a wait gives up
 };
 
 __device__ __forceinline__ bool persist_given_up(const PersistArgs &P)
 {
-    return __hip_atomic_load(&P.status->launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+    return __hip_atomic_load(P.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
 }
 
 // Every lane of the wavefront calls this; attempt() of a lane is true once it
@@ -145,8 +139,8 @@ __device__ __forceinline__ bool ll_wait(bool need, const PersistArgs &P, F attem
         __builtin_amdgcn_s_sleep(1);
         if ((n & 63u) == 63u && persist_given_up(P)) return false;
         if (n >= P.limit) {
-            __hip_atomic_store(&P.status->launch, P.launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (int *host = P.status->host) __hip_atomic_store(host, P.launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(P.status, P.launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (P.host) __hip_atomic_store(P.host, P.launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             return false;
         }
     }
@@ -197,18 +191,17 @@ struct ResidentRuns {
         double t0;
         double *in;  // the state the run began with
     };
-    // The status twice: workgroups read it in device memory (in host memory that
-    // cost 0.1 us a workgroup), the host in its own (a copy of it took 20 us of
-    // each wait for the model).
-    PersistStatus *status = nullptr;
-    int *hostStatus = nullptr;
+    // The status word twice: workgroups read it in device memory (in host memory
+    // that cost 0.1 us a workgroup), the host in its own (a copy of it took 20 us
+    // of each wait for the model).
+    int *status = nullptr, *hostStatus = nullptr;
     ll_quad *messages = nullptr;
     size_t messageBytes = 0;
     unsigned tag = 0;              // of the last stage launched; the cleared messages' is 0
     GiveUps ups;
     bool off = false;              // the model does not fit, or there was no memory for its buffers
     std::vector<Run> pending;
-    PersistArgs args() const { return {status, ups.launches + 1, persist_spin_limit()}; }
+    PersistArgs args() const { return {status, hostStatus, ups.launches + 1, persist_spin_limit()}; }
     // call it as soon as the launch is queued: its messages will have been written
     void launched(int first, int steps, double t0, double *in)
     {
@@ -216,7 +209,7 @@ struct ResidentRuns {
         pending.push_back({++ups.launches, first, steps, t0, in});
     }
     int clear(hipStream_t s);      // messages and status, with no launch in flight
-    hipError_t alloc_host();       // the host's word, told to the status
+    hipError_t alloc_host();
     void free_host();
     int settle(hipStream_t s, std::vector<Run> &again);
 };

@@ -267,20 +267,22 @@ __device__ __forceinline__ void trace3(const NodalLDS<N> &L, const double *qs, i
 template <int N>
 constexpr bool kMfStage = N == 7;
 
-// Node of lane tl.  At N = 3 and 7 the products are formed transposed: a result's
-// column, the fast lane index, is the node's first index, so that lanes next to
-// each other load nodes next to each other, 4 or 8 of them (N + 1 apart the other
-// way: a launched stage of 66x66, N = 7 FP64 12.2 us against 11.7, a resident one
-// of 64x64, N = 7 mixed 4.4 against 4.3; the 3-D kernels and the conjugate
-// gradients, whose node values go through LDS or stay, are 2 % faster that way).
+// Node of lane tl.  At N = 7 the products are formed transposed: a result's column,
+// the fast lane index, is the node's first index, so that eight lanes next to each
+// other load nodes next to each other (8 apart the other way: a launched stage of
+// 66x66, FP64 12.2 us against 11.7, a resident one of 64x64, mixed 4.4 against 4.3).
+// The resident form at N = 3, the 3-D kernels and the conjugate gradients, which
+// load once or by way of LDS, are 1 to 2 % faster the other way.
 template <int N, bool MF = Mf<N>::on>
 __device__ __forceinline__ int sw_node(int tl)
 {
-    if constexpr (MF) {
+    if constexpr (!MF) {
+        return tl;
+    } else if constexpr (N == 3) {
+        return lane_node<N>(tl);
+    } else {
         const MfLane<N> m(tl);
         return (4 * m.bi + m.c) + (N + 1) * (4 * m.bj + m.k);
-    } else {
-        return tl;
     }
 }
 
@@ -342,8 +344,14 @@ __device__ __forceinline__ void mf_volume(const MfOps<N> &M, const double *sC, c
     #pragma unroll
     for (int q = 0; q < Mf<N>::K; ++q) {
         const int m = 4 * q + a.k;
-        t1 = __builtin_amdgcn_mfma_f64_4x4x4f64(sC[m + n1 * (4 * a.bj + a.c)], M.s[q], t1, 0, 0, 0);
-        t2 = __builtin_amdgcn_mfma_f64_4x4x4f64(M.p[q], pC[(4 * a.bi + a.c) + n1 * m], t2, 0, 0, 0);
+        const double s = sC[m + n1 * (4 * a.bj + a.c)], p = pC[(4 * a.bi + a.c) + n1 * m];
+        if constexpr (N == 3) {
+            t1 = __builtin_amdgcn_mfma_f64_4x4x4f64(M.s[q], s, t1, 0, 0, 0);
+            t2 = __builtin_amdgcn_mfma_f64_4x4x4f64(p, M.p[q], t2, 0, 0, 0);
+        } else {
+            t1 = __builtin_amdgcn_mfma_f64_4x4x4f64(s, M.s[q], t1, 0, 0, 0);
+            t2 = __builtin_amdgcn_mfma_f64_4x4x4f64(M.p[q], p, t2, 0, 0, 0);
+        }
     }
 }
 

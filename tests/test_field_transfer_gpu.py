@@ -100,7 +100,7 @@ def test_a_request_reserves_what_its_model_holds(gpu_lib, precision, nX, N):
     check(lib.self_sw2d_device_bytes(h, C.byref(held)))
     check(lib.self_sw2d_destroy(h))
     nodes = g.nElems * (N + 1) ** 2
-    resident = 3 * 8 * nodes + 2 * 16 * g.nElems * 8 * (N + 1) + 16  # second state, messages, status
+    resident = 3 * 8 * nodes + 2 * 16 * g.nElems * 8 * (N + 1) + 4  # second state, messages, status
     m.GetSolution()
     assert m.DeviceBytes() == held.value + resident
     assert held.value <= res.bytes
