@@ -886,8 +886,8 @@ __device__ __forceinline__ void sw_stage_group(const SWKernelArgs &A0, int wg, S
     }
     constexpr int kLanes = WL ? 64 : 256;
     const int lane = WL ? threadIdx.x % 64 : threadIdx.x;
-    NodalRegs<N, MIXED, kLanes> R;
-    nodal_fetch<N, MIXED, kLanes>(R, A.dS, A.dS32, A.dP32, lane);
+    NodalRegs<N, Lds::DEV, kLanes> R;
+    nodal_fetch<N, Lds::DEV, kLanes>(R, A.dS, A.dS32, A.dP32, lane);
     SWPre P[G];
     int e[G];
     bool act[G];
@@ -897,7 +897,7 @@ __device__ __forceinline__ void sw_stage_group(const SWKernelArgs &A0, int wg, S
         act[g] = le < epb && e[g] < A.nE;
         sw_load<N, MIXED>(A, e[g], sw_node<N, kMfStage<N>>(tl), lane_side<N, kMfStage<N>>(tl), act[g], P[g]);
     }
-    nodal_put<N, MIXED, kLanes>(L, R, lane);
+    nodal_put<N, Lds::DEV, kLanes>(L, R, lane);
     if constexpr (WL) wave_sync();
     const int ls = le < epb ? le : 0;
     double *qsE = U.qs + ls * 3 * np, *sCE = U.sC + ls * 3 * np, *pCE = U.pC + ls * 3 * np;
@@ -998,11 +998,11 @@ __global__ __launch_bounds__(256, 4) void k_sw_steps(SWKernelArgs A, SWStepsArgs
     const size_t mstride = (size_t)A.nE * np, base = (size_t)e * np + nd;
     SWPre P;
     {
-        NodalRegs<N, MIXED, kLanes> R;
-        nodal_fetch<N, MIXED, kLanes>(R, A.dS, A.dS32, A.dP32, lane);
+        NodalRegs<N, Lds::DEV, kLanes> R;
+        nodal_fetch<N, Lds::DEV, kLanes>(R, A.dS, A.dS32, A.dP32, lane);
         A.a = 0.0;  // no register is read
         sw_load<N, MIXED>(A, e, nd, w0, act, P);
-        nodal_put<N, MIXED, kLanes>(L, R, lane);
+        nodal_put<N, Lds::DEV, kLanes>(L, R, lane);
     }
     sw_finish<MIXED>(A, act, P);
     const int ls = le < epb ? le : 0;
