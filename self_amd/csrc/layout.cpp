@@ -1,6 +1,8 @@
 // layout.cpp -- pinned buffers of the transfers in layout.hpp.
 #include "layout.hpp"
 
+#include <emmintrin.h>
+
 #include <cstdlib>
 #include <mutex>
 
@@ -30,6 +32,26 @@ size_t stage_doubles()
     if (s && *s) return (size_t)std::strtoull(s, nullptr, 10);
     return (size_t)1 << 19;
 }
+
+void store_past_caches(double *to, const double *from, size_t n)
+{
+    long long v;
+    size_t k = 0;
+    if (n > 0 && reinterpret_cast<uintptr_t>(to) % 16) {
+        std::memcpy(&v, from, sizeof v);
+        _mm_stream_si64(reinterpret_cast<long long *>(to), v);
+        k = 1;
+    }
+    for (; k + 2 <= n; k += 2)
+        _mm_stream_si128(reinterpret_cast<__m128i *>(to + k),
+                         _mm_loadu_si128(reinterpret_cast<const __m128i *>(from + k)));
+    if (k < n) {
+        std::memcpy(&v, from + k, sizeof v);
+        _mm_stream_si64(reinterpret_cast<long long *>(to + k), v);
+    }
+}
+
+void store_past_caches_fence() { _mm_sfence(); }
 
 StageLease::StageLease(size_t n, hipStream_t s) : s_(s)
 {

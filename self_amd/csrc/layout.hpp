@@ -8,11 +8,13 @@
 // fresher they are.  Measured, us, fresh pages (a hipMemcpy into a vector and a
 // memcpy; a reordering kernel and a copy into the caller's array; this): 6 KB of
 // three fields 12.8, 24.5, 12.2; 0.8 MB 415, 463, 114; 12.6 MB 1430, 954, 728;
-// 50 MB 15250, 4470, 3900.  Where no pinned memory is to be had, the vector
+// 50 MB 15250, 4470, 3900 (with ordinary stores; past the caches 31 MB of warm
+// pages take 1600 instead of 2200).  Where no pinned memory is to be had, the vector
 // serves.
 #pragma once
 
 #include <algorithm>
+#include <cstdint>
 #include <cstring>
 #include <vector>
 
@@ -24,6 +26,8 @@ namespace self {
 // SELF_AMD_STAGE_DOUBLES overrides it (a test of the way without the buffer
 // sets 0, of several pieces a small number).
 size_t stage_doubles();
+
+constexpr size_t kPastCaches = (size_t)1 << 17;  // doubles, 1 MB
 
 // A pinned buffer for one transfer, from a small process-wide pool: a new one
 // costs 0.3 ms a MB on its first use.  Any thread, any stream of the current
@@ -53,19 +57,32 @@ private:
     bool over_ = false;
 };
 
+// n values past the caches, any 8-byte alignment; fence() before others look.
+void store_past_caches(double *to, const double *from, size_t n);
+void store_past_caches_fence();
+
 // Work queued on s before the call is waited for; the copy is complete on return.
 inline int fields_to_host(const double *dev, double *host, size_t nE, int nf, int np, hipStream_t s)
 {
     const size_t row = (size_t)nf * np, most = stage_doubles();
     const size_t piece = std::min(nE, std::max<size_t>(1, most / row)), n = piece ? (nE + piece - 1) / piece : 0;
+    // An array of 1 MB does not stay in a core's second-level cache anyway, and
+    // an ordinary store reads each line first: three fields of 26367 x 49 nodes
+    // took 1773 us so, 983 past the caches, 804 without putting them anywhere.
+    const bool past = nE * row >= kPastCaches && reinterpret_cast<uintptr_t>(host) % sizeof(double) == 0;
+    const auto put = [&](double *to, const double *from, size_t k) {
+        if (past) store_past_caches(to, from, k);
+        else std::memcpy(to, from, sizeof(double) * k);
+    };
     const auto order = [&](const double *src, size_t e0, size_t m) {  // src: [field][m][node]
         if (nf == 1) {
-            std::memcpy(host + e0 * row, src, sizeof(double) * m * row);
-            return;
+            put(host + e0 * row, src, m * row);
+        } else {
+            for (size_t e = 0; e < m; ++e)
+                for (size_t f = 0; f < (size_t)nf; ++f)
+                    put(host + ((e0 + e) * nf + f) * np, src + (f * m + e) * np, (size_t)np);
         }
-        for (size_t e = 0; e < m; ++e)
-            for (size_t f = 0; f < (size_t)nf; ++f)
-                std::memcpy(host + ((e0 + e) * nf + f) * np, src + (f * m + e) * np, sizeof(double) * np);
+        if (past) store_past_caches_fence();
     };
     StageLease st(most ? std::min<size_t>(n, 2) * piece * row : 0, s);
     if (!st.ok()) {

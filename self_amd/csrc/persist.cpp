@@ -62,7 +62,7 @@ int persist_blocks_per_cu(const void *kernel, int threads)
     return n;
 }
 
-// About a microsecond a poll.  SELF_AMD_SPIN_LIMIT overrides it (a test of
+// Half a microsecond to one a poll.  SELF_AMD_SPIN_LIMIT overrides it (a test of
 // the fallback sets 0: the first unsuccessful poll gives up).
 unsigned persist_spin_limit()
 {

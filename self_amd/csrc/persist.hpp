@@ -6,7 +6,9 @@
 // belongs to.  A reader polls the words themselves until all carry the tag it
 // wants, so no fence, flag or ordering between words is needed: an aligned
 // 8-byte half of an access is single-copy atomic, and agent-scope accesses
-// (sc1) are coherent across the 8 XCDs' L2s.  Buffers are double-buffered by
+// (sc1) are coherent across the 8 XCDs' L2s.  Flags inside the data are the
+// method of the low-latency (LL) protocol of NCCL and RCCL; the words' layout,
+// their tags and the bounded waits are this library's.  Buffers are double-buffered by
 // the tag's parity: a writer overwrites a word only after it has received a
 // value its reader sent after reading that word, so a word holds the wanted
 // tag or that of two steps before and 16 bits of tag are enough.
@@ -21,8 +23,8 @@
 // last workgroup is placed is not the host's to say: kernels of other streams
 // that run at the start can leave a CU's LDS and registers in pieces too small
 // for it (seen: a launch of 1024 workgroups beside another model's stage
-// kernels).  So every wait is bounded: past `limit` polls (about a millisecond,
-// hundreds of times the longest wait of a resident launch) the launch records
+// kernels).  So every wait is bounded: past `limit` polls (2000, one to two
+// milliseconds, hundreds of times the longest wait of a resident launch) the launch records
 // its number in *status, every other wait sees that and all workgroups end,
 // leaving the launch's input untouched; the launches queued behind it return at
 // once, and the host runs the steps through ordinary launches.

@@ -42,6 +42,27 @@ def test_every_way_gives_the_same_bytes(gpu_lib, make, monkeypatch):
     assert np.array_equal(m.GetSolution(), want)
 
 
+@pytest.mark.parametrize("N,nX,nY", [(2, 70, 70), (6, 30, 30), (7, 34, 21)])
+def test_large_arrays_at_every_alignment(gpu_lib, N, nX, nY):
+    """From 1 MB on an array is written past the caches, in 16-byte stores with
+    8-byte ones at a row's ends: rows of odd and even lengths, the caller's
+    array on and off 16 bytes and off 8, nothing beside it touched."""
+    L = gpu_lib
+    m = sw2d_model(N=N, nX=nX, nY=nY, precision="fp64")
+    m.ForwardStepRK3(0.0, 1)
+    want = np.ascontiguousarray(m.GetSolution()).ravel()
+    assert want.nbytes >= 1 << 20 and np.isfinite(want).all()
+    buf = np.empty(want.nbytes + 64, np.uint8)
+    first = -buf.ctypes.data % 16 + 16
+    for off in (first, first + 8, first + 4):
+        buf[:] = 0xa5
+        L.check(L.lib().self_sw2d_get_field(m._h, 0, C.cast(buf.ctypes.data + off, L.dp)))
+        got = buf[off:off + want.nbytes]
+        assert np.array_equal(got, want.view(np.uint8))
+        assert (buf[:off] == 0xa5).all() and (buf[off + want.nbytes:] == 0xa5).all()
+    m.Trash()
+
+
 def test_reading_a_field_takes_no_device_memory(gpu_lib):
     m = _sw2d()
     before = m.DeviceBytes()
