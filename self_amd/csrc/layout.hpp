@@ -69,7 +69,12 @@ inline int fields_to_host(const double *dev, double *host, size_t nE, int nf, in
     // An array of 1 MB does not stay in a core's second-level cache anyway, and
     // an ordinary store reads each line first: three fields of 26367 x 49 nodes
     // took 1773 us so, 983 past the caches, 804 without putting them anywhere.
-    const bool past = nE * row >= kPastCaches && reinterpret_cast<uintptr_t>(host) % sizeof(double) == 0;
+    // Several fields of long rows, each a jump in the buffer, are better left to
+    // memcpy: GetSolution with it and past the caches, us, 3 x 49 nodes 2210,
+    // 1535; 5 x 216 950, 960; 2 x 343 1175, 1250; 5 x 512 8800, 11000; one field
+    // of 67 MB 4880, 4400.
+    const bool past = nE * row >= kPastCaches && (nf == 1 || np <= 128) &&
+                      reinterpret_cast<uintptr_t>(host) % sizeof(double) == 0;
     const auto put = [&](double *to, const double *from, size_t k) {
         if (past) store_past_caches(to, from, k);
         else std::memcpy(to, from, sizeof(double) * k);
