@@ -1,7 +1,7 @@
 """Run one workload for a fixed number of steps, for use under a profiler.
 
     python -m self_amd.profile_run copy
-    python -m self_amd.profile_run sw2d --precision mixed --form fused --steps 10
+    python -m self_amd.profile_run sw2d --precision mixed --form fused --steps 10 [--launched]
     python -m self_amd.profile_run sw2d-dipole --mesh box.mesh --N 10 --form plain --precision fp64
     python -m self_amd.profile_run adv2d --steps 10
     python -m self_amd.profile_run adv3d --steps 5 [--contraction fp32|bf16x3]
@@ -10,6 +10,8 @@
     python -m self_amd.profile_run hpe --steps 5
     python -m self_amd.profile_run cgsem-batched --nx 64 [--iters 64]
 
+sw2d --launched launches every stage from the host, as for models that do not
+fit the device; without it two or more steps are one launch.
 `sw2d-dipole` runs the shallow-water model on an ISM-V2 mesh file (the
 dipole run's box.mesh, scaled by 4e5) with the dipole state.
 `copy` runs the STREAM-style copy kernel on 24 MiB (read and written: about
@@ -45,6 +47,7 @@ def main(argv=None):
     ap.add_argument("--iters", type=int, default=20000, help="iteration limit (cgsem-batched)")
     ap.add_argument("--contraction", default="fp64", choices=["fp64", "fp32", "bf16x3"],
                     help="arithmetic of the 3-D volume contractions (adv3d)")
+    ap.add_argument("--launched", action="store_true", help="one launch a stage (sw2d)")
     a = ap.parse_args(argv)
     L.check(L.lib().self_init(0))
     if a.mode == "copy":
@@ -55,6 +58,8 @@ def main(argv=None):
     elif a.mode == "sw2d":
         from .workloads import sw2d_geostrophic
         m, _ = sw2d_geostrophic(a.nx or 64, a.N, precision=a.precision, form=a.form)
+        if a.launched:
+            m.SetGraph(False)
         m.ForwardStepRK3(0.0, a.steps)
         m.Synchronize()
         print(f"sw2d {a.precision} {a.form}: {a.steps} RK3 steps", flush=True)
