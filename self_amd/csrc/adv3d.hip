@@ -406,7 +406,9 @@ __global__ __launch_bounds__(Shape3<N>::threads) void k_adv3d_prologue(Adv3Args 
 // PREC 0: FP64 contractions; 1: FP32 matrix-core contractions; 2: split-BF16
 // matrix-core contractions (mfma.hpp).  State, register, geometry, face
 // fluxes, lift, Jacobian and the filter are FP64 in every form.
-// N = 7 in FP64 runs on the matrix cores.  Bound: HBM, 738 MB a stage at
+// N = 7 in FP64 runs on the matrix cores: a plane of 64 nodes is a wavefront's four
+// 4x4 tiles.  N = 3 divides into such tiles too, but four of its planes would share
+// a wavefront, a layout not written here.  Bound: HBM, 738 MB a stage at
 // 32x32x16 and one tracer, 154 us at the rate of a large copy; the LDS reads of
 // the line sums (16 b64 a node and contraction, ~80 us) and the occupancy they
 // left were added to that.  Measured a stage: 192.8 -> 158.7 us there, 55.2 ->

@@ -807,7 +807,9 @@ HpeArgs args_of(self_hpe_s *h)
     return A;
 }
 
-// The two kernels of a time derivative and update; N = 7 has its own.
+// The two kernels of a time derivative and update; N = 7, where a plane of 64
+// nodes is a wavefront's four matrix-core tiles, has its own.  Their single sweep
+// and folded sums would serve other degrees, whose kernels do not have them.
 int launch_columns(self_hpe_s *h, const HpeArgs &A)
 {
     HPE_DISPATCH_N(h->N, {
